@@ -293,6 +293,9 @@ struct Context {
     // FFT workspace
     DevBuf<double2> fa, fb;
     DevBuf<double2> tw[3];          // per-axis twiddles e^{-2 pi i k / n}
+    DevBuf<uint8_t> fft_stage[3];   // per-axis mixed-radix plan (FftStage array)
+    DevBuf<uint16_t> fft_rev[3];    // and its digit-reversed slots
+    int fft_stages[3] = {0, 0, 0};
     // 1D Dirichlet precomputed Thomas coefficients
     DevBuf<double> thomas_inv;       // 1D Dirichlet solve: first-difference scratch
     DevBuf<double> dft_cos, dft_sin;
