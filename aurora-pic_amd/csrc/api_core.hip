@@ -79,7 +79,7 @@ bool sort_needed(Context& c, Species& sp) {
 // step late (the previous step's push has completed by then), so the
 // decision lags by one step and the host never stalls the queue.
 bool adaptive_sort_due(Context& c, Species& sp) {
-    if (sp.precision != 32 || !c.tiled_push_ok()) return false;  // no tiled push to speed up
+    if (!c.tiled_push_ok()) return false;  // no tiled push to speed up
     if (!sp.tiled) return sp.slots > 0;
     if (sp.sort_ev.recorded && hipEventQuery(sp.sort_ev.b) == hipSuccess)
         sp.cycle_ms += sp.sort_ev.take_ms();

@@ -313,7 +313,7 @@ struct Context {
     int tile[3] = {8, 8, 8};
     int halo = 2;
     int push_block = 512;        // tiled push workgroup size
-    int push_prefetch = 0;       // tiled push loads the next particle early
+    int push_prefetch = -1;      // tiled push variant; -1: the library's choice for the tile shape
     bool tiled_enabled = true;
     DevBuf<int32_t> tile_count, tile_offset;
     DevBuf<unsigned> sort_keys, sort_keys2, sort_vals, sort_vals2;
@@ -377,14 +377,14 @@ struct Context {
     int64_t ntiles() const {
         return static_cast<int64_t>(tiles_axis(0)) * tiles_axis(1) * tiles_axis(2);
     }
-    // the LDS-tiled 2D and 3D pushes apply on periodic meshes whose extents
-    // the tiles divide and that hold a whole tile box without self-overlap
+    // the LDS-tiled 2D and 3D pushes apply on periodic meshes that hold a
+    // whole tile box without self-overlap (the tiles need not divide them)
     bool tiled_push_ok() const {
         if (!tiled_enabled || (dim != 3 && dim != 2) || bc != AURORA_PERIODIC) return false;
         for (int f = 0; f < 2 * dim; ++f)
             if (pb[f] != AURORA_PB_PERIODIC) return false;
         for (int a = 0; a < dim; ++a)
-            if (n[a] % tile[a] != 0 || n[a] < tile[a] + 1 + 2 * halo) return false;
+            if (n[a] < tile[a] + 1 + 2 * halo) return false;
         return true;
     }
 };

@@ -114,18 +114,18 @@ __device__ __forceinline__ bool drift_axis(int& idx, R& off, R& v, R dx, int nce
 
 // drift_axis on a periodic axis, also returning the cell shift (the
 // particle's move in cells before the wrap); same operations, same result.
-__device__ __forceinline__ void drift_periodic(int& idx, float& off, float dx, int n,
-                                               int& shift) {
-    const float x = off + dx;
-    if (x >= 0.f && x < 1.f) {
+template <typename R>
+__device__ __forceinline__ void drift_periodic(int& idx, R& off, R dx, int n, int& shift) {
+    const R x = off + dx;
+    if (x >= R(0) && x < R(1)) {
         off = x;
         shift = 0;
         return;
     }
-    const float fl = floorf(x);
+    const R fl = floor(x);
     int s = static_cast<int>(fl);
-    float f = x - fl;
-    if (f >= 1.f) { f = 0.f; s += 1; }
+    R f = x - fl;
+    if (f >= R(1)) { f = R(0); s += 1; }
     int ni = idx + s;
     if (static_cast<unsigned>(ni) >= static_cast<unsigned>(n)) ni = wrap_index(ni, n);
     idx = ni;

@@ -213,7 +213,8 @@ int aurora_hip_power_transfer(aurora_hip_ctx* ctx, int species_id, double* elect
 int aurora_hip_time(aurora_hip_ctx* ctx, double* time, int64_t* step);
 /* Tile shape (cells per axis) of the cell sort and of the LDS-tiled 2D and
  * 3D pushes, and its halo in cells; tx = 0 keeps the sort but disables the
- * tiled push.  Built 3D shapes: 8x8x8 (halo 1, 2), 8x8x4 (halo 1, 2),
+ * tiled push.  The tiles need not divide the mesh, which holds at least a
+ * tile with its halo per axis (else the untiled push runs).  Built 3D shapes: 8x8x8 (halo 1, 2), 8x8x4 (halo 1, 2),
  * 4x4x4, 16x8x4 (halo 2); 2D (tz ignored; 1 names them): 8x8 (halo 1, 2;
  * 512 threads, or 256 with prefetch), 16x16 and 16x8 (halo 2).
  * No reference counterpart (the reference keeps particles unsorted). */
@@ -223,11 +224,14 @@ int aurora_hip_set_tiling(aurora_hip_ctx* ctx, int tx, int ty, int tz,
  * flags (bit 0: the next particle's state is loaded while the current one
  * is processed; bit 1: registers capped at 64 so four 512-thread workgroups
  * share a CU; bit 2: the field box in LDS by component instead of float4
- * nodes; bit 3: non-temporal particle stores).  Built: 512/0 for every
- * shape; 512/1, 256/1, 256/0, 512/3, 512/5, 512/7, 512/11, 512/13, 512/15
- * for 8x8x4 halo 2; 512/3 for 8x8x4 halo 1; 512/1, 256/1, 512/5, 512/13 for 8x8x8
- * halo 2; 512/1, 512/3, 512/5, 512/7, 512/13, 512/15 for 8x8x8 halo 1.
- * Results do not depend on it. */
+ * nodes; bit 3: non-temporal particle stores).  Built for FP32 species:
+ * 512/0, 512/1, 256/1, 256/0, 512/3, 512/5, 512/7, 512/11, 512/13, 512/15
+ * for 8x8x4 halo 2; 512/3 for 8x8x4 halo 1; 512/0, 512/1, 256/1, 512/5,
+ * 512/13 for 8x8x8 halo 2; 512/0, 512/1, 512/3, 512/5, 512/7, 512/13, 512/15
+ * for 8x8x8 halo 1; 512/0 for 4x4x4 and 16x8x4.  Every shape also has the
+ * library's own choice, which runs when no variant was set, when the set one
+ * is not built for the shape, and for FP64 species.  Results do not depend
+ * on it. */
 int aurora_hip_set_push_variant(aurora_hip_ctx* ctx, int block, int prefetch);
 /* Cell sort every interval steps (0 = never) and an immediate sort. */
 int aurora_hip_set_sort_interval(aurora_hip_ctx* ctx, int64_t interval);

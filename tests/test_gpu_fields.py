@@ -819,3 +819,59 @@ def test_periodic_solve_any_size(hip_ctx, n):
     assert err(phi, np.fft.ifftn(p).real.reshape(-1)) <= 2.0e-13
     for a in range(len(n)):
         assert err(E[a], np.fft.ifftn(-1j * ks[a] * p).real.reshape(-1)) <= 2.0e-13
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,shape,precision", [
+    ([21, 13, 30], None, 32),                    # the default tile, a partial last one, the box's size
+    ([29, 14, 23], (8, 8, 8, 1), 32), ([33, 17, 13], (8, 8, 4, 2), 32),
+    ([19, 27, 13], (8, 8, 4, 1), 32), ([14, 9, 11], (4, 4, 4, 2), 32),
+    ([23, 21, 19], (16, 8, 4, 2), 32),
+    ([21, 13, 30], None, 64), ([16, 16, 16], (8, 8, 8, 1), 64), ([33, 17, 13], (8, 8, 4, 2), 64),
+    ([19, 27, 13], (8, 8, 4, 1), 64), ([14, 9, 11], (4, 4, 4, 2), 64),
+    ([23, 21, 19], (16, 8, 4, 2), 64),
+    ([37, 45], None, 32), ([13, 70], (8, 8, 1, 1), 32), ([50, 23], (16, 16, 1, 2), 32),
+    ([41, 30], (16, 8, 1, 2), 32),
+    ([37, 45], None, 64), ([13, 70], (8, 8, 1, 1), 64), ([50, 23], (16, 16, 1, 2), 64),
+    ([41, 30], (16, 8, 1, 2), 64)])
+@pytest.mark.parametrize("bfield", ["none", "uniform", "table"])
+def test_tiled_push_undivided_mesh_and_precisions(n, shape, precision, bfield):
+    """Tiles that do not divide the mesh, and FP64 species: particles and
+    charge of the tiled push equal the untiled push's bit for bit, across
+    re-sorts and with particles leaving the tile halo.  A tile shape runs with
+    the library's variant where the caller chose none."""
+    from aurora_pic import hip
+    print(f"case={n} {shape} {precision} {bfield}", flush=True)
+    rng = np.random.default_rng(31)
+    dim = len(n)
+    L = [1.0, 0.75, 1.25][:dim]
+    N = 20000
+    pos = rng.uniform(0, 1, (N, dim)) * np.asarray(L)
+    pos[:n[0]] = 0.0                                  # on the seam
+    vel = rng.normal(0, 0.8, (N, 3))
+    x = np.linspace(0, 1.0, 65)
+    bvals = np.stack([0.1 * np.ones(65), 3.0 * np.exp(-((x - 0.5) / 0.2) ** 2),
+                      1.5 * np.ones(65)], axis=1)
+    out = []
+    for tiled in (True, False):
+        with hip.Context(0) as c:
+            c.mesh(n, L, 0, 1.0)
+            if bfield == "uniform":
+                c.uniform_b([0.0, 0.3, 2.0])
+            elif bfield == "table":
+                c.b_profile(0, x, bvals)
+            if not tiled:
+                c.tiling(0)
+            elif shape is not None:
+                c.tiling(*shape)
+            sid = c.add_species(-1.0, 1.0, 1.0 / N, N, precision)
+            c.upload(sid, pos, vel, kind=1)
+            c.sort()
+            c.initialize(0.01)
+            c.sort_interval(5)
+            c.step(0.01, 12)
+            p_, v_, _, u_ = c.download(sid)
+            o = np.argsort(u_)
+            out.append((c.charge_fixed(sid), p_[o], v_[o]))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
