@@ -294,6 +294,75 @@ int64_t energy_rows(int g) { return static_cast<int64_t>(g) * (kBlk / 64); }
 
 }  // namespace
 
+namespace {
+
+// Range maxima of one table: level k holds the maxima of 2^k rows from each.
+struct RangeMax {
+    std::vector<std::vector<double>> level;
+    explicit RangeMax(const std::vector<double>& v) : level{v} {
+        for (size_t w = 1; 2 * w <= v.size(); w *= 2) {
+            const auto& p = level.back();
+            std::vector<double> q(v.size() - 2 * w + 1);
+            for (size_t i = 0; i < q.size(); ++i) q[i] = std::max(p[i], p[i + w]);
+            level.push_back(std::move(q));
+        }
+    }
+    double operator()(size_t lo, size_t hi) const {   // rows lo .. hi inclusive
+        size_t k = 0;
+        while ((size_t{2} << k) <= hi - lo + 1) ++k;
+        return std::max(level[k][lo], level[k][hi + 1 - (size_t{1} << k)]);
+    }
+};
+
+// The same for thermal neutrals: the largest particle speed s below which
+// the window bound n sum_c max sigma_c (s + lim) over relative speeds
+// [s - lim, s + lim], lim = 8 neutral_vstd (Collision.cpp:627-685), stays
+// under max_frequency (1 - 1e-5).  Speeds are taken in intervals of 0.4 %;
+// on one the bound is at most that of its top speed over the union of its
+// windows, their energies widened by 1e-5 for the FP32 evaluation's rounding.
+// A cross section between two rows is at most the larger of the two, so the
+// rows from the last one below a window to the first one above it bound it;
+// thresholds only shrink the windows and are left out.
+double thermal_safe_speed(const MccModelHost& h) {
+    const double limit = h.max_frequency * (1.0 - 1.0e-5);
+    const double lim = 8.0 * h.neutral_vstd;
+    double hc[kMaxChannels];
+    std::vector<RangeMax> rm;
+    double top = 0.0;
+    for (int c = 0; c < h.nchan; ++c) {
+        const double em = h.frame[c] == AURORA_FRAME_CENTER_OF_MASS
+                              ? h.particle_mass * h.neutral_mass / (h.particle_mass + h.neutral_mass)
+                              : h.particle_mass;
+        hc[c] = 0.5 * em;
+        rm.emplace_back(h.sigma_host[c]);
+        top = std::max(top, std::sqrt(h.energy_host[c].back() / hc[c]));
+    }
+    auto bound = [&](double s0, double s1) {
+        const double g0 = std::max(0.0, s0 - lim), g1 = s1 + lim;
+        double sum = 0.0;
+        for (int c = 0; c < h.nchan; ++c) {
+            const auto& E = h.energy_host[c];
+            const auto lo = std::upper_bound(E.begin(), E.end(), hc[c] * g0 * g0 * (1.0 - 1.0e-5));
+            const auto hi = std::lower_bound(E.begin(), E.end(), hc[c] * g1 * g1 * (1.0 + 1.0e-5));
+            const size_t i0 = lo == E.begin() ? 0 : static_cast<size_t>(lo - E.begin()) - 1;
+            const size_t i1 = hi == E.end() ? E.size() - 1 : static_cast<size_t>(hi - E.begin());
+            sum += rm[static_cast<size_t>(c)](i0, std::max(i0, i1));
+        }
+        return h.neutral_density * sum * g1;
+    };
+    double s0 = 0.0, s1 = 0.05 * lim;
+    for (int k = 0; k < 100000; ++k) {
+        // (a particle at rest is checked too when the first interval fails)
+        if (!(bound(s0, s1) < limit)) return k == 0 ? -1.0 : s0;
+        if (s0 > top + lim) break;      // constant cross sections from here on
+        s0 = s1;
+        s1 *= 1.004;
+    }
+    return s0;
+}
+
+}  // namespace
+
 // Largest relative speed below which the total collision rate of the model
 // (cold neutral) stays under max_frequency (1 - 1e-5) for every speed: the
 // per-candidate bound check (Collision.cpp:617-623) cannot fail there, with
@@ -302,7 +371,9 @@ int64_t energy_rows(int g) { return static_cast<int64_t>(g) * (kBlk / 64); }
 // linear in E = h g^2, so the rate is n (A g + B g^3), whose maximum is at an
 // end or at g^2 = -A / (3 B); the first interval whose maximum reaches the
 // limit ends the safe range.  Beyond the last breakpoint sigma is constant.
+// Thermal neutrals: thermal_safe_speed.
 double rate_safe_speed(const MccModelHost& h) {
+    if (h.neutral_vstd > 0.0) return thermal_safe_speed(h);
     const double limit = h.max_frequency * (1.0 - 1.0e-5);
     double hc[kMaxChannels];
     std::vector<double> br = {0.0};

@@ -50,7 +50,7 @@ struct MccParams {
     float half_mass;
     float neutral_mass;      // 0: infinitely heavy neutral
     float neutral_vstd;      // 0: cold neutral
-    float safe_speed;        // below it the total rate is provably under max_frequency
+    float safe_speed;        // below it the rate bound is provably under max_frequency
     // The 1D step books the kinetic energy of each ionization's secondary
     // and ion into the ionization channel (Simulation.cpp:880-902); half
     // their masses, 0 for the bare collide (NullCollisionModel::collide).
@@ -159,7 +159,10 @@ __device__ __forceinline__ bool above_bound(const MccParams& m, float total) {
     return total > m.max_frequency + 64.0f * 1.1920929e-7f * mx;
 }
 
-// Collision.cpp:627-685 for thermal neutrals: bound over the speed window
+// Collision.cpp:627-685 for thermal neutrals: bound over the speed window.
+// The largest cross section of the window is that of its ends and of the
+// table rows inside it, found by two binary searches (the energies increase)
+// instead of a pass over the whole table.
 template <int NCH>
 __device__ bool thermal_bound_exceeded(const MccParams& m, const XsView& X, float speed) {
     const float lim = 8.0f * m.neutral_vstd;
@@ -173,12 +176,16 @@ __device__ bool thermal_bound_exceeded(const MccParams& m, const XsView& X, floa
         float emin = collision_energy(m, c, vmin);
         if (emin < m.threshold[c]) emin = m.threshold[c];
         const int so = m.offset[c], eo = X.eshared ? 0 : so, n = m.rows[c];
-        float best = xs_at(X.E, X.S, eo, so, n, xs_upper(X.E, eo, n, emin), emin);
-        const float smax = xs_at(X.E, X.S, eo, so, n, xs_upper(X.E, eo, n, emax), emax);
+        const int up0 = xs_upper(X.E, eo, n, emin), up1 = xs_upper(X.E, eo, n, emax);
+        float best = xs_at(X.E, X.S, eo, so, n, up0, emin);
+        const float smax = xs_at(X.E, X.S, eo, so, n, up1, emax);
         if (smax > best) best = smax;
-        for (int i = 0; i < n; ++i)
-            if (X.E[eo + i] >= emin && X.E[eo + i] <= emax && X.S[so + i] > best)
-                best = X.S[so + i];
+        // rows with emin <= E <= emax (rows that round to one FP32 energy
+        // are all looked at)
+        int i = up0;
+        while (i > 0 && X.E[eo + i - 1] >= emin) --i;
+        for (; i < up1; ++i)
+            if (X.S[so + i] > best) best = X.S[so + i];
         bound += m.neutral_density * best * vmax;
     }
     return above_bound(m, bound);
@@ -333,7 +340,7 @@ __device__ __forceinline__ bool mcc_next_candidate(const MccParams& m, const XsV
             t.err = DEV_ERR_RATE;
             return false;
         }
-    } else if (thermal_bound_exceeded<NCH>(m, X, speed)) {
+    } else if (speed > m.safe_speed && thermal_bound_exceeded<NCH>(m, X, speed)) {
         t.err = DEV_ERR_RATE;
         return false;
     }
@@ -496,7 +503,7 @@ __device__ void mcc_collide_1v(const MccParams& m, const XsView& X, const Channe
                 t.err = DEV_ERR_RATE;
                 return;
             }
-        } else if (thermal_bound_exceeded<NCH>(m, X, speed)) {
+        } else if (speed > m.safe_speed && thermal_bound_exceeded<NCH>(m, X, speed)) {
             t.err = DEV_ERR_RATE;
             return;
         }

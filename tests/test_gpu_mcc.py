@@ -525,3 +525,50 @@ def test_1d_mcc_steps_with_sorts_inside_one_call():
         assert a[0] == b[0]
         for x, y in zip(a[1:], b[1:]):
             assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("spike_ev,height,density", [(0.05, 4.0, 1.0), (0.05, 1.2, 1.0),
+                                                     (3.0, 6.0, 1.0), (0.05, 4.0, 40.0)])
+def test_thermal_frequency_bound_at_every_speed(ctx, spike_ev, height, density):
+    """The thermal neutrals' rate bound (Collision.cpp:627-685: the largest
+    cross section over relative speeds within 8 sigma, times the largest
+    speed) raises at exactly the speeds where the formula over the whole
+    table exceeds max_frequency: below, inside and above the window of a
+    spike, at rest, and past the table; a high density makes the bound fail
+    from rest on.  Speeds whose bound is within 1e-4 of the limit (FP32
+    rounding of a few 1e-7) are left out."""
+    from aurora_pic import hip
+    mi = 4.0 * workloads.AMU
+    e = np.geomspace(1e-4, 10.0, 120)
+    sig = np.full(e.size, 1e-19)
+    sig[int(np.argmin(np.abs(e - spike_ev)))] *= height
+    ej = e * workloads.EV
+    n0, T = 1e21 * density, 300.0
+    lim = 8.0 * math.sqrt(workloads.KB * T / mi)
+    vtop = math.sqrt(2.0 * ej[-1] / mi)
+    numax = 1.5 * 1e21 * 1e-19 * (vtop + lim)
+
+    def bound(s):
+        g0, g1 = max(0.0, s - lim), s + lim
+        e0, e1 = 0.5 * mi * g0 * g0, 0.5 * mi * g1 * g1
+        inside = sig[(ej >= e0) & (ej <= e1)]
+        best = max([np.interp(e0, ej, sig), np.interp(e1, ej, sig), *inside])
+        return n0 * best * g1
+
+    sid = ctx.add_species(workloads.EV, mi, 1.0, 64)
+    gas = dict(channels=[(hip.ELASTIC, 0.0, ej, sig)], neutral_density=n0, max_frequency=numax,
+               neutral_mass=mi)
+    ctx.mcc_load(sid, gas, seed=5, neutral_temperature=T)
+    seen = set()
+    for s in np.concatenate([[0.0], np.geomspace(0.01 * lim, 2.0 * vtop, 70)]):
+        b = bound(float(s)) / numax
+        if abs(b - 1.0) < 1e-4:
+            continue
+        v = [[float(s), 0.0, 0.0]]
+        if b > 1.0:
+            with pytest.raises(hip.HipError, match="exceeds configured max_frequency"):
+                ctx.mcc_collide(v, 1e-3 / numax, step=0)
+        else:
+            ctx.mcc_collide(v, 1e-3 / numax, step=0)
+        seen.add(b > 1.0)
+    assert True in seen and (False in seen or density > 1.0)
