@@ -24,8 +24,6 @@
 #include <string>
 #include <vector>
 
-#include <rocprim/rocprim.hpp>
-
 #include "mcc_device.hpp"
 
 namespace aurora {
@@ -501,18 +499,32 @@ void validate_request(const SwarmState& s, const aurora_hip_swarm_request* r) {
 // plus one weight, and the systematic resample of the M survivors and
 // secondaries (equal weights) takes for output j the source
 // ceil((u + j) M / N) - 1, where the cumulative weight first reaches the
-// threshold (u + j) W / N.  One step is five launches: collide, scan of the
-// packed (secondaries, alive) counts, gather (survivors in order, then the
-// secondaries in parent order), resample, and a one-workgroup fold of the
-// step's tallies and samples in a fixed order.
+// threshold (u + j) W / N.  Survivors come first, in order, then the
+// secondaries in parent order.  Two forms of the same step:
+//   k_br_small    up to kBrSmall electrons: one workgroup keeps the
+//                 population in LDS and runs up to 512 steps in one launch.
+//                 A step is bound by its chain of dependent phases, so
+//                 launches are what it must not have: 512 electrons 25.0 ->
+//                 10.4 us a step (six launches before).  512 threads up to
+//                 512 electrons, else 1024 (1,024 electrons 13.8 us against
+//                 17.7; the register cap of 1024 threads costs 4 % at 512);
+//                 at 2,048 electrons (24.7 us) the launches take over (24.1)
+//   three launches per step otherwise: collide (each 256-electron chunk
+//                 compacts its survivors and secondaries in place), a
+//                 one-workgroup scan of the chunk totals that also books the
+//                 step, and the resample, which finds a source's chunk by
+//                 bisecting the scanned totals (33,000 electrons 29 us a step)
 constexpr int kBr = 256;
+constexpr int kBrSmall = 2048;
+constexpr int kBrSmallSteps = 512;
 
 struct BranchArgs {
     float* v;                    // the population, 3 x N (SoA)
-    float* pre;                  // survivors then secondaries, 3 x cap (SoA)
-    float* sec;                  // per slot: 2 secondaries x 3
-    long long* key;              // per slot: (secondaries << 32) | alive
-    long long* off;              // exclusive scan of key
+    float* pre;                  // survivors, compacted per chunk, 3 x N (SoA)
+    float* sec;                  // secondaries, per chunk 2 kBr x 3 (per slot 2 x 3 in k_br_small)
+    int32_t* tot;                // [chunks] survivors, then [chunks] secondaries
+    int32_t* off;                // their exclusive sums
+    long long* pop;              // survivors and secondaries of the step
     unsigned long long* step_counts;  // [candidates, nulls, chan...] of the step
     unsigned long long* totals;       // the same, summed over sampled steps
     unsigned* max_energy_bits;
@@ -520,62 +532,110 @@ struct BranchArgs {
     double* part;                // per resample block: sum v_x, sum energy (eV)
     double* state;               // [w, exposure, weighted[8], squared[8]]
     double* samples;             // [3][sampling]: mean v_x, mean energy, log W
-    int64_t N, cap, limit;
+    int64_t N, limit;
+    int chunks;
     float half_kick, dt, max_energy_ev, ev_per_v2;
     uint64_t seed;
     int step, burn_in, sampling;
     uint32_t attach_mask;        // channels whose collision removes the electron
 };
 
+// One electron's step: kick, energy check, collisions, kick, check.  Returns
+// whether it survives; v, t and err hold the outcome.
+template <int NCH>
+__device__ __forceinline__ bool br_electron(const BranchArgs& a, const MccParams& m,
+                                            const XsView& X, const ChannelSel* chan, int64_t p,
+                                            int step, float* v, MccTally<NCH>& t, float& emax,
+                                            uint32_t& err) {
+    v[0] += a.half_kick;
+    const float e_pre = a.ev_per_v2 * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+    emax = fmaxf(emax, e_pre);
+    if (e_pre > a.max_energy_ev) err |= DEV_ERR_ENERGY;
+    Philox rng;
+    rng.init(a.seed, 0u, static_cast<uint32_t>(p), static_cast<uint32_t>(step));
+    mcc_collide<NCH>(m, X, chan, v, a.dt, rng, t);
+    err |= t.err;
+    v[0] += a.half_kick;
+    const float e = a.ev_per_v2 * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+    emax = fmaxf(emax, e);
+    if (e > a.max_energy_ev) err |= DEV_ERR_ENERGY;
+    bool alive = true;
+#pragma unroll
+    for (int c = 0; c < NCH; ++c)
+        if (((a.attach_mask >> c) & 1u) && t.chan[c]) alive = false;
+    if (t.nsec > 2) err |= DEV_ERR_PRODUCTS;
+    return alive;
+}
+
+// the step's resample offset u
+__device__ __forceinline__ double br_offset(const BranchArgs& a, int step) {
+    Philox rng;
+    rng.init(a.seed, 1u, 0xFFFFFFFFu, static_cast<uint32_t>(step));
+    return static_cast<double>(rng.u01());
+}
+
+__device__ __forceinline__ int64_t br_source(double u, int64_t j, int64_t M, int64_t N) {
+    if (M == N) return j;
+    const int64_t s = static_cast<int64_t>(ceil((u + static_cast<double>(j)) *
+                                                static_cast<double>(M) / static_cast<double>(N))) - 1;
+    return s < 0 ? 0 : (s > M - 1 ? M - 1 : s);
+}
+
+__device__ __forceinline__ double br_energy(const BranchArgs& a, float vx, float vy, float vz) {
+    return static_cast<double>(a.ev_per_v2) *
+           (static_cast<double>(vx) * vx + static_cast<double>(vy) * vy +
+            static_cast<double>(vz) * vz);
+}
+
+// the checks of a step with A survivors and S secondaries (Swarm.cpp:1069-1100)
+__device__ __forceinline__ uint32_t br_checks(const BranchArgs& a, int64_t A, int64_t S) {
+    return (a.N + S > a.limit ? DEV_ERR_POPULATION : 0u) | (A + S == 0 ? DEV_ERR_EXTINCT : 0u);
+}
+
+__device__ __forceinline__ double br_weight(const BranchArgs& a, double w, int64_t M) {
+    return (M == a.N || M == 0) ? w : w * static_cast<double>(M) / static_cast<double>(a.N);
+}
+
 template <int NCH>
 __global__ void __launch_bounds__(kBr) k_br_collide(MccParams m, BranchArgs a) {
     __shared__ MccLds lds;
+    __shared__ int wsum[kBr / 64];
     const XsView X = stage_tables(m, lds);
     const bool sampling = a.step >= a.burn_in;
-    for (int64_t base = static_cast<int64_t>(blockIdx.x) * kBr; base < a.N;
-         base += static_cast<int64_t>(gridDim.x) * kBr) {
-        const int64_t p = base + threadIdx.x;
+    float emax = 0.f;
+    uint32_t err = 0;
+    for (int chunk = blockIdx.x; chunk < a.chunks; chunk += gridDim.x) {
+        const int64_t first = static_cast<int64_t>(chunk) * kBr, p = first + threadIdx.x;
         const bool active = p < a.N;
         MccTally<NCH> t{};
-        uint32_t err = 0;
+        float v[3] = {0.f, 0.f, 0.f};
+        bool alive = false;
         if (active) {
-            float v[3] = {a.v[p], a.v[a.N + p], a.v[2 * a.N + p]};
-            float emax = 0.f;
-            v[0] += a.half_kick;
-            const float e_pre = a.ev_per_v2 * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-            emax = fmaxf(emax, e_pre);
-            if (e_pre > a.max_energy_ev) err |= DEV_ERR_ENERGY;
-            Philox rng;
-            rng.init(a.seed, 0u, static_cast<uint32_t>(p), static_cast<uint32_t>(a.step));
-            mcc_collide<NCH>(m, X, lds.chan, v, a.dt, rng, t);
-            err |= t.err;
-            v[0] += a.half_kick;
-            const float e = a.ev_per_v2 * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-            emax = fmaxf(emax, e);
-            if (e > a.max_energy_ev) err |= DEV_ERR_ENERGY;
-            long long alive = 1;
-#pragma unroll
-            for (int c = 0; c < NCH; ++c)
-                if (((a.attach_mask >> c) & 1u) && t.chan[c]) alive = 0;
-            int ns = t.nsec;
-            if (ns > 2) {
-                err |= DEV_ERR_PRODUCTS;
-                ns = 2;
-            }
-            // both slots unrolled: a runtime index into t.sec would put the
-            // tally in scratch memory
-#pragma unroll
-            for (int k = 0; k < 2; ++k)
-                if (k < ns)
-#pragma unroll
-                    for (int d = 0; d < 3; ++d) a.sec[6 * p + 3 * k + d] = t.sec[k][d];
-            a.v[p] = v[0];
-            a.v[a.N + p] = v[1];
-            a.v[2 * a.N + p] = v[2];
-            a.key[p] = (static_cast<long long>(ns) << 32) | alive;
-            atomicMax(a.max_energy_bits, __float_as_uint(emax));
-            if (err) atomicOr(a.status, err);
+            v[0] = a.v[p]; v[1] = a.v[a.N + p]; v[2] = a.v[2 * a.N + p];
+            alive = br_electron<NCH>(a, m, X, lds.chan, p, a.step, v, t, emax, err);
         }
+        const int ns = active ? (t.nsec < 2 ? t.nsec : 2) : 0;
+        // survivors (at most 256) and secondaries (512) in one scan
+        int total = 0;
+        const int ex = block_scan_int<kBr>((alive ? 1 : 0) | (ns << 16), wsum, total);
+        if (threadIdx.x == 0) {
+            a.tot[chunk] = total & 0xffff;
+            a.tot[a.chunks + chunk] = total >> 16;
+        }
+        if (alive) {
+            const int64_t d = first + (ex & 0xffff);
+            a.pre[d] = v[0];
+            a.pre[a.N + d] = v[1];
+            a.pre[2 * a.N + d] = v[2];
+        }
+        float* sec = a.sec + 3 * (2 * first + (ex >> 16));
+        // both slots unrolled: a runtime index into t.sec would put the
+        // tally in scratch memory
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if (k < ns)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) sec[3 * k + d] = t.sec[k][d];
         if (sampling) {
             unsigned long long cnt[2 + NCH];
             cnt[0] = active ? t.candidates : 0;
@@ -584,94 +644,47 @@ __global__ void __launch_bounds__(kBr) k_br_collide(MccParams m, BranchArgs a) {
             for (int c = 0; c < NCH; ++c) cnt[2 + c] = active ? t.chan[c] : 0;
 #pragma unroll
             for (int k = 0; k < 2 + NCH; ++k) {
-                unsigned long long x = cnt[k];
-                for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o, 64);
+                const unsigned long long x = wave_sum_u64(cnt[k]);
                 if ((threadIdx.x & 63) == 0 && x) atomicAdd(a.step_counts + k, x);
             }
         }
     }
-}
-
-__device__ __forceinline__ void br_totals(const BranchArgs& a, int64_t& A, int64_t& S) {
-    const long long tot = a.off[a.N - 1] + a.key[a.N - 1];
-    A = tot & 0xffffffffll;
-    S = tot >> 32;
-}
-
-__global__ void __launch_bounds__(kBr) k_br_gather(BranchArgs a) {
-    int64_t A, S;
-    br_totals(a, A, S);
-    for (int64_t p = blockIdx.x * static_cast<int64_t>(kBr) + threadIdx.x; p < a.N;
-         p += static_cast<int64_t>(gridDim.x) * kBr) {
-        const long long k = a.key[p], o = a.off[p];
-        const int ns = static_cast<int>(k >> 32);
-        if (k & 1) {
-            const int64_t d = o & 0xffffffffll;
-            a.pre[d] = a.v[p];
-            a.pre[a.cap + d] = a.v[a.N + p];
-            a.pre[2 * a.cap + d] = a.v[2 * a.N + p];
-        }
-        const int64_t d0 = A + (o >> 32);
-        for (int i = 0; i < ns; ++i) {
-            a.pre[d0 + i] = a.sec[6 * p + 3 * i];
-            a.pre[a.cap + d0 + i] = a.sec[6 * p + 3 * i + 1];
-            a.pre[2 * a.cap + d0 + i] = a.sec[6 * p + 3 * i + 2];
-        }
+    for (int o = 32; o > 0; o >>= 1) {
+        emax = fmaxf(emax, __shfl_xor(emax, o, 64));
+        err |= __shfl_xor(err, o, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicMax(a.max_energy_bits, __float_as_uint(emax));
+        if (err) atomicOr(a.status, err);
     }
 }
 
-__global__ void __launch_bounds__(kBr) k_br_resample(BranchArgs a) {
-    int64_t A, S;
-    br_totals(a, A, S);
-    const int64_t M = A + S;
-    Philox rng;
-    rng.init(a.seed, 1u, 0xFFFFFFFFu, static_cast<uint32_t>(a.step));
-    const double u = static_cast<double>(rng.u01());
-    double sums[2] = {0.0, 0.0};
-    for (int64_t j = blockIdx.x * static_cast<int64_t>(kBr) + threadIdx.x; j < a.N;
-         j += static_cast<int64_t>(gridDim.x) * kBr) {
-        if (M == 0) break;                     // extinct: the fold reports it
-        int64_t src = j;
-        if (M != a.N) {
-            src = static_cast<int64_t>(ceil((u + static_cast<double>(j)) *
-                                            static_cast<double>(M) / static_cast<double>(a.N))) - 1;
-            src = src < 0 ? 0 : (src > M - 1 ? M - 1 : src);
-        }
-        const float vx = a.pre[src], vy = a.pre[a.cap + src], vz = a.pre[2 * a.cap + src];
-        a.v[j] = vx;
-        a.v[a.N + j] = vy;
-        a.v[2 * a.N + j] = vz;
-        sums[0] += vx;
-        sums[1] += static_cast<double>(a.ev_per_v2) *
-                   (static_cast<double>(vx) * vx + static_cast<double>(vy) * vy +
-                    static_cast<double>(vz) * vz);
-    }
-    const double r = block_sum<2, kBr>(sums);
-    if (threadIdx.x < 2) a.part[2 * blockIdx.x + threadIdx.x] = r;
-}
-
-// one workgroup: the step's checks, weights, tallies and samples
-__global__ void __launch_bounds__(kBr) k_br_fold(BranchArgs a, int blocks, int nch) {
-    int64_t A, S;
-    br_totals(a, A, S);
-    const int64_t M = A + S;
-    double v[2] = {0.0, 0.0};
-    for (int b = threadIdx.x; b < blocks; b += kBr) {
-        v[0] += a.part[2 * b];
-        v[1] += a.part[2 * b + 1];
-    }
-    const double sum = block_sum<2, kBr>(v);
-    __shared__ double sums[2];
-    if (threadIdx.x < 2) sums[threadIdx.x] = sum;
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    uint32_t err = 0;
-    if (a.N + S > a.limit) err |= DEV_ERR_POPULATION;   // Swarm.cpp:1069-1075
-    if (M == 0) err |= DEV_ERR_EXTINCT;                 // Swarm.cpp:1095-1100
-    if (err) atomicOr(a.status, err);
-    const double w = a.state[0];
+// One workgroup between a step's collide and resample: the previous step's
+// sample sums (fold), then (scan) the chunk totals scanned, the step's checks,
+// weight and tallies booked.
+__global__ void __launch_bounds__(kBr) k_br_book(BranchArgs a, int blocks, int nch, int fold,
+                                                 int scan) {
+    __shared__ int wsum[kBr / 64];
     const double n = static_cast<double>(a.N);
-    const double w_new = (M == a.N || M == 0) ? w : w * static_cast<double>(M) / n;
+    if (fold) {
+        double v[2] = {0.0, 0.0};
+        for (int b = threadIdx.x; b < blocks; b += kBr) {
+            v[0] += a.part[2 * b];
+            v[1] += a.part[2 * b + 1];
+        }
+        const double sum = block_sum<2, kBr>(v);
+        const int64_t k = a.step - 1 - a.burn_in;
+        if (threadIdx.x < 2) a.samples[threadIdx.x * a.sampling + k] = sum / n;
+    }
+    if (!scan) return;
+    const int64_t A = chunk_offsets<kBr>(a.tot, a.off, a.chunks, wsum);
+    const int64_t S = chunk_offsets<kBr>(a.tot + a.chunks, a.off + a.chunks, a.chunks, wsum);
+    if (threadIdx.x != 0) return;
+    a.pop[0] = A;
+    a.pop[1] = S;
+    const uint32_t err = br_checks(a, A, S);
+    if (err) atomicOr(a.status, err);
+    const double w = a.state[0], w_new = br_weight(a, w, A + S);
     a.state[0] = w_new;
     if (a.step >= a.burn_in) {
         a.state[1] += n * w * static_cast<double>(a.dt);
@@ -681,12 +694,249 @@ __global__ void __launch_bounds__(kBr) k_br_fold(BranchArgs a, int blocks, int n
             a.state[10 + c] += w * w * k;
         }
         for (int c = 0; c < 2 + nch; ++c) a.totals[c] += a.step_counts[c];
-        const int64_t k = a.step - a.burn_in;
-        a.samples[k] = sums[0] / n;
-        a.samples[a.sampling + k] = sums[1] / n;
-        a.samples[2 * a.sampling + k] = log(n * w_new);
+        a.samples[2 * static_cast<int64_t>(a.sampling) + a.step - a.burn_in] = log(n * w_new);
     }
     for (int c = 0; c < 2 + nch; ++c) a.step_counts[c] = 0;
+}
+
+// the chunk holding element x of the scanned totals: the last one whose
+// offset does not exceed x
+__device__ __forceinline__ int br_chunk_of(const int32_t* off, int chunks, int64_t x) {
+    int lo = 0, hi = chunks;          // off[0] = 0 <= x
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (off[mid] <= x) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+
+__global__ void __launch_bounds__(kBr) k_br_resample(BranchArgs a) {
+    const int64_t A = a.pop[0], M = A + a.pop[1];
+    const double u = br_offset(a, a.step);
+    double sums[2] = {0.0, 0.0};
+    for (int64_t j = blockIdx.x * static_cast<int64_t>(kBr) + threadIdx.x; j < a.N;
+         j += static_cast<int64_t>(gridDim.x) * kBr) {
+        if (M == 0) break;                     // extinct: reported by the booking
+        const int64_t src = br_source(u, j, M, a.N);
+        float vx, vy, vz;
+        if (src < A) {
+            const int c = br_chunk_of(a.off, a.chunks, src);
+            const int64_t d = static_cast<int64_t>(c) * kBr + (src - a.off[c]);
+            vx = a.pre[d]; vy = a.pre[a.N + d]; vz = a.pre[2 * a.N + d];
+        } else {
+            const int32_t* off = a.off + a.chunks;
+            const int c = br_chunk_of(off, a.chunks, src - A);
+            const float* q = a.sec + 3 * (2 * static_cast<int64_t>(c) * kBr + (src - A - off[c]));
+            vx = q[0]; vy = q[1]; vz = q[2];
+        }
+        a.v[j] = vx;
+        a.v[a.N + j] = vy;
+        a.v[2 * a.N + j] = vz;
+        sums[0] += vx;
+        sums[1] += br_energy(a, vx, vy, vz);
+    }
+    const double r = block_sum<2, kBr>(sums);
+    if (threadIdx.x < 2) a.part[2 * blockIdx.x + threadIdx.x] = r;
+}
+
+// Steps [a.step, a.step + nsteps) of a population of at most kBrSmall by one
+// workgroup.  Thread t owns electrons t, t + T, ...; a step has three
+// phases with a barrier after the first two:
+//   collide   each wave counts its survivors and secondaries per round
+//   place     the (round, wave) counts are scanned by every wave on its own,
+//             survivors and secondaries go to their order in pre (LDS;
+//             entries past twice the population to the global overflow);
+//             wave 0 books the step and the previous step's sample sums
+//   resample  each thread reads its electrons' sources
+// LDS: v[3][N], pre[3][2N], meta[N].
+template <int NCH, int T>
+__global__ void __launch_bounds__(T) k_br_small(MccParams m, BranchArgs a, int nsteps,
+                                                float* overflow) {
+    constexpr int W = T / 64, kRounds = kBrSmall / T;
+    extern __shared__ __align__(16) float br_lds[];
+    __shared__ MccLds lds;
+    __shared__ uint32_t s_wave[kRounds * W];       // survivors | secondaries << 16
+    __shared__ uint32_t s_cnt[2][2 + NCH];
+    __shared__ double s_red[2][W];
+    static_assert(kRounds * W <= 64, "one wave scans the (round, wave) counts");
+    const int N = static_cast<int>(a.N), cap = 2 * N;
+    float* v = br_lds;
+    float* pre = br_lds + 3 * N;
+    uint32_t* meta = reinterpret_cast<uint32_t*>(br_lds + 9 * N);
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int rounds = (N + T - 1) / T;
+    for (int p = tid; p < N; p += T)
+        for (int d = 0; d < 3; ++d) v[d * N + p] = a.v[d * a.N + p];
+    if (tid < 2 * (2 + NCH)) (&s_cnt[0][0])[tid] = 0u;
+    const XsView X = stage_tables(m, lds);         // ends with a barrier
+    // wave 0 keeps the running state: w in every lane, lane c its channel's
+    // sums and (c < 2 + NCH) counter c
+    double w = a.state[0], exposure = a.state[1];
+    double weighted = 0.0, squared = 0.0;
+    unsigned long long counted = 0;
+    if (wid == 0 && lane < NCH) {
+        weighted = a.state[2 + lane];
+        squared = a.state[10 + lane];
+    }
+    if (wid == 0 && lane < 2 + NCH) counted = a.totals[lane];
+    const double n = static_cast<double>(N);
+    double* vel_samples = a.samples;
+    double* log_samples = a.samples + 2 * static_cast<int64_t>(a.sampling);
+    auto book_sums = [&](int step) {               // the sums of `step`, by wave 0
+        if (step < a.burn_in || lane >= 2) return;
+        double sum = 0.0;
+#pragma unroll
+        for (int k = 0; k < W; ++k) sum += s_red[lane][k];
+        vel_samples[lane * static_cast<int64_t>(a.sampling) + step - a.burn_in] = sum / n;
+    };
+    float emax = 0.f;
+    uint32_t err = 0;
+    for (int it = 0; it < nsteps; ++it) {
+        const int step = a.step + it;
+        const bool sampling = step >= a.burn_in;
+        uint32_t* cnt = s_cnt[it & 1];
+        for (int k = 0; k < rounds; ++k) {
+            const int p = tid + k * T;
+            const bool active = p < N;
+            MccTally<NCH> t{};
+            bool alive = false;
+            if (active) {
+                float u[3] = {v[p], v[N + p], v[2 * N + p]};
+                alive = br_electron<NCH>(a, m, X, lds.chan, p, step, u, t, emax, err);
+                v[p] = u[0];
+                v[N + p] = u[1];
+                v[2 * N + p] = u[2];
+            }
+            const int ns = active ? (t.nsec < 2 ? t.nsec : 2) : 0;
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                if (q < ns)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) a.sec[6 * p + 3 * q + d] = t.sec[q][d];
+            const uint64_t ma = __ballot(alive), m1 = __ballot(ns > 0), m2 = __ballot(ns > 1);
+            const uint64_t below = (uint64_t{1} << lane) - 1;
+            if (active)
+                meta[p] = (alive ? 1u : 0u) | (static_cast<uint32_t>(ns) << 1) |
+                          (static_cast<uint32_t>(__popcll(ma & below)) << 8) |
+                          (static_cast<uint32_t>(__popcll(m1 & below) + __popcll(m2 & below)) << 16);
+            if (lane == 0)
+                s_wave[k * W + wid] = static_cast<uint32_t>(__popcll(ma)) |
+                                      (static_cast<uint32_t>(__popcll(m1) + __popcll(m2)) << 16);
+            if (sampling && active && t.candidates) {
+                atomicAdd(cnt, t.candidates);
+                if (t.nulls) atomicAdd(cnt + 1, t.nulls);
+#pragma unroll
+                for (int c = 0; c < NCH; ++c)
+                    if (t.chan[c]) atomicAdd(cnt + 2 + c, t.chan[c]);
+            }
+        }
+        __syncthreads();
+        // at most 2048 survivors and 4096 secondaries: both halves stay below 2^16
+        uint32_t x = lane < rounds * W ? s_wave[lane] : 0u, incl = x;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t y = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += y;
+        }
+        const uint32_t total = __shfl(incl, 63, 64), excl = incl - x;
+        const int A = static_cast<int>(total & 0xffffu), S = static_cast<int>(total >> 16);
+        const int M = A + S;
+        auto place = [&](int d, float x0, float x1, float x2) {
+            if (d < cap) {
+                pre[d] = x0;
+                pre[cap + d] = x1;
+                pre[2 * cap + d] = x2;
+            } else {
+                overflow[3 * (d - cap)] = x0;
+                overflow[3 * (d - cap) + 1] = x1;
+                overflow[3 * (d - cap) + 2] = x2;
+            }
+        };
+        for (int k = 0; k < rounds; ++k) {
+            const uint32_t base = __shfl(excl, k * W + wid, 64);
+            const int p = tid + k * T;
+            if (p >= N) continue;
+            const uint32_t mt = meta[p];
+            if (mt & 1u)
+                place(static_cast<int>((base & 0xffffu) + ((mt >> 8) & 0xffu)), v[p], v[N + p],
+                      v[2 * N + p]);
+            const int ns = static_cast<int>((mt >> 1) & 3u);
+            for (int q = 0; q < ns; ++q)
+                place(A + static_cast<int>((base >> 16) + (mt >> 16)) + q, a.sec[6 * p + 3 * q],
+                      a.sec[6 * p + 3 * q + 1], a.sec[6 * p + 3 * q + 2]);
+        }
+        if (wid == 0) {
+            if (it > 0) book_sums(step - 1);
+            err |= br_checks(a, A, S);
+            const double w_new = br_weight(a, w, M);
+            if (sampling) {
+                exposure += n * w * static_cast<double>(a.dt);
+                if (lane < NCH) {
+                    const double k = static_cast<double>(cnt[2 + lane]);
+                    weighted += w * k;
+                    squared += w * w * k;
+                }
+                if (lane < 2 + NCH) counted += cnt[lane];
+                // (the logarithm is taken for all steps of the launch at its end)
+                if (lane == 0) log_samples[step - a.burn_in] = n * w_new;
+            }
+            w = w_new;
+            if (lane < 2 + NCH) cnt[lane] = 0u;
+        }
+        __syncthreads();
+        const double u = br_offset(a, step);
+        double sums[2] = {0.0, 0.0};
+        if (M > 0)                                 // else extinct: reported
+            for (int p = tid; p < N; p += T) {
+                const int src = static_cast<int>(br_source(u, p, M, N));
+                float vx, vy, vz;
+                if (src < cap) {
+                    vx = pre[src]; vy = pre[cap + src]; vz = pre[2 * cap + src];
+                } else {
+                    const float* q = overflow + 3 * (src - cap);
+                    vx = q[0]; vy = q[1]; vz = q[2];
+                }
+                v[p] = vx;
+                v[N + p] = vy;
+                v[2 * N + p] = vz;
+                sums[0] += vx;
+                sums[1] += br_energy(a, vx, vy, vz);
+            }
+        if (sampling) {
+            const double s0 = wave_sum(sums[0]), s1 = wave_sum(sums[1]);
+            if (lane == 0) {
+                s_red[0][wid] = s0;
+                s_red[1][wid] = s1;
+            }
+        }
+    }
+    __syncthreads();
+    if (wid == 0) {
+        book_sums(a.step + nsteps - 1);
+        if (lane == 0) {
+            a.state[0] = w;
+            a.state[1] = exposure;
+        }
+        if (lane < NCH) {
+            a.state[2 + lane] = weighted;
+            a.state[10 + lane] = squared;
+        }
+        if (lane < 2 + NCH) a.totals[lane] = counted;
+    }
+    for (int it = tid; it < nsteps; it += T) {
+        const int k = a.step + it - a.burn_in;
+        if (k >= 0) log_samples[k] = log(log_samples[k]);
+    }
+    for (int p = tid; p < N; p += T)
+        for (int d = 0; d < 3; ++d) a.v[d * a.N + p] = v[d * N + p];
+    for (int o = 32; o > 0; o >>= 1) {
+        emax = fmaxf(emax, __shfl_xor(emax, o, 64));
+        err |= __shfl_xor(err, o, 64);
+    }
+    if (lane == 0) {
+        atomicMax(a.max_energy_bits, __float_as_uint(emax));
+        if (err) atomicOr(a.status, err);
+    }
 }
 
 // block_slope_and_error (Swarm.cpp:136-197)
@@ -1011,23 +1261,29 @@ int aurora_hip_swarm_branching(aurora_hip_ctx* h, const aurora_hip_swarm_request
         }
         AUR_REQUIRE(creates, AURORA_ERR_INVALID_ARGUMENT,
                     "branching swarm requires an ionization or attachment channel");
-        const int64_t cap = 3 * N;
+        const bool small = N <= kBrSmall;
         const int nch = s.gas.nchan;
+        const int chunks = static_cast<int>((N + kBr - 1) / kBr);
         DevBuf<float> v, pre, sec;
-        DevBuf<long long> key, off;
+        DevBuf<int32_t> ctot, coff;
+        DevBuf<long long> pop;
         DevBuf<unsigned long long> counts;     // step counters, then totals
         DevBuf<unsigned> maxe;
         DevBuf<uint32_t> status;
         DevBuf<double> part, st, samples;
         v.alloc(static_cast<size_t>(3 * N));
-        pre.alloc(static_cast<size_t>(3 * cap));
-        sec.alloc(static_cast<size_t>(6 * N));
-        key.alloc(static_cast<size_t>(N));
-        off.alloc(static_cast<size_t>(N));
+        // survivors; in the small form the entries past twice the population
+        pre.alloc(static_cast<size_t>(3 * N));
+        sec.alloc(static_cast<size_t>(6) * chunks * kBr);
+        if (!small) {
+            ctot.alloc(static_cast<size_t>(2 * chunks));
+            coff.alloc(static_cast<size_t>(2 * chunks));
+            pop.alloc(2);
+        }
         counts.alloc(2 * (kMaxChannels + 2));
         maxe.alloc(1);
         status.alloc(1);
-        int64_t g = (N + kBr - 1) / kBr;
+        int64_t g = chunks;
         if (g > static_cast<int64_t>(c.cu_count) * 8) g = static_cast<int64_t>(c.cu_count) * 8;
         part.alloc(static_cast<size_t>(2 * g));
         st.alloc(18);
@@ -1042,18 +1298,13 @@ int aurora_hip_swarm_branching(aurora_hip_ctx* h, const aurora_hip_swarm_request
         k_swarm_init<<<static_cast<unsigned>(std::min<int64_t>(g, 4096)), 256, 0, c.stream>>>(
             v.ptr, v.ptr + N, v.ptr + 2 * N, N, static_cast<float>(sigma), r->seed);
         AUR_HIP(hipGetLastError());
-        size_t temp = 0;
-        AUR_HIP(rocprim::exclusive_scan(nullptr, temp, key.ptr, off.ptr, 0LL,
-                                        static_cast<size_t>(N), rocprim::plus<long long>(),
-                                        c.stream));
-        DevBuf<unsigned char> scratch;
-        scratch.alloc(temp > 0 ? temp : 1);
         BranchArgs a{};
         a.v = v.ptr;
         a.pre = pre.ptr;
         a.sec = sec.ptr;
-        a.key = key.ptr;
-        a.off = off.ptr;
+        a.tot = ctot.ptr;
+        a.off = coff.ptr;
+        a.pop = pop.ptr;
         a.step_counts = counts.ptr;
         a.totals = counts.ptr + kMaxChannels + 2;
         a.max_energy_bits = maxe.ptr;
@@ -1062,8 +1313,8 @@ int aurora_hip_swarm_branching(aurora_hip_ctx* h, const aurora_hip_swarm_request
         a.state = st.ptr;
         a.samples = samples.ptr;
         a.N = N;
-        a.cap = cap;
         a.limit = population_limit;
+        a.chunks = chunks;
         const double efield = r->reduced_field_td * kTownsend * s.gas.neutral_density;
         a.half_kick = static_cast<float>(0.5 * (-kElementaryCharge * efield / kElectronMass) *
                                          r->timestep);
@@ -1109,19 +1360,36 @@ int aurora_hip_swarm_branching(aurora_hip_ctx* h, const aurora_hip_swarm_request
         };
         {
             KernelScope ks(c, "swarm_branching");
-            for (int64_t step = 0; step < r->steps; ++step) {
+            // errors are looked for every 512 steps (kBrSmallSteps)
+            for (int64_t step = 0; small && step < r->steps; step += kBrSmallSteps) {
+                a.step = static_cast<int>(step);
+                const int k = static_cast<int>(std::min<int64_t>(kBrSmallSteps, r->steps - step));
+                const size_t shmem = static_cast<size_t>(10 * N) * sizeof(float);
+                with_nchan(m.nchan, [&]<int NCH>() {
+                    if (N <= 512)
+                        k_br_small<NCH, 512><<<1, 512, shmem, c.stream>>>(m, a, k, pre.ptr);
+                    else
+                        k_br_small<NCH, 1024><<<1, 1024, shmem, c.stream>>>(m, a, k, pre.ptr);
+                });
+                AUR_HIP(hipGetLastError());
+                if (step + k < r->steps) check();
+            }
+            for (int64_t step = 0; !small && step < r->steps; ++step) {
                 a.step = static_cast<int>(step);
                 with_nchan(m.nchan, [&]<int NCH>() {
                     k_br_collide<NCH><<<static_cast<unsigned>(g), kBr, 0, c.stream>>>(m, a);
                 });
-                AUR_HIP(rocprim::exclusive_scan(scratch.ptr, temp, key.ptr, off.ptr, 0LL,
-                                                static_cast<size_t>(N),
-                                                rocprim::plus<long long>(), c.stream));
-                k_br_gather<<<static_cast<unsigned>(g), kBr, 0, c.stream>>>(a);
+                k_br_book<<<1, kBr, 0, c.stream>>>(a, static_cast<int>(g), nch,
+                                                   step > r->burn_in ? 1 : 0, 1);
                 k_br_resample<<<static_cast<unsigned>(g), kBr, 0, c.stream>>>(a);
-                k_br_fold<<<1, kBr, 0, c.stream>>>(a, static_cast<int>(g), nch);
                 AUR_HIP(hipGetLastError());
                 if ((step & 511) == 511) check();
+            }
+            if (!small) {
+                // the last step's sample sums
+                a.step = static_cast<int>(r->steps);
+                k_br_book<<<1, kBr, 0, c.stream>>>(a, static_cast<int>(g), nch, 1, 0);
+                AUR_HIP(hipGetLastError());
             }
         }
         check();

@@ -128,3 +128,46 @@ def test_branching_needs_a_creation_channel():
     with pytest.raises(hip.HipError, match="requires an ionization or attachment channel"):
         c.swarm_branching(gasdata.swarm_requests(cfg)[0], 10_000)
     c.close()
+
+
+@pytest.mark.parametrize("particles", [63, 64, 512, 513, 1025, 2048, 2049, 4500])
+@pytest.mark.parametrize("attaching", [False, True])
+def test_branching_step_matches_oracle_same_stream(bctx, oracle, particles, attaching):
+    """Twenty hot steps (60 eV: several ionizations a step; with a strong
+    attachment cross section also several losses) from the oracle's Philox
+    stream, at the edges of a wave, of a round of the one-workgroup form and
+    of its range: the same collision counts, so the same survivors, order and
+    resample sources throughout, the same weight (a product of ratios of those
+    integers, FP64) and mean energy and drift to FP32 rounding.  A decision
+    flips between FP32 and FP64 about once in 1e6; these runs make 1e4."""
+    import math
+
+    import oracle_py
+    from test_branching_swarm import model_vstd, strong_attachment_gas
+    from test_gpu_swarm import _initial_velocities
+    c, cfg, ds, gas = bctx
+    if attaching:
+        gas = strong_attachment_gas(gas)
+        c.swarm_gas(gas)
+        gasdata.apply_channel_options(c, ds, model=1)
+    opts = {k: (ch.angular, ch.energy_frame, ch.mean_cosine_energy, ch.mean_cosine)
+            for k, ch in enumerate(ds.channels)}
+    model = oracle_py.model_from_gas(gas, neutral_vstd=model_vstd(cfg, ds), options=opts)
+    q = gasdata.swarm_requests(cfg)[2]
+    q.particles, q.steps, q.burn_in, q.blocks = particles, 20, 10, 5
+    q.initial_mean_energy_ev, q.seed = 60.0, 77
+    r, g = c.swarm_branching(q, 2 * particles)
+    o, og = oracle.swarm_branching(
+        model, dict(neutral_density=cfg.neutral_density, max_frequency=cfg.max_frequency,
+                    timestep=cfg.timestep, reduced_field_td=q.reduced_field_td, steps=20,
+                    burn_in=10, particles=particles, blocks=5, initial_mean_energy_ev=60.0,
+                    max_energy_ev=cfg.max_energy_ev),
+        _initial_velocities(oracle, particles, 60.0, 77), 77, 2 * particles)
+    assert r.status == 0 and o.status == 0
+    assert (r.candidates, r.nulls) == (o.candidates, o.nulls)
+    assert list(r.collisions)[:4] == list(o.collisions)[:4]
+    assert math.isclose(g.final_weight, og.final_weight, rel_tol=1e-12)
+    assert math.isclose(r.mean_energy_ev, o.mean_energy_ev, rel_tol=1e-5)
+    assert abs(r.drift - o.drift) <= 1e-5 * math.sqrt(2 * 60.0 / 5.68563e-12)
+    if particles >= 512:
+        assert g.final_weight != g.initial_weight
