@@ -465,6 +465,12 @@ MccParams mcc_params_of(const MccModelHost& h) {
     m.safe_speed = std::isfinite(gs) && gs < 3.0e38
                        ? std::nextafter(static_cast<float>(gs), 0.0f) * (1.0f - 1.0e-6f)
                        : 3.0e38f;
+    // a squared speed's FP32 evaluation is off by a few 1e-7
+    m.safe_speed2 = m.safe_speed < 0.0f
+                        ? -1.0f
+                        : static_cast<float>(std::min(
+                              3.0e38, (1.0 - 1.0e-5) * static_cast<double>(m.safe_speed) *
+                                          static_cast<double>(m.safe_speed)));
     return m;
 }
 

@@ -51,6 +51,7 @@ struct MccParams {
     float neutral_mass;      // 0: infinitely heavy neutral
     float neutral_vstd;      // 0: cold neutral
     float safe_speed;        // below it the rate bound is provably under max_frequency
+    float safe_speed2;       // just under its square: the check is looked at only above
     // The 1D step books the kinetic energy of each ionization's secondary
     // and ion into the ionization channel (Simulation.cpp:880-902); half
     // their masses, 0 for the bare collide (NullCollisionModel::collide).
@@ -93,6 +94,15 @@ void with_nchan(int nchan, F&& f) {
         case 7: f.template operator()<7>(); break;
         default: f.template operator()<8>(); break;
     }
+}
+
+// with_nchan plus where the tables live: f.template operator()<NCH, LDS>().
+template <typename F>
+void with_model(int nchan, bool lds, F&& f) {
+    with_nchan(nchan, [&]<int NCH>() {
+        if (lds) f.template operator()<NCH, true>();
+        else f.template operator()<NCH, false>();
+    });
 }
 
 // Linear interpolation with constant extrapolation (Collision.cpp:221-237,
@@ -321,6 +331,18 @@ __device__ __forceinline__ void apply_channel(const MccParams& m, const ChannelS
     }
 }
 
+// validate_frequency_bound before a waiting time (Collision.cpp:617-632):
+// below safe_speed it cannot fail, so it is evaluated only above
+template <int NCH>
+__device__ __forceinline__ bool mcc_rate_fails(const MccParams& m, const XsView& X,
+                                               const float* v) {
+    const float speed = sqrtf(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+    if (!(speed > m.safe_speed)) return false;
+    if (m.neutral_vstd != 0.f) return thermal_bound_exceeded<NCH>(m, X, speed);
+    float rate[NCH];
+    return above_bound(m, mcc_rates<NCH>(m, X, speed, rate));
+}
+
 // The candidate loop of one particle-step, in two resumable pieces (the
 // swarm kernel interleaves particles' candidates): mcc_next_candidate is the
 // loop top -- the rate-bound checks at the current speed, then the next
@@ -331,16 +353,7 @@ template <int NCH, typename Tally>
 __device__ __forceinline__ bool mcc_next_candidate(const MccParams& m, const XsView& X,
                                                    const float* v, float dt, Philox& rng,
                                                    float& elapsed, Tally& t) {
-    float rate[NCH];
-    const float speed = sqrtf(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-    if (m.neutral_vstd == 0.f) {
-        // validate_frequency_bound (Collision.cpp:627-632): below
-        // safe_speed the check cannot fail, so it is evaluated only above
-        if (speed > m.safe_speed && above_bound(m, mcc_rates<NCH>(m, X, speed, rate))) {
-            t.err = DEV_ERR_RATE;
-            return false;
-        }
-    } else if (speed > m.safe_speed && thermal_bound_exceeded<NCH>(m, X, speed)) {
+    if (mcc_rate_fails<NCH>(m, X, v)) {
         t.err = DEV_ERR_RATE;
         return false;
     }
@@ -881,7 +894,15 @@ struct MccLds {
     ChannelSel chan[kMaxChannels];
 };
 
-__device__ __forceinline__ XsView stage_tables(const MccParams& m, MccLds& lds) {
+// energy rows staged: one grid for all channels, or every channel's
+__host__ __device__ __forceinline__ int mcc_energy_rows(const MccParams& m) {
+    return m.grid_shared ? m.rows[0] : m.total_rows;
+}
+inline bool mcc_tables_fit(const MccParams& m) {
+    return mcc_energy_rows(m) + m.total_rows <= kMccLdsWords;
+}
+
+__device__ __forceinline__ void stage_channels(const MccParams& m, MccLds& lds) {
     if (threadIdx.x == 0) {
 #pragma unroll
         for (int k = 0; k < kMaxChannels; ++k)
@@ -889,8 +910,12 @@ __device__ __forceinline__ XsView stage_tables(const MccParams& m, MccLds& lds) 
                 lds.chan[k] = ChannelSel{m.kind[k], m.angular[k], m.threshold[k], m.half_emass[k],
                                          m.mc_offset[k], m.mc_rows[k]};
     }
+}
+
+__device__ __forceinline__ XsView stage_tables(const MccParams& m, MccLds& lds) {
+    stage_channels(m, lds);
     XsView X{m.energy, m.sigma, 0};
-    const int ne = m.grid_shared ? m.rows[0] : m.total_rows;
+    const int ne = mcc_energy_rows(m);
     if (ne + m.total_rows <= kMccLdsWords) {
         for (int i = threadIdx.x; i < ne; i += blockDim.x) lds.words[i] = m.energy[i];
         for (int i = threadIdx.x; i < m.total_rows; i += blockDim.x)
@@ -899,6 +924,28 @@ __device__ __forceinline__ XsView stage_tables(const MccParams& m, MccLds& lds) 
     }
     __syncthreads();
     return X;
+}
+
+// The same with the choice made at compile time (LDS: mcc_tables_fit): the
+// tables' address space is known, so their reads are LDS reads and not
+// generic ones.
+template <bool LDS>
+__device__ __forceinline__ void stage_tables_as(const MccParams& m, MccLds& lds) {
+    stage_channels(m, lds);
+    if constexpr (LDS) {
+        const int ne = mcc_energy_rows(m);
+        for (int i = threadIdx.x; i < ne; i += blockDim.x) lds.words[i] = m.energy[i];
+        for (int i = threadIdx.x; i < m.total_rows; i += blockDim.x)
+            lds.words[ne + i] = m.sigma[i];
+    }
+    __syncthreads();
+}
+template <bool LDS>
+__device__ __forceinline__ XsView table_view(const MccParams& m, const MccLds& lds) {
+    if constexpr (LDS)
+        return XsView{lds.words, lds.words + mcc_energy_rows(m), m.grid_shared};
+    else
+        return XsView{m.energy, m.sigma, 0};
 }
 
 // ------------------------------------------------------------- host side

@@ -18,6 +18,7 @@
 // fixed order, for the diffusion coefficients (Swarm.cpp:1139-1176).
 #include <algorithm>
 #include <cmath>
+#include <limits>
 #include <map>
 #include <cstring>
 #include <memory>
@@ -48,7 +49,7 @@ struct RequestDesc {
     int64_t particles;
     float half_kick;
     float dt;
-    float max_energy_ev;
+    float v2_max;                 // largest squared speed whose energy is within the ceiling
     float ev_per_v2;              // 0.5 m / e
     float scale_v;                // fixed-point scales (powers of two)
     float scale_e;
@@ -57,6 +58,7 @@ struct RequestDesc {
     int burn_in;
     int sampling;                 // steps - burn_in
     int blocks;
+    uint32_t no_candidate;        // first draws below this (of 2^23) hold no candidate
     uint64_t seed;
 };
 
@@ -68,65 +70,46 @@ struct WorkItem {
 // lanes of a wave that wait with a collision candidate before the wave
 // runs the candidate code for them together
 constexpr int kCandidateBatch = 32;
+constexpr int kLdsBlocks = 32;
 
-// the rest of a swarm step after its candidate loop: the second half kick,
-// the energy checks, and (after burn-in) the counters and block sums
-template <int NCH>
-__device__ __forceinline__ void swarm_end_step(const RequestDesc& d, bool sampling,
-                                               const MccCounts<NCH>& t, float* v, uint32_t& err,
-                                               float& emax, uint32_t& cand, uint32_t& nulls,
-                                               uint32_t* chan, long long& acc_v,
-                                               long long& acc_e, int& s) {
-    err |= t.err;
-    v[0] += d.half_kick;
-    const float e = d.ev_per_v2 * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-    emax = fmaxf(emax, e);
-    if (e > d.max_energy_ev) err |= DEV_ERR_ENERGY;
-    if (sampling) {
-        cand += t.candidates;
-        nulls += t.nulls;
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) chan[c] += t.chan[c];
-        acc_v += __float2ll_rn(v[0] * d.scale_v);
-        acc_e += __float2ll_rn(e * d.scale_e);
-    }
-    ++s;
+// Draws of a step's first uniform u = (2k + 1) 2^-24 that cannot hold a
+// candidate: -log(u) / max_frequency >= dt for every k below this, with 1e-4
+// of the exponent left for the FP32 logarithm, product and timestep (off by
+// a few 1e-7 of it).
+uint32_t no_candidate_draws(float dt, float inv_max_frequency) {
+    const double x = static_cast<double>(dt) / static_cast<double>(inv_max_frequency);
+    const double k = std::floor(std::exp(-x * (1.0 + 1.0e-4)) * 0x1p23) - 2.0;
+    return k > 0.0 ? static_cast<uint32_t>(k) : 0u;
 }
 
-template <int NCH>
-__global__ void __launch_bounds__(kChunk, 4) k_swarm(MccParams m, const RequestDesc* __restrict__ descs,
-                                                  const WorkItem* __restrict__ items, int nitems,
-                                                  int* head) {
+// the largest FP32 squared speed x with fl(ev x) <= limit: the energy check
+// e > limit on an electron is x > v2_ceiling
+float v2_ceiling(float limit, float ev) {
+    float x = limit / ev;
+    while (x > 0.0f && ev * x > limit) x = std::nextafter(x, 0.0f);
+    for (;;) {
+        const float y = std::nextafter(x, std::numeric_limits<float>::infinity());
+        if (!(y < std::numeric_limits<float>::infinity()) || ev * y > limit) return x;
+        x = y;
+    }
+}
+
+// (m_arg is the first argument: first_kernel_argument<MccParams>)
+template <int NCH, bool LDS>
+__global__ void __launch_bounds__(kChunk, 4) k_swarm(MccParams m_arg,
+                                                     const RequestDesc* __restrict__ descs,
+                                                     const WorkItem* __restrict__ items, int nitems,
+                                                     int* head) {
     __shared__ MccLds lds;
     __shared__ int item_s;
-    // small reduction buffers (LDS limits how many blocks share a CU): one
-    // slot per wave for the integer sums (exact in any order), half a chunk
-    // for the cross-wave steps of the FP64 moment tree
-    __shared__ long long red_w[2][kChunk / 64];
+    // half a chunk for the cross-wave steps of the FP64 moment tree
     __shared__ double red_m[5][kChunk / 2];
-    const XsView X = stage_tables(m, lds);
-    // the chunk's integer sums of acc_v and acc_e added to q[0], q[1]
-    auto add_chunk_sums = [&](long long av, long long ae, long long* q) {
-        for (int o = 32; o > 0; o >>= 1) {
-            av += __shfl_down(av, o, 64);
-            ae += __shfl_down(ae, o, 64);
-        }
-        if ((threadIdx.x & 63) == 0) {
-            red_w[0][threadIdx.x >> 6] = av;
-            red_w[1][threadIdx.x >> 6] = ae;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            long long sv = 0, se = 0;
-            for (int wv = 0; wv < kChunk / 64; ++wv) {
-                sv += red_w[0][wv];
-                se += red_w[1][wv];
-            }
-            q[0] += sv;
-            q[1] += se;
-        }
-        __syncthreads();
-    };
+    stage_tables_as<LDS>(m_arg, lds);
+    const float safe_speed2 = m_arg.safe_speed2;
+    // sums of v_x and energy per uncertainty block of the launch (further
+    // blocks of a launch go to global memory)
+    __shared__ unsigned long long block_sum_s[2 * kLdsBlocks];
+    for (int q = threadIdx.x; q < 2 * kLdsBlocks; q += kChunk) block_sum_s[q] = 0ull;
     for (;;) {
         if (threadIdx.x == 0) item_s = atomicAdd(head, 1);
         __syncthreads();
@@ -149,90 +132,197 @@ __global__ void __launch_bounds__(kChunk, 4) k_swarm(MccParams m, const RequestD
         }
         uint32_t cand = 0, nulls = 0, chan[NCH] = {};
         uint32_t err = 0;
-        float emax = 0.f;
-        long long acc_v = 0, acc_e = 0;
-        // The launch's steps in segments that end at the burn-in end, at
-        // every uncertainty-block boundary and at the launch end (the
-        // chunk's block sums are flushed per segment).  Inside a segment
-        // every lane steps on its own: a lane whose step holds a collision
-        // candidate waits until kCandidateBatch lanes of its wave do (or no
-        // lane can step on), then the wave runs the candidate code for all
-        // of them at once -- a rare event no longer costs the whole wave
-        // every step.  Each lane's operations and draws are those of the
-        // step-synchronous loop, so results are unchanged.
+        // the largest squared speed, as bits (squares order like integers)
+        uint32_t max_v2 = 0u;
+        // a step needs a closer look where the squared speed exceeds this:
+        // the energy ceiling, the rate bound, or not a number
+        const float look_v2 = fminf(safe_speed2, d.v2_max);
+        // The launch's steps in two segments, before and after the burn-in
+        // end.  Inside a segment every lane steps on its own, and the common
+        // step -- no collision candidate -- is all a lane runs by itself: two
+        // half kicks with their energy checks, one Philox block and an
+        // integer compare of its first draw (no_candidate_draws).  A lane
+        // waits when its draw may hold a candidate, and when it reaches the
+        // end of its uncertainty block; once kCandidateBatch lanes of the
+        // wave wait (or no lane can step on) the wave takes the waiting time,
+        // the candidate and the next draw for all of the former at once, and
+        // the latter add their block sums in LDS.  Each lane's operations and
+        // draws are those of the step-synchronous loop and the sums are of
+        // integers, so results are unchanged.  VALU issue bounds the kernel:
+        // 1.2e11 electron-steps/s in runs of 8,000 steps (6.8e10 with the logarithm,
+        // square root and tallies in every step and blocks as segments).
         const int s_stop = d.step0 + d.nsteps;
         for (int s0 = d.step0; s0 < s_stop;) {
-            int seg_end, group = -1;
-            if (s0 < d.burn_in) {
-                seg_end = min(s_stop, d.burn_in);
-            } else {
-                // uncertainty block b covers samples [floor(b S / B),
-                // floor((b + 1) S / B)); blocks are at least one sample long
-                const int64_t k = s0 - d.burn_in;
-                group = static_cast<int>(((k + 1) * d.blocks - 1) / d.sampling);
-                const int64_t gend = (static_cast<int64_t>(group) + 1) * d.sampling / d.blocks;
-                seg_end = static_cast<int>(min(static_cast<int64_t>(s_stop), d.burn_in + gend));
-            }
-            const bool sampling = group >= 0;
-            int s = s0;
-            bool pending = false;
-            float elapsed = 0.f;
-            Philox rng;
+            const bool sampling = s0 >= d.burn_in;
+            const int seg_end = sampling ? s_stop : min(s_stop, d.burn_in);
+            // block sums of the lane: integers below 2^53 (the scales leave
+            // a chunk's 256 lanes 2^61), so FP64 adds them exactly
+            double acc_v = 0.0, acc_e = 0.0;
             MccCounts<NCH> t;
             mcc_tally_reset(t);
-            for (;;) {
-                if (__ballot(active && s < seg_end) == 0ull) break;
-                if (active && s < seg_end && !pending) {
-                    if (err) {
-                        // a failed particle keeps its velocity; the block
-                        // sums still take it every step
-                        if (sampling) {
-                            const float e = d.ev_per_v2 * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-                            acc_v += __float2ll_rn(v[0] * d.scale_v);
-                            acc_e += __float2ll_rn(e * d.scale_e);
-                        }
-                        ++s;
-                    } else {
+            int s = active ? s0 : seg_end;
+            // uncertainty block b covers samples [floor(b S / B),
+            // floor((b + 1) S / B)); blocks are at least one sample long
+            int group = -1, first_group = 0, block_end = seg_end;
+            auto end_of = [&](int g) {
+                const int64_t e = (static_cast<int64_t>(g) + 1) * d.sampling / d.blocks;
+                return static_cast<int>(min(static_cast<int64_t>(seg_end), d.burn_in + e));
+            };
+            if (sampling) {
+                const int64_t k = s0 - d.burn_in;
+                first_group = group = static_cast<int>(((k + 1) * d.blocks - 1) / d.sampling);
+                block_end = end_of(group);
+            }
+            int run_to = block_end;    // a lane with a candidate: 0, it does not step
+            float elapsed = 0.f;
+            int step_candidates = 0;
+            Philox rng;
+            rng.init(d.seed, 0u, static_cast<uint32_t>(p), 0u);
+            auto square = [&]() { return v[0] * v[0] + v[1] * v[1] + v[2] * v[2]; };
+            // a failed particle keeps its velocity; the block sums still
+            // take it at every step left (a product of exact integers)
+            auto book_rest = [&]() {
+                const double k = static_cast<double>(block_end - s);
+                if (sampling && s < block_end) {
+                    acc_v += k * static_cast<double>(rintf(v[0] * d.scale_v));
+                    acc_e += k * static_cast<double>(rintf(d.ev_per_v2 * square() * d.scale_e));
+                }
+                s = block_end;
+            };
+            // the step's end: second half kick, energy check, block sums
+            auto end_step = [&]<bool SAMPLING>() {
+                v[0] += d.half_kick;
+                const float v2 = square();
+                max_v2 = max(max_v2, __float_as_uint(v2));
+                if constexpr (SAMPLING) {
+                    acc_v += static_cast<double>(rintf(v[0] * d.scale_v));
+                    acc_e += static_cast<double>(rintf(d.ev_per_v2 * v2 * d.scale_e));
+                }
+                ++s;
+                if (v2 > d.v2_max) err |= DEV_ERR_ENERGY;
+                if (err) book_rest();
+            };
+            if (err && active) book_rest();
+            // every lane steps until enough wait or none can step on
+            auto step_lanes = [&]<bool SAMPLING>() {
+                for (;;) {
+                    if (s < run_to) {
                         v[0] += d.half_kick;
-                        const float e_pre = d.ev_per_v2 * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-                        emax = fmaxf(emax, e_pre);
-                        if (e_pre > d.max_energy_ev) err |= DEV_ERR_ENERGY;
-                        if (sampling) {
+                        const float v2 = square();
+                        max_v2 = max(max_v2, __float_as_uint(v2));
+                        if constexpr (SAMPLING) {
                             x[0] += v[0] * d.dt;
                             x[1] += v[1] * d.dt;
                             x[2] += v[2] * d.dt;
                         }
-                        rng.init(d.seed, 0u, static_cast<uint32_t>(p), static_cast<uint32_t>(s));
-                        mcc_tally_reset(t);
-                        elapsed = 0.f;
-                        if (!isfinite(v[0]) || !isfinite(v[1]) || !isfinite(v[2]))
-                            t.err = DEV_ERR_NONFINITE;
-                        else
-                            pending = mcc_next_candidate<NCH>(m, X, v, d.dt, rng, elapsed, t);
-                        if (!pending)
-                            swarm_end_step<NCH>(d, sampling, t, v, err, emax, cand, nulls, chan, acc_v, acc_e, s);
+                        rng.c0 = 0u;
+                        rng.c2 = static_cast<uint32_t>(s);
+                        rng.refill();
+                        bool may_collide = (rng.b0 >> 9) >= d.no_candidate;
+                        if (!(v2 <= look_v2)) {
+                            if (v2 > d.v2_max) err |= DEV_ERR_ENERGY;
+                            if (!(v2 <= safe_speed2)) {
+                                const MccParams& m = first_kernel_argument<MccParams>();
+                                const XsView X = table_view<LDS>(m, lds);
+                                uint32_t failed = 0u;
+                                if (!isfinite(v[0]) || !isfinite(v[1]) || !isfinite(v[2]))
+                                    failed = DEV_ERR_NONFINITE;
+                                else if (mcc_rate_fails<NCH>(m, X, v))
+                                    failed = DEV_ERR_RATE;
+                                err |= failed;
+                                may_collide = may_collide && failed == 0u;
+                            }
+                        }
+                        if (may_collide) {
+                            run_to = 0;
+                            elapsed = 0.f;
+                            step_candidates = 0;
+                        } else {
+                            end_step.template operator()<SAMPLING>();
+                        }
+                    }
+                    const uint64_t stepping = __ballot(s < run_to);
+                    const uint64_t waiting = __ballot(s < seg_end) & ~stepping;
+                    if (stepping == 0ull || __popcll(waiting) >= kCandidateBatch) break;
+                }
+            };
+            for (;;) {
+                if (sampling) step_lanes.template operator()<true>();
+                else step_lanes.template operator()<false>();
+                if (s < seg_end && run_to == 0) {
+                    // mcc_collide's loop from one waiting time to the next
+                    const MccParams& m = first_kernel_argument<MccParams>();
+                    const XsView X = table_view<LDS>(m, lds);
+                    bool again = false;
+                    const float waiting = -logf(rng.u01()) * m.inv_max_frequency;
+                    if (waiting < d.dt - elapsed) {
+                        elapsed += waiting;
+                        ++t.candidates;
+                        if (++step_candidates > m.max_candidates)
+                            err |= DEV_ERR_CANDIDATES;
+                        else if (mcc_candidate<NCH>(m, X, lds.chan, v, rng, t)) {
+                            if (!(square() <= safe_speed2) && mcc_rate_fails<NCH>(m, X, v))
+                                err |= DEV_ERR_RATE;
+                            else
+                                again = true;
+                        }
+                        err |= t.err;
+                        t.err = 0u;
+                    }
+                    if (!again) {
+                        run_to = block_end;
+                        if (sampling) end_step.template operator()<true>();
+                        else end_step.template operator()<false>();
                     }
                 }
-                const uint64_t waiting_lanes = __ballot(pending);
-                if (waiting_lanes == 0ull) continue;
-                const uint64_t stepping = __ballot(active && s < seg_end && !pending);
-                if (__popcll(waiting_lanes) < kCandidateBatch && stepping != 0ull) continue;
-                if (pending) {
-                    if (!(mcc_candidate<NCH>(m, X, lds.chan, v, rng, t) &&
-                          mcc_next_candidate<NCH>(m, X, v, d.dt, rng, elapsed, t))) {
-                        pending = false;
-                        swarm_end_step<NCH>(d, sampling, t, v, err, emax, cand, nulls, chan, acc_v, acc_e, s);
+                // lanes at the end of their block add its sums
+                if (sampling && active && s == block_end && group >= 0) {
+                    const int slot = 2 * (group - first_group);
+                    if (slot < 2 * kLdsBlocks) {
+                        atomicAdd(&block_sum_s[slot],
+                                  static_cast<unsigned long long>(__double2ll_rn(acc_v)));
+                        atomicAdd(&block_sum_s[slot + 1],
+                                  static_cast<unsigned long long>(__double2ll_rn(acc_e)));
+                    } else {
+                        unsigned long long* q = reinterpret_cast<unsigned long long*>(
+                            d.part + (static_cast<int64_t>(w.chunk) * d.blocks + group) * 2);
+                        atomicAdd(q, static_cast<unsigned long long>(__double2ll_rn(acc_v)));
+                        atomicAdd(q + 1, static_cast<unsigned long long>(__double2ll_rn(acc_e)));
+                    }
+                    acc_v = 0.0;
+                    acc_e = 0.0;
+                    ++group;
+                    if (s < seg_end) {
+                        block_end = end_of(group);
+                        run_to = block_end;
+                        if (err) book_rest();
+                    } else {
+                        group = -1;
                     }
                 }
+                if (__ballot(s < seg_end || (sampling && active && group >= 0)) == 0ull) break;
             }
             if (sampling) {
-                add_chunk_sums(acc_v, acc_e,
-                               d.part + (static_cast<int64_t>(w.chunk) * d.blocks + group) * 2);
-                acc_v = 0;
-                acc_e = 0;
+                cand += t.candidates;
+                nulls += t.nulls;
+#pragma unroll
+                for (int c = 0; c < NCH; ++c) chan[c] += t.chan[c];
+                // the chunk's block sums of this launch (every lane has added
+                // its own) to the request's partials
+                const int64_t k1 = s_stop - d.burn_in;
+                const int last_group = static_cast<int>((k1 * d.blocks - 1) / d.sampling);
+                const int nsum = 2 * min(last_group - first_group + 1, kLdsBlocks);
+                __syncthreads();
+                for (int q = threadIdx.x; q < nsum; q += kChunk) {
+                    d.part[(static_cast<int64_t>(w.chunk) * d.blocks + first_group) * 2 + q] +=
+                        static_cast<long long>(block_sum_s[q]);
+                    block_sum_s[q] = 0ull;
+                }
+                __syncthreads();
             }
             s0 = seg_end;
         }
+        const float emax = d.ev_per_v2 * __uint_as_float(max_v2);
         const bool last = d.step0 + d.nsteps == d.burn_in + d.sampling;
         if (last) {
             // displacement moments of the chunk, reduced in a fixed order
@@ -269,12 +359,26 @@ __global__ void __launch_bounds__(kChunk, 4) k_swarm(MccParams m, const RequestD
             d.vx[p] = v[0];
             d.vy[p] = v[1];
             d.vz[p] = v[2];
-            if (cand) atomicAdd(d.counts, static_cast<unsigned long long>(cand));
-            if (nulls) atomicAdd(d.counts + 1, static_cast<unsigned long long>(nulls));
+        }
+        // one atomic per wave and counter (per lane they queue up on the
+        // request's few addresses: 20 ms of a 66 ms launch of 1,000 steps)
+        uint64_t sums[2 + NCH];
+        sums[0] = cand;
+        sums[1] = nulls;
 #pragma unroll
-            for (int c = 0; c < NCH; ++c)
-                if (chan[c]) atomicAdd(d.counts + 2 + c, static_cast<unsigned long long>(chan[c]));
-            atomicMax(d.max_energy_bits, __float_as_uint(emax));
+        for (int c = 0; c < NCH; ++c) sums[2 + c] = chan[c];
+        float top = active ? emax : 0.f;
+        for (int o = 32; o > 0; o >>= 1) {
+            top = fmaxf(top, __shfl_xor(top, o, 64));
+            err |= __shfl_xor(err, o, 64);
+        }
+#pragma unroll
+        for (int k = 0; k < 2 + NCH; ++k) {
+            const unsigned long long n = wave_sum_u64(sums[k]);
+            if ((threadIdx.x & 63) == 0 && n) atomicAdd(d.counts + k, n);
+        }
+        if ((threadIdx.x & 63) == 0) {
+            atomicMax(d.max_energy_bits, __float_as_uint(top));
             if (err) atomicOr(d.status, err);
         }
     }
@@ -968,6 +1072,7 @@ void block_slope_error(const double* y, int64_t n, double dt, int64_t blocks, do
 void queue_launch(Context& c, SwarmState& s, int64_t max_steps) {
     LaunchBuffers& b = s.buf[s.cur];
     if (b.done) AUR_HIP(hipEventSynchronize(b.done));   // the buffers' previous launch
+    const MccParams m = swarm_params(s);
     std::vector<RequestDesc> descs;
     std::vector<WorkItem> items;
     s.finishing.clear();
@@ -993,8 +1098,8 @@ void queue_launch(Context& c, SwarmState& s, int64_t max_steps) {
         const double accel = -kElementaryCharge * efield / kElectronMass;
         d.half_kick = static_cast<float>(0.5 * accel * q.timestep);
         d.dt = static_cast<float>(q.timestep);
-        d.max_energy_ev = static_cast<float>(q.max_energy_ev);
         d.ev_per_v2 = static_cast<float>(0.5 * kElectronMass / kElementaryCharge);
+        d.v2_max = v2_ceiling(static_cast<float>(q.max_energy_ev), d.ev_per_v2);
         d.scale_v = static_cast<float>(scales(q).first);
         d.scale_e = static_cast<float>(scales(q).second);
         d.step0 = static_cast<int>(r.steps_done);
@@ -1002,6 +1107,7 @@ void queue_launch(Context& c, SwarmState& s, int64_t max_steps) {
         d.burn_in = static_cast<int>(q.burn_in);
         d.sampling = static_cast<int>(q.steps - q.burn_in);
         d.blocks = static_cast<int>(q.blocks);
+        d.no_candidate = no_candidate_draws(d.dt, m.inv_max_frequency);
         d.seed = q.seed;
         const int ridx = static_cast<int>(descs.size());
         descs.push_back(d);
@@ -1035,13 +1141,12 @@ void queue_launch(Context& c, SwarmState& s, int64_t max_steps) {
     AUR_HIP(hipMemcpyAsync(b.items.ptr, b.h_items, items.size() * sizeof(WorkItem),
                            hipMemcpyHostToDevice, c.stream));
     AUR_HIP(hipMemsetAsync(b.head.ptr, 0, sizeof(int), c.stream));
-    const MccParams m = swarm_params(s);
     if (s.blocks_per_cu == 0) {
         // as many workgroups as the CUs hold at once: the kernel pulls
         // chunks from the queue, so more would only wait
         int per_cu = 0;
-        with_nchan(m.nchan, [&]<int NCH>() {
-            AUR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_swarm<NCH>, kChunk, 0));
+        with_model(m.nchan, mcc_tables_fit(m), [&]<int NCH, bool LDS>() {
+            AUR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_swarm<NCH, LDS>, kChunk, 0));
         });
         s.blocks_per_cu = per_cu > 0 ? per_cu : 4;
     }
@@ -1049,8 +1154,8 @@ void queue_launch(Context& c, SwarmState& s, int64_t max_steps) {
     if (grid > static_cast<int64_t>(items.size())) grid = static_cast<int64_t>(items.size());
     {
         KernelScope ks(c, "swarm");
-        with_nchan(m.nchan, [&]<int NCH>() {
-            k_swarm<NCH><<<static_cast<unsigned>(grid), kChunk, 0, c.stream>>>(
+        with_model(m.nchan, mcc_tables_fit(m), [&]<int NCH, bool LDS>() {
+            k_swarm<NCH, LDS><<<static_cast<unsigned>(grid), kChunk, 0, c.stream>>>(
                 m, b.descs.ptr, b.items.ptr, static_cast<int>(items.size()), b.head.ptr);
         });
         AUR_HIP(hipGetLastError());
