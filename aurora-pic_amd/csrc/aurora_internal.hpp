@@ -237,9 +237,8 @@ struct MccModelHost {
     DevBuf<unsigned long long> counts;  // [candidates, nulls, chan...]
     DevBuf<double> energy_change;       // per channel, cumulative
     DevBuf<double> energy_rows;         // per workgroup of the last 1D MCC launch
-    DevBuf<int32_t> product_count;      // per target particle
-    DevBuf<int32_t> product_loff;       // per target particle: products before it in its chunk
-    DevBuf<int32_t> chunk_tot, chunk_off;   // per 256-slot chunk: products, exclusive offset
+    DevBuf<int32_t> product_list;       // the parents of each run, at the run's first slot
+    DevBuf<int32_t> run_tot, run_off, run_parents;   // per run: products, exclusive offset, parents
     DevBuf<float> product_vel;          // secondaries: up to 2 per particle x 6 floats
 };
 

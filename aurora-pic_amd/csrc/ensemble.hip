@@ -39,7 +39,6 @@ namespace {
 constexpr int kEnsMaxSpecies = 4;
 constexpr int kEnsThreads = 256;
 constexpr int kEnsPushChunk = 2048;   // particles per push workgroup
-constexpr int kEnsMccChunk = 256;     // target particles per MCC workgroup
 constexpr int kEnsLdsNodes = 4096;    // nodes accumulated in LDS (32 KiB of int64)
 constexpr int kEnsRing = 4096;        // electrode potentials per host segment
 constexpr int kBaseFields = 6;        // per instance: sec slot, ion slot, sec uid, ion uid, ok, parents
@@ -84,13 +83,13 @@ struct EnsArgs {
     // MCC
     int target, sec, ion;
     const uint64_t* seeds;          // [M]
-    int32_t* nprod;                 // [M * cap_target]
-    int32_t* loff;                  // in-chunk exclusive offsets
     float* prod;                    // 12 floats per target slot
-    int32_t* chunk_tot;             // [M][mchunks]
-    int32_t* chunk_off;
-    int mchunks;
-    int mgroups;                    // MCC workgroups per instance (each walks chunks mgroups apart)
+    int32_t* list;                  // [M * cap_target]: the parents of each run
+    int32_t* run_tot;               // [M][mruns]: products, offset and parents of each run
+    int32_t* run_off;
+    int32_t* run_parents;
+    int mruns;
+    int mgroups;                    // MCC workgroups per instance
     double* energy_rows;            // [M][mgroups][kTallyStride]: per-workgroup tallies
     int64_t* base;                  // [M][kBaseFields]
     unsigned long long* counts;     // [M][kMaxChannels + 3]
@@ -227,56 +226,43 @@ __global__ void __launch_bounds__(kEnsThreads) k_ens_field(EnsArgs a, int solve_
                            a.eps, pv[0], pv[1]);
 }
 
-// MCC on the target species.  mgroups workgroups per instance walk its
-// 256-slot chunks mgroups apart, so the cross-section tables are staged in
-// LDS once per workgroup; product pairs are staged per parent with in-chunk
-// offsets, and the energy change goes to one row per workgroup (its waves
-// in wave order; the rows summed in a fixed order by k_ens_products).
-template <int NCH>
-__global__ void __launch_bounds__(kEnsThreads, mcc_min_waves(NCH))
-    k_ens_mcc(EnsArgs a, MccParams m) {
+// MCC on the target species (collide_run): mgroups workgroups per instance,
+// whose waves each take runs of its slots; the energy change goes to one row
+// per workgroup (the rows summed in a fixed order by k_ens_products).
+template <int NCH, bool LDS>
+__global__ void __launch_bounds__(kMccBlock, kMccWaves) k_ens_mcc(MccParams, EnsArgs a) {
     __shared__ MccLds lds;
-    __shared__ int scan_sh[kEnsThreads];
-    const XsView X = stage_tables(m, lds);
+    __shared__ WaveQueue queue[kMccBlock / 64];
+    stage_model<LDS>(lds);
     const int inst = blockIdx.x / a.mgroups;
     const int group = blockIdx.x - inst * a.mgroups;
     const EnsSpecies& sp = a.sp[a.target];
     const int64_t n = a.slots[a.target * a.M + inst];
-    const float* E32 = a.E32 + static_cast<int64_t>(inst) * a.nx;
-    WaveTally<NCH> w{};
-    for (int chunk = group; chunk < a.mchunks; chunk += a.mgroups) {
-        const int64_t lo = static_cast<int64_t>(chunk) * kEnsMccChunk;
-        const int64_t ci = static_cast<int64_t>(inst) * a.mchunks + chunk;
-        if (lo >= n) {
-            if (threadIdx.x == 0) a.chunk_tot[ci] = 0;
-            continue;
-        }
-        const int64_t q = lo + threadIdx.x;
+    const uint64_t seed = a.seeds[inst];
+    const uint32_t step = static_cast<uint32_t>(*a.step);
+    LaneTally<NCH> t{};
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t waves = a.mgroups * (kMccBlock / 64);
+    const RunPlan plan(n, waves);
+    for (uint32_t r = group * (kMccBlock / 64) + wid; r < plan.runs; r += waves) {
+        const int64_t q = static_cast<int64_t>(r) * plan.chunks * 64;
+        const int64_t left = n - q;
+        const int slots = static_cast<int>(left < 64 * plan.chunks ? left : 64 * plan.chunks);
         const int64_t p = static_cast<int64_t>(inst) * sp.cap + q;
-        const bool in = q < n;
-        const int c = in ? sp.cell[p] : -1;
-        const bool active = c >= 0;
-        MccTally<NCH> t{};
-        int np = 0;
-        if (active)
-            np = mcc_1d_particle<NCH>(m, X, lds.chan, c, sp.off[p], sp.v0 + p, sp.v1 + p,
-                                      sp.v2 + p, sp.uid[p], E32, a.nx, sp.half_qm_dt, a.dt,
-                                      a.seeds[inst], static_cast<uint32_t>(*a.step),
-                                      a.prod + 12 * p, t, a.err + inst);
-        flush_tally_rows<NCH>(t, active, w);
-        int total = 0;
-        const int ex = block_scan_int<kEnsThreads>(np, scan_sh, total);
-        if (in) {
-            a.nprod[p] = np;
-            a.loff[p] = ex;
-        }
-        if (threadIdx.x == 0) a.chunk_tot[ci] = total;
+        const Run1d io{sp.cell + p, sp.off + p, sp.v0 + p, sp.v1 + p, sp.v2 + p, sp.uid + p,
+                       a.sec >= 0 ? a.prod + 12 * p : nullptr,
+                       a.E32 + static_cast<int64_t>(inst) * a.nx, a.nx, sp.half_qm_dt};
+        const bool made = collide_run<NCH, LDS, false>(lds, queue[wid], io, slots, a.dt, seed, 0u,
+                                                       step, t);
+        const int64_t k = static_cast<int64_t>(inst) * a.mruns + r;
+        if (a.sec >= 0)
+            list_parents(queue[wid], slots, made, a.list + p, a.run_parents + k, a.run_tot + k);
     }
-    store_block_row<NCH, kEnsThreads>(w, a.energy_rows,
-                                      static_cast<int64_t>(inst) * a.mgroups + group);
+    store_block_row<NCH, kMccBlock>(t, a.energy_rows,
+                                    static_cast<int64_t>(inst) * a.mgroups + group);
 }
 
-// Per instance: chunk offsets, all-or-nothing capacity check
+// Per instance: run offsets, all-or-nothing capacity check
 // (Simulation.cpp:929-964), slot and uid reservation.
 template <int NCH>
 __global__ void __launch_bounds__(kEnsThreads) k_ens_products(EnsArgs a) {
@@ -285,15 +271,17 @@ __global__ void __launch_bounds__(kEnsThreads) k_ens_products(EnsArgs a) {
     {
         // this step's MCC tallies: the instance's workgroup rows, in order
         const int64_t nrows = a.mgroups;
-        fold_tally_rows<NCH, kEnsThreads>(
+        const uint32_t err = fold_tally_rows<NCH, kEnsThreads>(
             a.energy_rows + static_cast<int64_t>(inst) * nrows * kTallyStride, nrows,
             a.ech + static_cast<int64_t>(inst) * kMaxChannels,
             a.counts + static_cast<int64_t>(inst) * (kMaxChannels + 3));
+        if (threadIdx.x == 0 && err) atomicOr(a.err + inst, err);
     }
     if (a.sec < 0) return;
-    const int32_t* tot = a.chunk_tot + static_cast<int64_t>(inst) * a.mchunks;
-    int32_t* off = a.chunk_off + static_cast<int64_t>(inst) * a.mchunks;
-    const int total = chunk_offsets<kEnsThreads>(tot, off, a.mchunks, scan_sh);
+    const RunPlan plan(a.slots[a.target * a.M + inst], a.mgroups * (kMccBlock / 64));
+    const int32_t* tot = a.run_tot + static_cast<int64_t>(inst) * a.mruns;
+    int32_t* off = a.run_off + static_cast<int64_t>(inst) * a.mruns;
+    const int total = chunk_offsets<kEnsThreads>(tot, off, plan.runs, scan_sh);
     if (threadIdx.x != 0) return;
     int64_t* b = a.base + static_cast<int64_t>(inst) * kBaseFields;
     const int M = a.M;
@@ -345,21 +333,23 @@ __device__ __forceinline__ AppendSide ens_side(const EnsSpecies& sp, int inst, i
 // (and advances the step counter: nothing after it in the step reads it)
 __global__ void __launch_bounds__(kEnsThreads) k_ens_append(EnsArgs a) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *a.step += 1;
-    const int inst = blockIdx.x / a.mchunks;
-    const int chunk = blockIdx.x - inst * a.mchunks;
+    const int inst = blockIdx.x / a.mgroups;
+    const int group = blockIdx.x - inst * a.mgroups;
     const int64_t* b = a.base + static_cast<int64_t>(inst) * kBaseFields;
     if (b[4] == 0) return;
-    const int64_t q = static_cast<int64_t>(chunk) * kEnsMccChunk + threadIdx.x;
-    if (q >= b[5]) return;
     const EnsSpecies& sp = a.sp[a.target];
-    const int64_t p = static_cast<int64_t>(inst) * sp.cap + q;
-    const int np = a.nprod[p];
-    if (np == 0) return;
     const AppendSide sec = ens_side(a.sp[a.sec], inst, b[0], b[2]);
     const AppendSide ion = ens_side(a.sp[a.ion], inst, b[1], b[3]);
-    const int64_t j0 = a.chunk_off[blockIdx.x] + a.loff[p];
-    append_products_of(sp.cell[p], sp.off[p], np, j0, a.prod + 12 * p,
-                       a.E32 + static_cast<int64_t>(inst) * a.nx, a.nx, sec, ion);
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t waves = a.mgroups * (kMccBlock / 64);
+    const RunPlan plan(b[5], waves);
+    for (uint32_t r = group * (kMccBlock / 64) + wid; r < plan.runs; r += waves) {
+        const int64_t p = static_cast<int64_t>(inst) * sp.cap +
+                          static_cast<int64_t>(r) * plan.chunks * 64;
+        const int64_t k = static_cast<int64_t>(inst) * a.mruns + r;
+        append_run(a.list + p, a.run_parents[k], a.run_off[k], sp.cell + p, sp.off + p,
+                   a.prod + 12 * p, a.E32 + static_cast<int64_t>(inst) * a.nx, a.nx, sec, ion);
+    }
 }
 
 __global__ void k_ens_tick(int64_t* step) {
@@ -487,10 +477,9 @@ struct Ensemble {
     DevBuf<double> wall_rows;
     DevBuf<uint32_t> err;
     DevBuf<uint64_t> seeds;
-    DevBuf<int32_t> nprod, loff;
     DevBuf<float> prod;
-    DevBuf<int32_t> chunk_tot, chunk_off;
-    int mgroups = 0;
+    DevBuf<int32_t> list, run_tot, run_off, run_parents;
+    int mgroups = 0, mruns = 0;
     DevBuf<double> energy_rows;
     DevBuf<int64_t> base;
     DevBuf<unsigned long long> counts;
@@ -596,14 +585,12 @@ EnsArgs make_args(Context& c, Ensemble& e, double dt) {
     a.sec = c.mcc.secondary_species;
     a.ion = c.mcc.ion_species;
     a.seeds = e.seeds.ptr;
-    a.nprod = e.nprod.ptr;
-    a.loff = e.loff.ptr;
     a.prod = e.prod.ptr;
-    a.chunk_tot = e.chunk_tot.ptr;
-    a.chunk_off = e.chunk_off.ptr;
-    a.mchunks = a.target >= 0
-                    ? static_cast<int>((e.sp[a.target].cap + kEnsMccChunk - 1) / kEnsMccChunk)
-                    : 0;
+    a.list = e.list.ptr;
+    a.run_tot = e.run_tot.ptr;
+    a.run_off = e.run_off.ptr;
+    a.run_parents = e.run_parents.ptr;
+    a.mruns = e.mruns;
     a.mgroups = e.mgroups;
     a.energy_rows = e.energy_rows.ptr;
     a.base = e.base.ptr;
@@ -645,19 +632,29 @@ CompactArgs compact_args(Ensemble& e, int s) {
     return k;
 }
 
+MccParams ens_mcc_params(const Context& c, const EnsArgs& a) {
+    MccParams m{};
+    if (!c.mcc.loaded) return m;
+    m = mcc_step_params(c);
+    m.no_candidate = no_candidate_draws(a.dt, m.inv_max_frequency);
+    return m;
+}
+
 // Queue one step (or the compaction) of every instance on the stream.
 void enqueue_step(Context& c, Ensemble& e, const EnsArgs& a, const MccParams& m) {
     const size_t shmem = a.periodic ? spectral_1d_lds(a.nx) : 0;
     k_ens_push<true><<<push_grid(a), kEnsThreads, 0, c.stream>>>(a);
     k_ens_field<<<a.M, kEnsThreads, shmem, c.stream>>>(a, 1);
     if (a.target >= 0) {
-        const int g = a.M * a.mchunks;
+        const int g = a.M * a.mgroups;
+        with_model(m.nchan, mcc_tables_fit(m), [&]<int NCH, bool LDS>() {
+            k_ens_mcc<NCH, LDS><<<g, kMccBlock, 0, c.stream>>>(m, a);
+        });
         with_nchan(m.nchan, [&]<int NCH>() {
-            k_ens_mcc<NCH><<<a.M * a.mgroups, kEnsThreads, 0, c.stream>>>(a, m);
             k_ens_products<NCH><<<a.M, kEnsThreads, 0, c.stream>>>(a);
         });
         if (a.sec >= 0) {
-            k_ens_append<<<g, kEnsThreads, 0, c.stream>>>(a);
+            k_ens_append<<<g, kMccBlock, 0, c.stream>>>(a);
             return;
         }
     }
@@ -700,7 +697,7 @@ void capture_graph(Context& c, Ensemble& e, double dt, int steps) {
         e.graph = nullptr;
     }
     const EnsArgs a = make_args(c, e, dt);
-    const MccParams m = c.mcc.loaded ? mcc_step_params(c) : MccParams{};
+    const MccParams m = ens_mcc_params(c, a);
     AUR_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
     for (int k = 0; k < steps; ++k) enqueue_step(c, e, a, m);
     enqueue_compaction(c, e);
@@ -825,24 +822,17 @@ int aurora_hip_ensemble_create(aurora_hip_ctx* h, int64_t instances, const int64
         if (c.mcc.loaded) {
             const int t = c.mcc.target;
             const int64_t n = M * capacity[t];
-            const int64_t mch = (capacity[t] + kEnsMccChunk - 1) / kEnsMccChunk;
-            e->nprod.alloc(static_cast<size_t>(n));
-            e->loff.alloc(static_cast<size_t>(n));
+            // the waves of one resident round shared by the instances
+            const int all = mcc_groups(c.cu_count, n);
+            e->mgroups = static_cast<int>(std::clamp<int64_t>(
+                (all + M - 1) / M, 1, (capacity[t] + kMccBlock - 1) / kMccBlock));
+            e->mruns = static_cast<int>(
+                max_runs(capacity[t], static_cast<int64_t>(e->mgroups) * (kMccBlock / 64)));
             e->prod.alloc(static_cast<size_t>(12 * n));
-            e->chunk_tot.alloc(static_cast<size_t>(M * mch));
-            e->chunk_off.alloc(static_cast<size_t>(M * mch));
-            // one round of resident MCC workgroups over all instances (a
-            // partial further round would leave most of the chip idle)
-            int per_cu = 1;
-            with_nchan(c.mcc.nchan, [&]<int NCH>() {
-                int v = 0;
-                if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, k_ens_mcc<NCH>, kEnsThreads,
-                                                                 0) == hipSuccess &&
-                    v > 0)
-                    per_cu = v;
-            });
-            const int64_t want = static_cast<int64_t>(c.cu_count) * per_cu;
-            e->mgroups = static_cast<int>(std::clamp<int64_t>((want + M - 1) / M, 1, mch));
+            e->list.alloc(static_cast<size_t>(n));
+            e->run_tot.alloc(static_cast<size_t>(M * e->mruns));
+            e->run_off.alloc(static_cast<size_t>(M * e->mruns));
+            e->run_parents.alloc(static_cast<size_t>(M * e->mruns));
             e->energy_rows.alloc(static_cast<size_t>(M * e->mgroups * kTallyStride));
             e->base.alloc(static_cast<size_t>(M * kBaseFields));
             AUR_HIP(hipMemsetAsync(e->base.ptr, 0, M * kBaseFields * 8, c.stream));
@@ -957,7 +947,7 @@ int aurora_hip_ensemble_step(aurora_hip_ctx* h, int64_t handle, double dt, int64
         const int G = e.requested_graph_steps;
         if (G > 0 && (e.graph_steps != G || e.dt_graph != dt)) capture_graph(c, e, dt, G);
         const EnsArgs a = make_args(c, e, dt);
-        const MccParams m = c.mcc.loaded ? mcc_step_params(c) : MccParams{};
+        const MccParams m = ens_mcc_params(c, a);
         int64_t left = nsteps;
         while (left > 0) {
             const int64_t k = (G > 0 && left >= G) ? G : std::min<int64_t>(left, kEnsRing - 2);

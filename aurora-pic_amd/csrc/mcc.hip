@@ -28,37 +28,58 @@ namespace aurora {
 namespace {
 
 constexpr int kBlk = 256;
+constexpr int kFold = 1024;   // the one-workgroup folds
 
 
-// standalone collide of count velocities (parity checks): uid = index
-template <int NCH>
-__global__ void __launch_bounds__(kBlk, mcc_min_waves(NCH))
-    k_collide(MccParams m, float* v, int64_t count, float dt, uint64_t seed, uint32_t stream,
-              uint32_t step, double* rows, uint32_t* err, int one_v) {
-    __shared__ MccLds lds;
-    const XsView X = stage_tables(m, lds);
-    WaveTally<NCH> w{};
-    for (int64_t base = static_cast<int64_t>(blockIdx.x) * blockDim.x; base < count;
-         base += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        const int64_t p = base + threadIdx.x;
-        const bool active = p < count;
-        MccTally<NCH> t{};
-        if (active) {
-            float u[3] = {v[3 * p], v[3 * p + 1], v[3 * p + 2]};
-            Philox rng;
-            rng.init(seed, stream, static_cast<uint32_t>(p), step);
-            if (one_v)
-                mcc_collide_1v<NCH>(m, X, lds.chan, u[0], dt, rng, t);
-            else
-                mcc_collide<NCH>(m, X, lds.chan, u, dt, rng, t);
-            if (t.err) atomicOr(err, t.err);
-            v[3 * p] = u[0];
-            v[3 * p + 1] = u[1];
-            v[3 * p + 2] = u[2];
-        }
-        flush_tally_rows<NCH>(t, active, w);
+// standalone collide of velocities (parity checks): uid = index
+struct RunPlain {
+    float* v;            // the run's first
+    uint32_t first;
+    static constexpr bool kProducts = false;
+    struct State {
+        float v[3];
+    };
+    __device__ __forceinline__ bool fetch(int i, State& s) const {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) s.v[a] = v[3 * i + a];
+        return true;
     }
-    store_wave_row<NCH>(w, rows);
+    __device__ __forceinline__ void velocity(const State& s, float* u) const {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) u[a] = s.v[a];
+    }
+    __device__ __forceinline__ uint32_t id(const State&, int i) const {
+        return first + static_cast<uint32_t>(i);
+    }
+    __device__ __forceinline__ float* products(int) const { return nullptr; }
+    __device__ __forceinline__ void pass(int, const State&, const float*) const {}
+    __device__ __forceinline__ void store(int i, const State&, const float* u) const {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) v[3 * i + a] = u[a];
+    }
+};
+
+template <int NCH, bool LDS, bool ONE_V>
+__global__ void __launch_bounds__(kMccBlock, kMccWaves)
+    k_collide(MccParams, float* v, int64_t count, float dt, uint64_t seed, uint32_t stream,
+              uint32_t step, double* rows) {
+    __shared__ MccLds lds;
+    __shared__ WaveQueue queue[kMccBlock / 64];
+    stage_model<LDS>(lds);
+    LaneTally<NCH> t{};
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t waves = gridDim.x * (kMccBlock / 64);
+    const RunPlan plan(count, waves);
+    for (uint32_t r = blockIdx.x * (kMccBlock / 64) + wid; r < plan.runs; r += waves) {
+        const int64_t first = static_cast<int64_t>(r) * plan.chunks * 64;
+        const int64_t left = count - first;
+        const RunPlain io{v + 3 * first, static_cast<uint32_t>(first)};
+        collide_run<NCH, LDS, ONE_V>(
+            lds, queue[wid], io,
+            static_cast<int>(left < 64 * plan.chunks ? left : 64 * plan.chunks), dt, seed, stream,
+            step, t);
+    }
+    store_block_row<NCH, kMccBlock>(t, rows, blockIdx.x);
 }
 
 struct Mcc1dArgs {
@@ -77,49 +98,41 @@ struct Mcc1dArgs {
     uint32_t stream;        // the model's index: its own random stream
     int one_v;              // 1D1V: the scalar collide on v_x
     uint32_t step;
-    int32_t* nprod;         // per particle ionization events (0..2)
-    float* prod;            // per particle: 2 x (secondary v[3], ion v[3])
-    uint32_t* err;
-    int32_t* loff;          // per particle: products before it in its 256-slot chunk
-    int32_t* chunk_tot;     // per chunk: its products (null: the model has none)
+    float* prod;            // per particle: 2 x (secondary v[3], ion v[3]); null: no products
+    int32_t* list;          // the parents of each run, at its first slot (list_parents)
+    int32_t* run_tot;       // per run: its products
+    int32_t* run_parents;
     const long long* nslots;   // the slot count on the device (slots is then the capacity), or null
 };
 
-// sync -> collide -> rebuild v_half for every live target particle
-// (with products: each 256-slot chunk's event counts scanned in the block,
-// so a parent's product index is its chunk's offset plus its own prefix)
+// sync -> collide -> rebuild v_half for every live target particle, run by
+// run (collide_run), and the list of each run's parents.
 // ONE_V: the 1D1V scalar collide (a.one_v), a separate build so that the
 // 3V kernel carries no registers of the other path
-template <int NCH, bool ONE_V>
-__global__ void __launch_bounds__(kBlk, mcc_min_waves(NCH))
-    k_mcc_1d(MccParams m, Mcc1dArgs a, double* rows) {
+template <int NCH, bool LDS, bool ONE_V>
+__global__ void __launch_bounds__(kMccBlock, kMccWaves)
+    k_mcc_1d(MccParams, Mcc1dArgs a, double* rows) {
     __shared__ MccLds lds;
-    __shared__ int wsum[kBlk / 64];
-    const XsView X = stage_tables(m, lds);
-    WaveTally<NCH> w{};
+    __shared__ WaveQueue queue[kMccBlock / 64];
+    stage_model<LDS>(lds);
+    LaneTally<NCH> t{};
     const int64_t nslot = a.nslots ? static_cast<int64_t>(*a.nslots) : a.slots;
-    for (int64_t base = static_cast<int64_t>(blockIdx.x) * kBlk; base < nslot;
-         base += static_cast<int64_t>(gridDim.x) * kBlk) {
-        const int64_t p = base + threadIdx.x;
-        const bool in = p < nslot;
-        const int c = in ? a.cell[p] : -1;
-        const bool active = c >= 0;
-        MccTally<NCH> t{};
-        int np = 0;
-        if (active)
-            np = mcc_1d_particle<NCH>(m, X, lds.chan, c, a.off[p], a.v0 + p, a.v1 + p, a.v2 + p,
-                                      a.uid[p], a.E32, a.nx, a.half_qm_dt, a.dt, a.seed, a.step,
-                                      a.prod + 12 * p, t, a.err, a.stream, ONE_V);
-        if (in) a.nprod[p] = np;
-        flush_tally_rows<NCH>(t, active, w);
-        if (a.chunk_tot) {
-            int total = 0;
-            const int ex = block_scan_int<kBlk>(np, wsum, total);
-            if (in) a.loff[p] = ex;
-            if (threadIdx.x == 0) a.chunk_tot[base / kBlk] = total;
-        }
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t waves = gridDim.x * (kMccBlock / 64);
+    const RunPlan plan(nslot, waves);
+    for (uint32_t r = blockIdx.x * (kMccBlock / 64) + wid; r < plan.runs; r += waves) {
+        const int64_t p = static_cast<int64_t>(r) * plan.chunks * 64;
+        const int64_t left = nslot - p;
+        const int slots = static_cast<int>(left < 64 * plan.chunks ? left : 64 * plan.chunks);
+        const Run1d io{a.cell + p, a.off + p, a.v0 + p,  a.v1 + p, a.v2 + p,
+                       a.uid + p,  a.prod ? a.prod + 12 * p : nullptr, a.E32, a.nx,
+                       a.half_qm_dt};
+        const bool made = collide_run<NCH, LDS, ONE_V>(lds, queue[wid], io, slots, a.dt, a.seed,
+                                                       a.stream, a.step, t);
+        if (a.prod)
+            list_parents(queue[wid], slots, made, a.list + p, a.run_parents + r, a.run_tot + r);
     }
-    store_block_row<NCH, kBlk>(w, rows, blockIdx.x);
+    store_block_row<NCH, kMccBlock>(t, rows, blockIdx.x);
 }
 
 // All models' products reserved together on the device (the counts kept
@@ -178,40 +191,50 @@ __device__ void commit_products(const CommitArgs& a, long long* need) {
     }
 }
 
-// After one model's k_mcc_1d: its tally rows added in row order (as
-// k_fold_rows), then, with products, the chunk totals scanned into chunk
-// offsets and the model's product count written to *total; with commit
-// (the last model while the counts are on the device), every model's
-// products reserved.
+// After one model's k_mcc_1d: its tally rows (one per workgroup) added in row
+// order, then, with products, the run totals scanned into run offsets and the
+// model's product count written to *total; with commit (the last model while
+// the counts are on the device), every model's products reserved.
 template <int NCH>
-__global__ void __launch_bounds__(kBlk) k_mcc_finish(const double* rows, int64_t nrows,
+__global__ void __launch_bounds__(kFold) k_mcc_finish(const double* rows, int groups,
                                                      double* energy, unsigned long long* counts,
-                                                     const int32_t* chunk_tot, int32_t* chunk_off,
-                                                     int64_t nchunks, const long long* nslots,
-                                                     long long* total, CommitArgs commit) {
-    fold_tally_rows<NCH, kBlk>(rows, nrows, energy, counts);
-    __shared__ int wsum[kBlk / 64];
+                                                     const int32_t* run_tot, int32_t* run_off,
+                                                     int64_t slots, const long long* nslots,
+                                                     long long* total, uint32_t* err,
+                                                     CommitArgs commit) {
+    // (the runs the collide wrote: its slot count on the device, if there)
+    const RunPlan plan(nslots ? static_cast<int64_t>(*nslots) : slots, groups * (kMccBlock / 64));
+    const uint32_t bits = fold_tally_rows<NCH, kFold>(rows, groups, energy, counts);
+    __shared__ int wsum[kFold / 64];
     __shared__ long long need[kMaxChannels];
     int all = 0;
-    if (chunk_tot) {
-        // the chunks the collide wrote (its slot count on the device, if there)
-        if (nslots) nchunks = (static_cast<int64_t>(*nslots) + kBlk - 1) / kBlk;
-        all = chunk_offsets<kBlk>(chunk_tot, chunk_off, nchunks, wsum);
-    }
+    if (run_tot) all = chunk_offsets<kFold>(run_tot, run_off, plan.runs, wsum);
     if (threadIdx.x == 0) {
+        if (bits) atomicOr(err, bits);
         *total = all;
         if (commit.models > 0) commit_products(commit, need);
     }
 }
 
-// Adds the tally rows of one launch, in row order, to the energy change
-// [NCH] and the counters [NCH + 3].
+// Ends a bare collide: the energy change [NCH], the counters [NCH + 3] and
+// the error bits of its tally rows; as_status: the bits as an aurora_status
+// (no rows: zeros).
 template <int NCH>
-__global__ void __launch_bounds__(kBlk) k_fold_rows(const double* rows, int64_t nrows,
-                                                    double* energy, unsigned long long* counts) {
-    fold_tally_rows<NCH, kBlk>(rows, nrows, energy, counts);
+__global__ void __launch_bounds__(kFold) k_collide_finish(const double* rows, int groups,
+                                                         double* energy,
+                                                         unsigned long long* counts,
+                                                         uint32_t* err, int as_status) {
+    const uint32_t b = fold_tally_rows<NCH, kFold, false>(rows, groups, energy, counts);
+    if (threadIdx.x != 0) return;
+    if (!as_status) {
+        if (b) atomicOr(err, b);
+        return;
+    }
+    *err = b == 0                     ? AURORA_OK
+           : (b & DEV_ERR_RATE)       ? AURORA_ERR_RATE_ABOVE_BOUND
+           : (b & DEV_ERR_CANDIDATES) ? AURORA_ERR_CANDIDATE_LIMIT
+                                      : AURORA_ERR_INVALID_ARGUMENT;
 }
-
 
 __global__ void k_zero_total(long long* total) { *total = 0; }
 
@@ -221,12 +244,12 @@ __global__ void k_mcc_commit(CommitArgs a) {
     if (blockIdx.x == 0 && threadIdx.x == 0) commit_products(a, need);
 }
 
-// write the products of parent p at product index chunk_off[p / kBlk] +
-// loff[p] + k (grid-stride over 256-slot chunks); with place (device
-// counts), the parents and the bases come from commit_products' placement
+// the products of every listed parent, a wave per run (the runs of the
+// collide: groups workgroups of it); with place (device counts), the parents
+// and the bases come from commit_products' placement
 __global__ void __launch_bounds__(kBlk) k_append_products(
-    const int32_t* pcell, const float* poff, const int32_t* nprod, const int32_t* loff,
-    const int32_t* chunk_off, const float* prod, int64_t parents, const float* E32, int nx,
+    const int32_t* pcell, const float* poff, const int32_t* list, const int32_t* run_parents,
+    const int32_t* run_off, const float* prod, int64_t slots, int groups, const float* E32, int nx,
     AppendSide sec, AppendSide ion, const long long* place) {
     if (place) {
         if (place[5] == 0) return;
@@ -234,63 +257,40 @@ __global__ void __launch_bounds__(kBlk) k_append_products(
         ion.base_slot = place[1];
         sec.base_uid = static_cast<uint32_t>(place[2]);
         ion.base_uid = static_cast<uint32_t>(place[3]);
-        parents = place[4];
+        slots = place[4];
     }
-    for (int64_t base = static_cast<int64_t>(blockIdx.x) * kBlk; base < parents;
-         base += static_cast<int64_t>(gridDim.x) * kBlk) {
-        const int64_t p = base + threadIdx.x;
-        if (p >= parents) continue;
-        const int np = nprod[p];
-        if (np == 0) continue;
-        append_products_of(pcell[p], poff[p], np, static_cast<int64_t>(chunk_off[base / kBlk]) +
-                                                      loff[p],
-                           prod + 12 * p, E32, nx, sec, ion);
+    const RunPlan plan(slots, groups * (kMccBlock / 64));
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (uint32_t r = blockIdx.x * (kBlk / 64) + wid; r < plan.runs;
+         r += gridDim.x * (kBlk / 64)) {
+        const int64_t p = static_cast<int64_t>(r) * plan.chunks * 64;
+        append_run(list + p, run_parents[r], run_off[r], pcell + p, poff + p, prod + 12 * p, E32,
+                   nx, sec, ion);
     }
 }
 
 // ------------------------------------------- allocation-free collide
 // aurora_hip_mcc_collide_device keeps its only scratch, one tally row
-// (per-channel energy sums and counters) per wave of its launch, in this
-// array: at most kNoAllocGroups workgroups, so kNoAllocRows rows of
-// kTallyStride words (1.19 MiB per device, held until the process ends).  Host code never passes the array's name to a
-// kernel: it uses the device address resolved per device by
+// (per-channel energy sums and counters) per workgroup of its launch, in this
+// array: at most kNoAllocGroups rows of kTallyStride words (320 KiB per
+// device, held until the process ends).  Host code never passes the array's
+// name to a kernel: it uses the device address resolved per device by
 // collide_scratch_init.
 constexpr int kNoAllocGroups = 2048;
-constexpr int64_t kNoAllocRows = static_cast<int64_t>(kNoAllocGroups) * (kBlk / 64);
-static __device__ __align__(256) double scratch[kNoAllocRows * kTallyStride];
+static __device__ __align__(256) double scratch[kNoAllocGroups * kTallyStride];
 
 constexpr int kMaxDevices = 64;
 std::mutex scratch_mutex;
 std::array<double*, kMaxDevices> scratch_ptr{};
 
-// Clears the caller's outputs (a kernel, not a memset, so the call can be
-// captured in a graph).
-__global__ void k_clear_collide_outputs(unsigned long long* counts, int ncounts,
-                                        double* energy, int nenergy, uint32_t* status) {
-    const int t = threadIdx.x;
-    if (t < ncounts) counts[t] = 0;
-    if (t < nenergy) energy[t] = 0.0;
-    if (t == 0) *status = 0;
+// the launch of a bare collide: fn<NCH, LDS, ONE_V>
+template <typename F>
+void with_collide(const MccParams& m, bool one_v, F&& fn) {
+    with_model(m.nchan, mcc_tables_fit(m), [&]<int NCH, bool LDS>() {
+        if (one_v) fn.template operator()<NCH, LDS, true>();
+        else fn.template operator()<NCH, LDS, false>();
+    });
 }
-
-// The device error bits of a collide as an aurora_status.
-__global__ void k_collide_status(uint32_t* status) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    const uint32_t b = *status;
-    *status = b == 0                          ? AURORA_OK
-              : (b & DEV_ERR_RATE)            ? AURORA_ERR_RATE_ABOVE_BOUND
-              : (b & DEV_ERR_CANDIDATES)      ? AURORA_ERR_CANDIDATE_LIMIT
-                                              : AURORA_ERR_INVALID_ARGUMENT;
-}
-
-int blocks(const Context& c, int64_t n) {
-    int64_t g = (n + kBlk - 1) / kBlk;
-    const int64_t cap = static_cast<int64_t>(c.cu_count) * 8;
-    return static_cast<int>(g < 1 ? 1 : (g > cap ? cap : g));
-}
-
-// energy rows of a launch of g workgroups: one row per wave
-int64_t energy_rows(int g) { return static_cast<int64_t>(g) * (kBlk / 64); }
 
 }  // namespace
 
@@ -510,18 +510,22 @@ void mcc_collide_pass(Context& c, int model, double dt, const CommitArgs& commit
         AUR_HIP(hipGetLastError());
         return;
     }
-    const int64_t nchunks = (n + kBlk - 1) / kBlk;
-    if (h.product_count.count < static_cast<size_t>(n)) {
-        h.product_count.alloc(n);
-        h.product_loff.alloc(n);
+    const bool products = h.secondary_species >= 0;
+    const int g = mcc_groups(c.cu_count, n);
+    const int64_t runs = max_runs(n, static_cast<int64_t>(g) * (kMccBlock / 64));
+    if (products && h.product_list.count < static_cast<size_t>(n)) {
+        h.product_list.alloc(n);
         h.product_vel.alloc(static_cast<size_t>(n) * 12);
     }
-    if (h.chunk_tot.count < static_cast<size_t>(nchunks)) {
-        h.chunk_tot.alloc(nchunks);
-        h.chunk_off.alloc(nchunks);
+    if (products && h.run_tot.count < static_cast<size_t>(runs)) {
+        h.run_tot.alloc(runs);
+        h.run_off.alloc(runs);
+        h.run_parents.alloc(runs);
     }
-    const bool products = h.secondary_species >= 0;
-    const MccParams m = mcc_step_params(c, model);
+    if (h.energy_rows.count < static_cast<size_t>(g * kTallyStride))
+        h.energy_rows.alloc(static_cast<size_t>(g * kTallyStride));
+    MccParams m = mcc_step_params(c, model);
+    m.no_candidate = no_candidate_draws(static_cast<float>(dt), m.inv_max_frequency);
     Mcc1dArgs a{};
     a.cell = sp.cell.ptr;
     a.off = reinterpret_cast<float*>(sp.off[0].ptr);
@@ -538,37 +542,20 @@ void mcc_collide_pass(Context& c, int model, double dt, const CommitArgs& commit
     a.stream = static_cast<uint32_t>(model);
     a.one_v = c.velocity_dims == 1 ? 1 : 0;
     a.step = static_cast<uint32_t>(c.step_count);
-    a.nprod = h.product_count.ptr;
-    a.prod = h.product_vel.ptr;
-    a.err = c.dev_error.ptr;
-    a.loff = products ? h.product_loff.ptr : nullptr;
-    a.chunk_tot = products ? h.chunk_tot.ptr : nullptr;
+    a.prod = products ? h.product_vel.ptr : nullptr;
+    a.list = h.product_list.ptr;
+    a.run_tot = h.run_tot.ptr;
+    a.run_parents = h.run_parents.ptr;
     a.nslots = nslots;
     KernelScope ks(c, "mcc");
+    with_collide(m, a.one_v != 0, [&]<int NCH, bool LDS, bool ONE_V>() {
+        k_mcc_1d<NCH, LDS, ONE_V><<<g, kMccBlock, 0, c.stream>>>(m, a, h.energy_rows.ptr);
+    });
     with_nchan(m.nchan, [&]<int NCH>() {
-        // one round of resident workgroups (grid-stride; a partial second
-        // round would leave most of the chip idle at its end), which also
-        // keeps the tally rows few for the one-block fold that follows
-        auto occupancy = [](auto kernel) {
-            int v = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, kernel, kBlk, 0) != hipSuccess)
-                v = 1;
-            return std::max(1, v);
-        };
-        static const int per_cu[2] = {occupancy(k_mcc_1d<NCH, false>),
-                                      occupancy(k_mcc_1d<NCH, true>)};
-        const int g = std::min(blocks(c, n), per_cu[a.one_v ? 1 : 0] * c.cu_count);
-        const int64_t rows = g;   // one per workgroup
-        if (h.energy_rows.count < static_cast<size_t>(rows * kTallyStride))
-            h.energy_rows.alloc(static_cast<size_t>(rows * kTallyStride));
-        if (a.one_v)
-            k_mcc_1d<NCH, true><<<g, kBlk, 0, c.stream>>>(m, a, h.energy_rows.ptr);
-        else
-            k_mcc_1d<NCH, false><<<g, kBlk, 0, c.stream>>>(m, a, h.energy_rows.ptr);
-        k_mcc_finish<NCH><<<1, kBlk, 0, c.stream>>>(h.energy_rows.ptr, rows,
-                                                    h.energy_change.ptr, h.counts.ptr,
-                                                    a.chunk_tot, h.chunk_off.ptr, nchunks, nslots,
-                                                    total, commit);
+        k_mcc_finish<NCH><<<1, kFold, 0, c.stream>>>(
+            h.energy_rows.ptr, g, h.energy_change.ptr, h.counts.ptr,
+            products ? h.run_tot.ptr : nullptr, h.run_off.ptr, n, nslots, total, c.dev_error.ptr,
+            commit);
     });
     AUR_HIP(hipGetLastError());
 }
@@ -606,9 +593,10 @@ void mcc_append(Context& c, int model, int64_t total, double dt, const long long
     }
     {
         KernelScope ks(c, "append_products");
-        k_append_products<<<std::min(blocks(c, n), 4 * c.cu_count), kBlk, 0, c.stream>>>(
-            sp.cell.ptr, reinterpret_cast<const float*>(sp.off[0].ptr), h.product_count.ptr,
-            h.product_loff.ptr, h.chunk_off.ptr, h.product_vel.ptr, n, c.E32.ptr,
+        const int g = mcc_groups(c.cu_count, n);
+        k_append_products<<<g, kBlk, 0, c.stream>>>(
+            sp.cell.ptr, reinterpret_cast<const float*>(sp.off[0].ptr), h.product_list.ptr,
+            h.run_parents.ptr, h.run_off.ptr, h.product_vel.ptr, n, g, c.E32.ptr,
             static_cast<int>(c.n[0]), sec, ion, place);
         AUR_HIP(hipGetLastError());
     }
@@ -1129,21 +1117,21 @@ int aurora_hip_mcc_collide(aurora_hip_ctx* hctx, int64_t count, double* velocity
         DevBuf<double> ech;
         cnt.alloc(kMaxChannels + 3);
         ech.alloc(kMaxChannels);
-        AUR_HIP(hipMemset(cnt.ptr, 0, (kMaxChannels + 3) * sizeof(unsigned long long)));
-        AUR_HIP(hipMemset(ech.ptr, 0, kMaxChannels * sizeof(double)));
-        const MccParams m = mcc_params(c);
+        MccParams m = mcc_params(c);
+        m.no_candidate = no_candidate_draws(static_cast<float>(dt), m.inv_max_frequency);
         {
             KernelScope ks(c, "collide");
-            const int g = blocks(c, count);
+            const int g = mcc_groups(c.cu_count, count);
             DevBuf<double> rows;
-            rows.alloc(static_cast<size_t>(energy_rows(g) * kTallyStride));
-            with_nchan(m.nchan, [&]<int NCH>() {
-                k_collide<NCH><<<g, kBlk, 0, c.stream>>>(
+            rows.alloc(static_cast<size_t>(g * kTallyStride));
+            with_collide(m, c.velocity_dims == 1, [&]<int NCH, bool LDS, bool ONE_V>() {
+                k_collide<NCH, LDS, ONE_V><<<g, kMccBlock, 0, c.stream>>>(
                     m, dv.ptr, count, static_cast<float>(dt), h.seed, stream_id,
-                    static_cast<uint32_t>(step), rows.ptr, c.dev_error.ptr,
-                    c.velocity_dims == 1 ? 1 : 0);
-                k_fold_rows<NCH><<<1, kBlk, 0, c.stream>>>(rows.ptr, energy_rows(g), ech.ptr,
-                                                           cnt.ptr);
+                    static_cast<uint32_t>(step), rows.ptr);
+            });
+            with_nchan(m.nchan, [&]<int NCH>() {
+                k_collide_finish<NCH><<<1, kFold, 0, c.stream>>>(rows.ptr, g, ech.ptr, cnt.ptr,
+                                                                c.dev_error.ptr, 0);
             });
             AUR_HIP(hipGetLastError());
             AUR_HIP(hipStreamSynchronize(c.stream));
@@ -1180,24 +1168,21 @@ int aurora_hip_mcc_collide_device(aurora_hip_ctx* hctx, int64_t count, float* ve
                     "velocity array required");
         double* rows = scratch_ptr[static_cast<size_t>(c.device)];
         AUR_REQUIRE(rows, AURORA_ERR_HIP, "collide scratch not resolved for this device");
-        const int nch = h.nchan;
-        const MccParams m = mcc_params(c);
-        k_clear_collide_outputs<<<1, 64, 0, c.stream>>>(
-            reinterpret_cast<unsigned long long*>(counts), nch + 3, energy_change, nch, status);
+        MccParams m = mcc_params(c);
+        m.no_candidate = no_candidate_draws(static_cast<float>(dt), m.inv_max_frequency);
+        int g = 0;
         if (count > 0) {
-            int64_t g = (count + kBlk - 1) / kBlk;
-            if (g > kNoAllocGroups) g = kNoAllocGroups;
-            const int gi = static_cast<int>(g);
-            with_nchan(m.nchan, [&]<int NCH>() {
-                k_collide<NCH><<<gi, kBlk, 0, c.stream>>>(
+            g = std::min(mcc_groups(c.cu_count, count), kNoAllocGroups);
+            with_collide(m, c.velocity_dims == 1, [&]<int NCH, bool LDS, bool ONE_V>() {
+                k_collide<NCH, LDS, ONE_V><<<g, kMccBlock, 0, c.stream>>>(
                     m, velocity, count, static_cast<float>(dt), h.seed, stream_id,
-                    static_cast<uint32_t>(step), rows, status, c.velocity_dims == 1 ? 1 : 0);
-                k_fold_rows<NCH><<<1, kBlk, 0, c.stream>>>(
-                    rows, energy_rows(gi), energy_change,
-                    reinterpret_cast<unsigned long long*>(counts));
+                    static_cast<uint32_t>(step), rows);
             });
         }
-        k_collide_status<<<1, 64, 0, c.stream>>>(status);
+        with_nchan(m.nchan, [&]<int NCH>() {
+            k_collide_finish<NCH><<<1, kFold, 0, c.stream>>>(
+                rows, g, energy_change, reinterpret_cast<unsigned long long*>(counts), status, 1);
+        });
         AUR_HIP(hipGetLastError());
     });
 }

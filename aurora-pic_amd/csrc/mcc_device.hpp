@@ -16,6 +16,9 @@
 // on the model's channel count with with_nchan().
 #pragma once
 
+#include <algorithm>
+#include <cmath>
+
 #include "aurora_internal.hpp"
 #include "push_device.hpp"
 
@@ -52,6 +55,7 @@ struct MccParams {
     float neutral_vstd;      // 0: cold neutral
     float safe_speed;        // below it the rate bound is provably under max_frequency
     float safe_speed2;       // just under its square: the check is looked at only above
+    uint32_t no_candidate;   // a step's first draws below this (of 2^23) hold no candidate
     // The 1D step books the kinetic energy of each ionization's secondary
     // and ion into the ionization channel (Simulation.cpp:880-902); half
     // their masses, 0 for the bare collide (NullCollisionModel::collide).
@@ -105,11 +109,11 @@ void with_model(int nchan, bool lds, F&& f) {
     });
 }
 
-// Linear interpolation with constant extrapolation (Collision.cpp:221-237,
-// MeanCosineTable::evaluate 296-313) of a table whose n energies start at
-// E + eo and values at S + so (LDS or global).
+// First of n increasing energies at E + eo (LDS or global) that is above x
+// (n: none).  (Three probes a step instead of one, so that half the reads wait
+// for each other: no faster in the collide, 5 % slower in the swarm.)
 __device__ __forceinline__ int xs_upper(const float* E, int eo, int n, float x) {
-    int lo = 0, hi = n;  // first index with E > x
+    int lo = 0, hi = n;
     while (lo < hi) {
         const int mid = (lo + hi) >> 1;
         if (x < E[eo + mid]) hi = mid; else lo = mid + 1;
@@ -117,14 +121,17 @@ __device__ __forceinline__ int xs_upper(const float* E, int eo, int n, float x) 
     return lo;
 }
 
+// Linear interpolation with constant extrapolation (Collision.cpp:221-237,
+// MeanCosineTable::evaluate 296-313) of the table whose n energies start at
+// E + eo and values at S + so; up = xs_upper of x.
 __device__ __forceinline__ float xs_at(const float* E, const float* S, int eo, int so, int n,
                                        int up, float x) {
-    if (x <= E[eo]) return S[so];
-    if (x >= E[eo + n - 1]) return S[so + n - 1];
-    const float e0 = E[eo + up - 1], e1 = E[eo + up];
-    const float s0 = S[so + up - 1], s1 = S[so + up];
+    const int i0 = up > 0 ? up - 1 : 0, i1 = up < n ? up : n - 1;
+    const float first = E[eo], e0 = E[eo + i0], e1 = E[eo + i1];
+    const float s0 = S[so + i0], s1 = S[so + i1];
     const float f = (x - e0) / (e1 - e0);
-    return s0 + f * (s1 - s0);
+    if (x <= first) return S[so];       // (rows may round to one FP32 energy)
+    return i0 < i1 && up > 0 ? s0 + f * (s1 - s0) : s0;
 }
 
 // Cross-section tables as the kernels read them: E holds one energy grid
@@ -415,6 +422,16 @@ __device__ __forceinline__ bool mcc_candidate(const MccParams& m, const XsView& 
         if constexpr (!kLedger) return ch.kind != AURORA_ATTACHMENT;   // draws consumed
         else {
         const float s0 = w[0] + sec[0], s1 = w[1] + sec[1], s2 = w[2] + sec[2];
+        if constexpr (requires { t.prod; }) {
+            if (t.prod && t.nsec < 2) {
+                float* d = t.prod + 6 * t.nsec;
+                d[0] = s0;
+                d[1] = s1;
+                d[2] = s2;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) d[3 + a] = w[a];
+            }
+        } else {
         // selects, not a store through a computed index (which would put the
         // tally in scratch memory)
 #pragma unroll
@@ -425,6 +442,7 @@ __device__ __forceinline__ bool mcc_candidate(const MccParams& m, const XsView& 
             t.sec[k][2] = here ? s2 : t.sec[k][2];
 #pragma unroll
             for (int a = 0; a < 3; ++a) t.ion[k][a] = here ? w[a] : t.ion[k][a];
+        }
         }
         ++t.nsec;
         if (m.half_sec_mass != 0.f) {
@@ -573,139 +591,98 @@ __device__ void mcc_collide_1v(const MccParams& m, const XsView& X, const Channe
     }
 }
 
-// block-level tally reduction into global counters
-struct TallyOut {
-    unsigned long long* counts;  // [candidates, nulls, chan..., secondaries]
-    double* energy_change;       // per channel (J, unweighted)
+// The tallies of a launch without atomics: each lane adds up its particles',
+// at the end the block's lanes are summed in a fixed order and one row per
+// workgroup is stored: NCH energy sums (J, unweighted) at [0, NCH), then
+// candidates, nulls, per-channel collisions and secondaries as integers at
+// [kMaxChannels, kMaxChannels + NCH + 3), and the error bits.  The rows are
+// added in row order, so counts are exact and energies repeat to the bit;
+// and many waves never contend for one counter.
+constexpr int kTallyStride = 2 * kMaxChannels + 4;
+constexpr int kTallyErr = 2 * kMaxChannels + 3;
+
+// A lane's tally: the counters of mcc_candidate, of which candidates, nsec
+// and err are the current particle's (begin, finish) and the others sums.
+// Products go to memory when they are made (prod: 2 x (secondary, ion), or
+// null).  A lane has at most 2^32 / (64 waves) particles, so 32 bits do.
+template <int NCH>
+struct LaneTally {
+    uint32_t candidates, nsec, err;
+    float* prod;
+    uint32_t nulls, chan[NCH];
+    double energy_change[NCH];
+    uint32_t all_candidates, all_nsec, all_err;
+    __device__ __forceinline__ void begin(float* products) {
+        candidates = nsec = err = 0u;
+        prod = products;
+    }
+    __device__ __forceinline__ void finish() {
+        all_candidates += candidates;
+        all_nsec += nsec;
+        all_err |= err;
+    }
+    __device__ __forceinline__ void add(const MccTally<NCH>& t) {
+        all_candidates += t.candidates;
+        all_nsec += static_cast<uint32_t>(t.nsec);
+        all_err |= t.err;
+        nulls += t.nulls;
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            chan[c] += t.chan[c];
+            energy_change[c] += static_cast<double>(t.energy_change[c]);
+        }
+    }
 };
 
-template <int NCH>
-__device__ void flush_tally(const MccTally<NCH>& t, TallyOut out, bool active) {
-    // wave-level sums, then one atomic per counter per wave (integer adds
-    // commute, so counts do not depend on the reduction order)
-    unsigned long long cand = active ? t.candidates : 0, nul = active ? t.nulls : 0;
-    unsigned long long sec = active ? static_cast<unsigned long long>(t.nsec) : 0;
-    for (int off = 32; off > 0; off >>= 1) {
-        cand += __shfl_down(cand, off, 64);
-        nul += __shfl_down(nul, off, 64);
-        sec += __shfl_down(sec, off, 64);
-    }
-    const bool lead = (threadIdx.x & 63) == 0;
-    if (lead) {
-        if (cand) atomicAdd(out.counts, cand);
-        if (nul) atomicAdd(out.counts + 1, nul);
-        if (sec) atomicAdd(out.counts + 2 + NCH, sec);
-    }
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-        unsigned long long n = active ? t.chan[c] : 0;
-        double e = active ? static_cast<double>(t.energy_change[c]) : 0.0;
-        for (int off = 32; off > 0; off >>= 1) {
-            n += __shfl_down(n, off, 64);
-            e += __shfl_down(e, off, 64);
-        }
-        if (lead) {
-            if (n) atomicAdd(out.counts + 2 + c, n);
-            if (e != 0.0) atomicAdd(out.energy_change + c, e);
-        }
-    }
-}
-
-// The tallies of a launch without atomics: each wave sums its lanes'
-// counts and energy changes in a fixed order and, at the end, stores one
-// row: NCH energy sums (J, unweighted) at [0, NCH), then candidates, nulls,
-// per-channel collisions and secondaries as integers at [kMaxChannels,
-// kMaxChannels + NCH + 3).  k_fold_rows adds the rows in row order, so
-// counts are exact and energies repeat to the bit; and many waves never
-// contend for one counter.
-constexpr int kTallyStride = 2 * kMaxChannels + 3;
-
-// Waves per SIMD that the MCC kernels over particles ask of the register
-// allocator: four (at most 128 VGPRs) for three channels, where that fits
-// without spilling; no cap for other channel counts, which would spill.
-constexpr int mcc_min_waves(int nch) { return nch == 3 ? 4 : 1; }
-
-template <int NCH>
-struct WaveTally {
-    double energy[NCH];
-    unsigned long long count[NCH + 3];
-};
-
-__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
-template <int NCH>
-__device__ void flush_tally_rows(const MccTally<NCH>& t, bool active, WaveTally<NCH>& w) {
-    w.count[0] += wave_sum_u64(active ? t.candidates : 0);
-    w.count[1] += wave_sum_u64(active ? t.nulls : 0);
-    w.count[2 + NCH] += wave_sum_u64(active ? static_cast<unsigned long long>(t.nsec) : 0);
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-        w.count[2 + c] += wave_sum_u64(active ? t.chan[c] : 0);
-        w.energy[c] += wave_sum(active ? static_cast<double>(t.energy_change[c]) : 0.0);
-    }
-}
-
-// Stores the wave's row at rows + row * kTallyStride (lane 0).
-template <int NCH>
-__device__ __forceinline__ void store_tally_row(const WaveTally<NCH>& w, double* rows,
-                                                int64_t row) {
-    if ((threadIdx.x & 63) != 0) return;
-    double* r = rows + row * kTallyStride;
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) r[c] = w.energy[c];
-    unsigned long long* n = reinterpret_cast<unsigned long long*>(r + kMaxChannels);
-#pragma unroll
-    for (int k = 0; k < NCH + 3; ++k) n[k] = w.count[k];
-}
-
-// One row per wave of the launch, in wave order.
-template <int NCH>
-__device__ __forceinline__ void store_wave_row(const WaveTally<NCH>& w, double* rows) {
-    store_tally_row<NCH>(w, rows,
-                         static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6));
-}
-
-// One row per workgroup (BLOCK threads, every thread calls it): the waves'
-// tallies added in wave order, stored at rows + row * kTallyStride.
+// One row per workgroup (BLOCK threads, every thread calls it): the lanes'
+// tallies summed per wave, the waves' in wave order, stored at
+// rows + row * kTallyStride.
 template <int NCH, int BLOCK>
-__device__ __forceinline__ void store_block_row(const WaveTally<NCH>& w, double* rows,
+__device__ __forceinline__ void store_block_row(const LaneTally<NCH>& t, double* rows,
                                                 int64_t row) {
     constexpr int W = BLOCK / 64;
     __shared__ double se[W][NCH];
     __shared__ unsigned long long sc[W][NCH + 3];
+    __shared__ uint32_t sx[W];
     const int wid = static_cast<int>(threadIdx.x) >> 6;
-    if ((threadIdx.x & 63) == 0) {
+    const bool lead = (threadIdx.x & 63) == 0;
 #pragma unroll
-        for (int c = 0; c < NCH; ++c) se[wid][c] = w.energy[c];
-#pragma unroll
-        for (int k = 0; k < NCH + 3; ++k) sc[wid][k] = w.count[k];
+    for (int c = 0; c < NCH; ++c) {
+        const double e = wave_sum(t.energy_change[c]);
+        if (lead) se[wid][c] = e;
     }
+#pragma unroll
+    for (int k = 0; k < NCH + 3; ++k) {
+        const unsigned long long n = wave_sum_u64(k == 0         ? t.all_candidates
+                                                  : k == 1       ? t.nulls
+                                                  : k == NCH + 2 ? t.all_nsec
+                                                                 : t.chan[k - 2 < NCH ? k - 2 : 0]);
+        if (lead) sc[wid][k] = n;
+    }
+    const uint32_t err = wave_or(t.all_err);
+    if (lead) sx[wid] = err;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        WaveTally<NCH> t;
+    double* r = rows + row * kTallyStride;
+    unsigned long long* n = reinterpret_cast<unsigned long long*>(r + kMaxChannels);
+    const int i = static_cast<int>(threadIdx.x);
+    if (i < NCH) {
+        double e = se[0][i];
 #pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-            double e = se[0][c];
+        for (int v = 1; v < W; ++v) e += se[v][i];
+        r[i] = e;
+    } else if (i >= 16 && i < 16 + NCH + 3) {
+        unsigned long long k = 0;
 #pragma unroll
-            for (int v = 1; v < W; ++v) e += se[v][c];
-            t.energy[c] = e;
-        }
+        for (int v = 0; v < W; ++v) k += sc[v][i - 16];
+        n[i - 16] = k;
+    } else if (i == 32) {
+        uint32_t e = 0u;
 #pragma unroll
-        for (int k = 0; k < NCH + 3; ++k) {
-            unsigned long long n = 0;
-#pragma unroll
-            for (int v = 0; v < W; ++v) n += sc[v][k];
-            t.count[k] = n;
-        }
-        store_tally_row<NCH>(t, rows, row);
+        for (int v = 0; v < W; ++v) e |= sx[v];
+        reinterpret_cast<unsigned long long*>(r)[kTallyErr] = e;
     }
 }
 
-// Adds rows [0, nrows) in row order: energies into energy[NCH], counts into
-// counts[NCH + 3].  Block of BLOCK threads; every thread calls it.
 // Exclusive scan of one int per thread over a BLOCK-thread block: the
 // wave's prefix by shuffles, the wave totals through LDS (wsum: BLOCK / 64
 // ints); sets total.
@@ -733,11 +710,10 @@ __device__ __forceinline__ int block_scan_int(int x, int* wsum, int& total) {
 }
 
 // off[c] = tot[0] + ... + tot[c - 1] for c < nchunks, by one BLOCK-thread
-// block: each thread sums a consecutive run, its loads issued eight at a
-// time; returns the sum of all totals.
+// block: each thread sums a consecutive run, its loads issued together; returns the sum of all totals.
 template <int BLOCK>
 __device__ int chunk_offsets(const int32_t* tot, int32_t* off, int64_t nchunks, int* wsum) {
-    constexpr int kB = 8;
+    constexpr int kB = BLOCK >= 1024 ? 4 : 8;
     const int64_t per = (nchunks + BLOCK - 1) / BLOCK;
     const int64_t c0 = static_cast<int64_t>(threadIdx.x) * per;
     const int64_t c1 = c0 + per < nchunks ? c0 + per : nchunks;
@@ -765,17 +741,21 @@ __device__ int chunk_offsets(const int32_t* tot, int32_t* off, int64_t nchunks, 
     return total;
 }
 
+// Rows [0, nrows) added in row order and the sums added to (ADD) or stored at
+// energy[NCH] and counts[NCH + 3]; returns the rows' error bits to every
+// thread.  Block of BLOCK threads; every thread calls it.
 // A thread's rows r, r + BLOCK, ... are loaded kFoldBatch at a time (the
 // loads in flight together) and added in that same order.
-template <int NCH, int BLOCK>
-__device__ void fold_tally_rows(const double* rows, int64_t nrows, double* energy,
-                                unsigned long long* counts) {
-    constexpr int kFoldBatch = NCH <= 4 ? 8 : 4;
+template <int NCH, int BLOCK, bool ADD = true>
+__device__ uint32_t fold_tally_rows(const double* rows, int64_t nrows, double* energy,
+                                    unsigned long long* counts) {
+    constexpr int kFoldBatch = BLOCK >= 1024 ? 2 : (NCH <= 4 ? 8 : 4);
     double v[NCH] = {};
     unsigned long long u[NCH + 3] = {};
+    uint32_t err = 0u;
     for (int64_t r0 = threadIdx.x; r0 < nrows; r0 += kFoldBatch * BLOCK) {
         double e[kFoldBatch][NCH];
-        unsigned long long n[kFoldBatch][NCH + 3];
+        unsigned long long n[kFoldBatch][NCH + 3], x[kFoldBatch];
 #pragma unroll
         for (int b = 0; b < kFoldBatch; ++b) {
             const int64_t r = r0 + static_cast<int64_t>(b) * BLOCK;
@@ -786,6 +766,7 @@ __device__ void fold_tally_rows(const double* rows, int64_t nrows, double* energ
             for (int c = 0; c < NCH; ++c) e[b][c] = row[c];
 #pragma unroll
             for (int k = 0; k < NCH + 3; ++k) n[b][k] = cnt[k];
+            x[b] = reinterpret_cast<const unsigned long long*>(row)[kTallyErr];
         }
 #pragma unroll
         for (int b = 0; b < kFoldBatch; ++b) {
@@ -794,60 +775,29 @@ __device__ void fold_tally_rows(const double* rows, int64_t nrows, double* energ
             for (int c = 0; c < NCH; ++c) v[c] += e[b][c];
 #pragma unroll
             for (int k = 0; k < NCH + 3; ++k) u[k] += n[b][k];
+            err |= static_cast<uint32_t>(x[b]);
         }
     }
     const double s = block_sum<NCH, BLOCK>(v);
-    if (threadIdx.x < NCH) energy[threadIdx.x] += s;
+    if (threadIdx.x < NCH) energy[threadIdx.x] = ADD ? energy[threadIdx.x] + s : s;
     // counts: integer sums, any order gives the same value
     __shared__ unsigned long long cs[NCH + 3];
+    __shared__ uint32_t sx;
     if (threadIdx.x < NCH + 3) cs[threadIdx.x] = 0;
+    if (threadIdx.x == 0) sx = 0u;
     __syncthreads();
+    if (err) atomicOr(&sx, err);
 #pragma unroll
     for (int k = 0; k < NCH + 3; ++k) {
         const unsigned long long x = wave_sum_u64(u[k]);
         if ((threadIdx.x & 63) == 0 && x) atomicAdd(cs + k, x);
     }
     __syncthreads();
-    if (threadIdx.x < NCH + 3) counts[threadIdx.x] += cs[threadIdx.x];
+    if (threadIdx.x < NCH + 3)
+        counts[threadIdx.x] = (ADD ? counts[threadIdx.x] : 0ull) + cs[threadIdx.x];
+    const uint32_t all = sx;
     __syncthreads();
-}
-
-// One live 1D target particle of the MCC step (Simulation.cpp:900-926):
-// synchronise v from v_half with E(x) at t+dt (Pusher.cpp:74-76), collide,
-// rebuild v_half (Pusher.cpp:66-68).  Up to two ionization product pairs
-// (secondary v, ion v) are staged at prod[0..12); returns their number.
-template <int NCH>
-__device__ __forceinline__ int mcc_1d_particle(const MccParams& m, const XsView& X,
-                                               const ChannelSel* chan, int c, float o, float* v0, float* v1, float* v2,
-                                               uint32_t uid, const float* E32, int nx,
-                                               float half_qm_dt, float dt, uint64_t seed,
-                                               uint32_t step, float* prod, MccTally<NCH>& t,
-                                               uint32_t* err, uint32_t stream = 0u,
-                                               bool one_v = false) {
-    const float ex = gather_1d_f32(E32, nx, c, o);
-    const float kick = half_qm_dt * ex;
-    float u[3] = {*v0 + kick, *v1, *v2};
-    Philox rng;
-    rng.init(seed, stream, uid, step);
-    if (one_v)
-        mcc_collide_1v<NCH>(m, X, chan, u[0], dt, rng, t);   // 1D1V: v_y, v_z stay as they are
-    else
-        mcc_collide<NCH>(m, X, chan, u, dt, rng, t);
-    if (t.err) atomicOr(err, t.err);
-    *v0 = u[0] - kick;
-    *v1 = u[1];
-    *v2 = u[2];
-    const int np = t.nsec < 2 ? t.nsec : 2;
-    if (t.nsec > 2) atomicOr(err, DEV_ERR_CAPACITY);
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-        if (k < np)
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                prod[6 * k + q] = t.sec[k][q];
-                prod[6 * k + 3 + q] = t.ion[k][q];
-            }
-    return np;
+    return all;
 }
 
 struct AppendSide {
@@ -892,6 +842,7 @@ __device__ __forceinline__ void append_products_of(int c, float o, int np, int64
 struct MccLds {
     float words[kMccLdsWords];
     ChannelSel chan[kMaxChannels];
+    MccParams params;        // collide_run's copy
 };
 
 // energy rows staged: one grid for all channels, or every channel's
@@ -940,6 +891,15 @@ __device__ __forceinline__ void stage_tables_as(const MccParams& m, MccLds& lds)
     }
     __syncthreads();
 }
+// and the parameters
+template <bool LDS>
+__device__ __forceinline__ void stage_model(MccLds& lds) {
+    using Words = const __attribute__((address_space(4))) uint32_t*;
+    const Words m = (Words)__builtin_amdgcn_kernarg_segment_ptr();
+    for (unsigned i = threadIdx.x; i < sizeof(MccParams) / 4; i += blockDim.x)
+        reinterpret_cast<uint32_t*>(&lds.params)[i] = m[i];
+    stage_tables_as<LDS>(first_kernel_argument<MccParams>(), lds);
+}
 template <bool LDS>
 __device__ __forceinline__ XsView table_view(const MccParams& m, const MccLds& lds) {
     if constexpr (LDS)
@@ -948,7 +908,306 @@ __device__ __forceinline__ XsView table_view(const MccParams& m, const MccLds& l
         return XsView{m.energy, m.sigma, 0};
 }
 
+// ------------------------------------------------ collisions of many particles
+// One step's collisions of a run of slots, by one wave.  Nine particles in
+// ten meet no candidate, so the wave goes over its slots twice:
+//   sweep    every particle's first Philox block; a first draw that cannot
+//            hold a candidate (no_candidate, proved on the host) ends its
+//            step, the others' indices go to the wave's LDS queue
+//   collide  each lane takes a queued particle and runs its candidate loop
+//            one waiting time at a time; a lane that is done takes the next,
+//            so the long code runs on full waves
+// A particle's operations and draws are those of mcc_collide, and its result
+// does not depend on its lane, so neither does anything written per particle.
+// A run holds at most 64 kRunChunks slots.  Latency bounds a launch of up to a
+// million particles (62 % of the wave cycles wait, mostly on LDS), VALU issue
+// larger ones.  Measured, 1e6 bare collides 55.8 -> 21.6 us; the 1D step at
+// 5e5 electrons 38.5 -> 25.1 us, 64 instances of 1e5 155 -> 60.7 us (one
+// particle per lane before, every lane through the whole candidate code).
+constexpr int kRunChunks = 16;
+constexpr int kSweepUnroll = 4;     // chunks whose loads are in flight together
+constexpr int kRefill = 32;         // lanes that are done before the wave takes new ones
+
+struct WaveQueue {
+    uint16_t index[64 * kRunChunks];
+    uint8_t products[64 * kRunChunks];   // ionizations of each particle
+};
+
+// The runs of n slots over `waves` waves: `passes` runs each, of `chunks`
+// 64-slot chunks (one pass of short runs until they are full).
+struct RunPlan {
+    uint32_t chunks, runs;
+    __host__ __device__ __forceinline__ RunPlan(int64_t n, uint32_t waves) {
+        const uint32_t all = static_cast<uint32_t>((n + 63) >> 6);
+        chunks = (all + waves - 1) / waves;
+        if (chunks > kRunChunks) {
+            const uint32_t passes = (chunks + kRunChunks - 1) / kRunChunks;
+            chunks = (chunks + passes - 1) / passes;
+        }
+        if (chunks < 1) chunks = 1;
+        runs = (all + chunks - 1) / chunks;
+    }
+};
+// at least the runs of any slot count up to n
+inline int64_t max_runs(int64_t n, int64_t waves) {
+    const int64_t full = 64 * kRunChunks * waves;
+    return waves * std::max<int64_t>(1, (n + full - 1) / full);
+}
+
+// The waves that collide one population: kMccWaves per SIMD of the chip, in
+// workgroups of kMccBlock; fewer when there are fewer chunks.  More
+// waves hide more latency, fewer pack their lanes better: 2, 3 and 4 per SIMD
+// take 26.8, 27.0 and 28.7 us at 5e5 electrons, 76.8, 63.4 and 59.7 us at 64
+// instances (3.2e6), and the one-workgroup folds grow with them.
+constexpr int kMccBlock = 256;
+constexpr int kMccWaves = 3;
+inline int mcc_groups(int cu_count, int64_t n) {
+    const int64_t resident = static_cast<int64_t>(cu_count) * kMccWaves * 4 / (kMccBlock / 64);
+    return static_cast<int>(std::clamp<int64_t>((n + kMccBlock - 1) / kMccBlock, 1, resident));
+}
+
+// orders a wave's LDS accesses before and after it (its lanes run together)
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Collides the run's `slots` slots; Io gives them:
+//   fetch(i, state)     loads slot i; false: nothing alive there
+//   velocity(state, u)  the velocity to collide
+//   id(state, i)        the random stream
+//   products(i)         where its products go, or null
+//   pass(i, state, u)   a particle that meets no candidate
+//   store(i, state, u)  one that went through the candidate loop
+// and whether any particle of the run made products (their numbers in
+// q.products) is returned.
+template <int NCH, bool LDS, bool ONE_V, typename Io>
+__device__ __forceinline__ bool collide_run(const MccLds& lds, WaveQueue& q, const Io& io,
+                                            int slots, float dt, uint64_t seed, uint32_t stream,
+                                            uint32_t step, LaneTally<NCH>& t) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t below = (uint64_t{1} << lane) - 1;
+    int queued = 0;
+    {
+        const MccParams& m = lds.params;
+        const uint32_t no_candidate = m.no_candidate;
+        const float safe_speed2 = m.safe_speed2;
+        for (int base = 0; base < slots; base += 64 * kSweepUnroll) {
+            typename Io::State st[kSweepUnroll];
+            bool in[kSweepUnroll];
+            float u[kSweepUnroll][3];
+#pragma unroll
+            for (int k = 0; k < kSweepUnroll; ++k) {
+                const int i = base + 64 * k + lane;
+                in[k] = io.fetch(i < slots ? i : 0, st[k]) && i < slots;
+            }
+#pragma unroll
+            for (int k = 0; k < kSweepUnroll; ++k) io.velocity(st[k], u[k]);
+#pragma unroll
+            for (int k = 0; k < kSweepUnroll; ++k) {
+                if (base + 64 * k >= slots) break;
+                const int i = base + 64 * k + lane;
+                Philox rng;
+                rng.init(seed, stream, io.id(st[k], i), step);
+                rng.refill();
+                const float v2 = ONE_V ? u[k][0] * u[k][0]
+                                       : u[k][0] * u[k][0] + u[k][1] * u[k][1] + u[k][2] * u[k][2];
+                const bool collide =
+                    in[k] && ((rng.b0 >> 9) >= no_candidate || !(v2 <= safe_speed2));
+                if (in[k] && !collide) io.pass(i, st[k], u[k]);
+                const uint64_t mask = __ballot(collide);
+                if (collide) q.index[queued + __popcll(mask & below)] = static_cast<uint16_t>(i);
+                queued += __popcll(mask);
+                if (Io::kProducts) q.products[i] = 0;
+            }
+        }
+    }
+    wave_lds_fence();
+    if constexpr (ONE_V) {
+        for (int h = lane; h < queued; h += 64) {
+            const MccParams& m = lds.params;
+            const XsView X = table_view<LDS>(m, lds);
+            const int i = q.index[h];
+            typename Io::State st;
+            float u[3];
+            io.fetch(i, st);
+            io.velocity(st, u);
+            Philox rng;
+            rng.init(seed, stream, io.id(st, i), step);
+            MccTally<NCH> one{};
+            mcc_collide_1v<NCH>(m, X, lds.chan, u[0], dt, rng, one);
+            io.store(i, st, u);
+            t.add(one);
+        }
+        wave_lds_fence();
+        return false;
+    } else {
+        int head = 0, i = -1;
+        bool made = false;
+        typename Io::State st{};
+        float u[3] = {0.f, 0.f, 0.f};
+        float elapsed = 0.f;
+        Philox rng;
+        rng.init(seed, stream, 0u, step);
+        while (head < queued || __ballot(i >= 0) != 0ull) {
+            const uint64_t idle = __ballot(i < 0);
+            if (head < queued && __popcll(idle) >= kRefill) {
+                const int h = head + __popcll(idle & below);
+                if (i < 0 && h < queued) {
+                    i = q.index[h];
+                    io.fetch(i, st);
+                    io.velocity(st, u);
+                    rng.c0 = 0u;
+                    rng.c1 = io.id(st, i);
+                    rng.used = 4;
+                    t.begin(io.products(i));
+                    elapsed = 0.f;
+                }
+                head += __popcll(idle);
+            }
+            if (i >= 0) {
+                // mcc_collide from one waiting time to the next
+                const MccParams& m = lds.params;
+                const XsView X = table_view<LDS>(m, lds);
+                bool again = false;
+                if (!(u[0] * u[0] + u[1] * u[1] + u[2] * u[2] <= m.safe_speed2)) {
+                    if (t.candidates == 0u &&
+                        (!isfinite(u[0]) || !isfinite(u[1]) || !isfinite(u[2])))
+                        t.err = DEV_ERR_NONFINITE;
+                    else if (mcc_rate_fails<NCH>(m, X, u))
+                        t.err = DEV_ERR_RATE;
+                }
+                if (t.err == 0u) {
+                    const float waiting = -logf(rng.u01()) * m.inv_max_frequency;
+                    if (waiting < dt - elapsed) {
+                        elapsed += waiting;
+                        ++t.candidates;
+                        if (t.candidates > static_cast<uint32_t>(m.max_candidates))
+                            t.err = DEV_ERR_CANDIDATES;
+                        else
+                            again = mcc_candidate<NCH>(m, X, lds.chan, u, rng, t);
+                    }
+                }
+                if (!again) {
+                    io.store(i, st, u);
+                    if (Io::kProducts && t.nsec != 0u) {
+                        q.products[i] = static_cast<uint8_t>(t.nsec < 2u ? t.nsec : 2u);
+                        made = true;
+                        if (t.nsec > 2u) t.err |= DEV_ERR_CAPACITY;
+                    }
+                    t.finish();
+                    i = -1;
+                }
+            }
+        }
+        wave_lds_fence();
+        return __ballot(made) != 0ull;
+    }
+}
+
+// The parents of a run with products, in slot order, as words
+// slot | products << 10 | products before it in the run << 12; written at
+// list, their number to *parents and the products' to *total.
+__device__ __forceinline__ void list_parents(const WaveQueue& q, int slots, bool made,
+                                             int32_t* list, int32_t* parents, int32_t* total) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t below = (uint64_t{1} << lane) - 1;
+    int np = 0, nt = 0;
+    if (made)
+        for (int base = 0; base < slots; base += 64) {
+            const int i = base + lane;
+            const int c = i < slots ? q.products[i] : 0;
+            const uint64_t m1 = __ballot(c > 0), m2 = __ballot(c > 1);
+            if (c > 0)
+                list[np + __popcll(m1 & below)] =
+                    i | (c << 10) |
+                    ((nt + __popcll(m1 & below) + __popcll(m2 & below)) << 12);
+            np += __popcll(m1);
+            nt += __popcll(m1) + __popcll(m2);
+        }
+    if (lane == 0) {
+        *parents = np;
+        *total = nt;
+    }
+}
+
+// A 1D target species' run (Simulation.cpp:900-926): the velocity to collide
+// is v synchronised from v_half with E(x) at t+dt (Pusher.cpp:74-76), the
+// stored one v_half rebuilt (Pusher.cpp:66-68), also without a collision.
+struct Run1d {
+    const int32_t* cell;     // the run's first slot, as all below
+    const float* off;
+    float* v0;
+    float* v1;
+    float* v2;
+    const uint32_t* uid;
+    float* prod;             // per slot: 2 x (secondary v[3], ion v[3])
+    const float* E32;
+    int nx;
+    float half_qm_dt;
+    static constexpr bool kProducts = true;
+    struct State {
+        float kick;
+        float v[3];
+        uint32_t uid;
+        int c;
+        float o;
+    };
+    __device__ __forceinline__ bool fetch(int i, State& s) const {
+        s.c = cell[i];
+        s.o = off[i];
+        s.v[0] = v0[i];
+        s.v[1] = v1[i];
+        s.v[2] = v2[i];
+        s.uid = uid[i];
+        return s.c >= 0;
+    }
+    __device__ __forceinline__ void velocity(State& s, float* u) const {
+        s.kick = half_qm_dt * gather_1d_f32(E32, nx, s.c >= 0 ? s.c : 0, s.o);
+        u[0] = s.v[0] + s.kick;
+        u[1] = s.v[1];
+        u[2] = s.v[2];
+    }
+    __device__ __forceinline__ uint32_t id(const State& s, int) const { return s.uid; }
+    __device__ __forceinline__ float* products(int i) const {
+        return prod ? prod + 12 * static_cast<int64_t>(i) : nullptr;
+    }
+    __device__ __forceinline__ void pass(int i, const State& s, const float* u) const {
+        v0[i] = u[0] - s.kick;
+    }
+    __device__ __forceinline__ void store(int i, const State& s, const float* u) const {
+        v0[i] = u[0] - s.kick;
+        v1[i] = u[1];
+        v2[i] = u[2];
+    }
+};
+
+// Adds a run's products to the secondary and ion species: lane after lane
+// takes a listed parent (see list_parents), whose products start at index
+// first + (those before it in the run).
+__device__ __forceinline__ void append_run(const int32_t* list, int parents, int64_t first,
+                                           const int32_t* cell, const float* off,
+                                           const float* prod, const float* E32, int nx,
+                                           const AppendSide& sec, const AppendSide& ion) {
+    for (int k = threadIdx.x & 63; k < parents; k += 64) {
+        const int e = list[k];
+        const int i = e & 1023;
+        append_products_of(cell[i], off[i], (e >> 10) & 3, first + (e >> 12),
+                           prod + 12 * static_cast<int64_t>(i), E32, nx, sec, ion);
+    }
+}
+
 // ------------------------------------------------------------- host side
+// Draws of a step's first uniform u = (2k + 1) 2^-24 that cannot hold a
+// candidate: -log(u) / max_frequency >= dt for every k below this, with 1e-4
+// of the exponent left for the FP32 logarithm, product and timestep (off by
+// a few 1e-7 of it).
+inline uint32_t no_candidate_draws(float dt, float inv_max_frequency) {
+    const double x = static_cast<double>(dt) / static_cast<double>(inv_max_frequency);
+    const double k = std::floor(std::exp(-x * (1.0 + 1.0e-4)) * 0x1p23) - 2.0;
+    return k > 0.0 ? static_cast<uint32_t>(k) : 0u;
+}
+
 // Validated model tables (NullCollisionModel ctor, Collision.cpp:315-577)
 // into h; particle_mass is the projectile mass.
 void load_mcc_model(MccModelHost& h, int nchan, const int* kind, const double* threshold,

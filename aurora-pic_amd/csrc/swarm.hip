@@ -72,16 +72,6 @@ struct WorkItem {
 constexpr int kCandidateBatch = 32;
 constexpr int kLdsBlocks = 32;
 
-// Draws of a step's first uniform u = (2k + 1) 2^-24 that cannot hold a
-// candidate: -log(u) / max_frequency >= dt for every k below this, with 1e-4
-// of the exponent left for the FP32 logarithm, product and timestep (off by
-// a few 1e-7 of it).
-uint32_t no_candidate_draws(float dt, float inv_max_frequency) {
-    const double x = static_cast<double>(dt) / static_cast<double>(inv_max_frequency);
-    const double k = std::floor(std::exp(-x * (1.0 + 1.0e-4)) * 0x1p23) - 2.0;
-    return k > 0.0 ? static_cast<uint32_t>(k) : 0u;
-}
-
 // the largest FP32 squared speed x with fl(ev x) <= limit: the energy check
 // e > limit on an electron is x > v2_ceiling
 float v2_ceiling(float limit, float ev) {

@@ -572,3 +572,36 @@ def test_thermal_frequency_bound_at_every_speed(ctx, spike_ev, height, density):
             ctx.mcc_collide(v, 1e-3 / numax, step=0)
         seen.add(b > 1.0)
     assert True in seen and (False in seen or density > 1.0)
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 257, 131073, 2097153])
+@pytest.mark.parametrize("part", [0.05, 1.0])
+def test_collide_at_the_edges_of_a_waves_run(ctx, oracle, n, part):
+    # a wave sweeps a run of up to 1,024 particles and collides the few that
+    # may meet a candidate (most of them with the full step) packed into its
+    # lanes: a particle's outcome is that of its own stream wherever it lies.
+    # Particles on both sides of every chunk and run edge near the ends and in
+    # the middle against the oracle, by the bar of this file.
+    g = golden("mcc_stats.npz")
+    gas = workloads.synthetic_gas(rows=200)
+    model = oracle_py.model_from_gas(workloads.synthetic_gas(rows=200))
+    _load(ctx, gas["channels"], gas["neutral_density"], gas["max_frequency"], workloads.ME,
+          neutral_mass=gas["neutral_mass"], seed=8128)
+    some = g["vin"].astype(np.float32).astype(np.float64)
+    vin = some[np.arange(n) % some.shape[0]]
+    dt = float(g["dt"]) * part
+    vout, counts, ech = ctx.mcc_collide(vin, dt, step=3, stream_id=2)
+    again, counts2, ech2 = ctx.mcc_collide(vin, dt, step=3, stream_id=2)
+    assert np.array_equal(vout, again) and list(counts) == list(counts2)
+    assert list(ech) == list(ech2)
+    assert int(counts[0]) == int(sum(counts[1:5]))
+    edges = np.concatenate([np.arange(0, n, e)[[0, 1, -2, -1] if n > 2 * e else [0, -1]]
+                            for e in (64, 128, 576, 1024)] + [[n]])
+    at = np.unique(np.clip(np.concatenate([edges + k for k in (-33, -2, -1, 0, 1, 31)]), 0, n - 1))
+    far = []
+    for p in at:
+        ov, st = oracle.collide(model, vin[p], dt, 8128, 2, int(p), 3)
+        if np.max(np.abs(vout[p] - ov)) > 1e-4 * np.linalg.norm(ov) + 1e-3:
+            far.append(st.margin)
+    assert max(far, default=0.0) <= MARGIN
+    assert len(far) <= 0.02 * at.size + 1
