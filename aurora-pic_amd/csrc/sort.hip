@@ -654,6 +654,7 @@ void sort_species(Context& c, Species& sp) {
                           sp.tile_keyspace == static_cast<int64_t>(keyspace);
     if (local_ok && (sp.precision == 64 ? local_sort<double>(c, sp, k, ntz, bits)
                                         : local_sort<float>(c, sp, k, ntz, bits))) {
+        sp.general_sort = false;
         finish_sort(c, sp, timed);
         return;
     }
@@ -694,6 +695,7 @@ void sort_species(Context& c, Species& sp) {
     AUR_HIP(hipStreamSynchronize(c.stream));
     sp.slots = live;
     sp.tile_keyspace = static_cast<int64_t>(keyspace);
+    sp.general_sort = true;
     finish_sort(c, sp, timed);
 }
 
