@@ -660,6 +660,7 @@ int aurora_hip_initialize(aurora_hip_ctx* h, double dt) {
             if (sp.ledger.ptr)
                 AUR_HIP(hipMemsetAsync(sp.ledger.ptr, 0, 3 * sizeof(double), c.stream));
             sp.ledger_pending = false;
+            sp.work = Species::kWorkNone;
         }
         deposit_all(c);
         convert_rho(c);
@@ -681,14 +682,16 @@ int aurora_hip_step(aurora_hip_ctx* h, double dt, int64_t nsteps) {
         const bool dev_counts = nsteps > 0 && device_counts_apply(c);
         struct Leave {
             Context& c;
+            double dt;
             ~Leave() {
                 try {
+                    if (c.dim == 1) ledger_flush_1d(c, dt);
                     device_counts_leave(c);
                 } catch (...) {
                     c.counts_on_device = false;
                 }
             }
-        } leave{c};
+        } leave{c, dt};
         if (dev_counts) device_counts_enter(c);
         for (int64_t s = 0; s < nsteps; ++s) {
             // kick + drift + boundary + deposit at x^{n+1} (fused)
@@ -702,16 +705,19 @@ int aurora_hip_step(aurora_hip_ctx* h, double dt, int64_t nsteps) {
             if (c.sort_policy == AURORA_SORT_ADAPTIVE) {
                 for (auto& sp : c.species)
                     if (adaptive_sort_due(c, sp)) {
+                        if (c.dim == 1) ledger_flush_1d(c, dt);
                         device_counts_leave(c);
                         sort_species(c, sp);
                     }
             } else if (c.sort_interval > 0 && c.step_count % c.sort_interval == 0) {
+                if (c.dim == 1) ledger_flush_1d(c, dt);
                 device_counts_leave(c);
                 for (auto& sp : c.species)
                     if (sort_needed(c, sp)) sort_species(c, sp);
             }
             if (dev_counts && !c.counts_on_device && s + 1 < nsteps) device_counts_enter(c);
         }
+        if (c.dim == 1) ledger_flush_1d(c, dt);
         device_counts_leave(c);
         check_device_error(c);
         flush_timers(c);

@@ -186,10 +186,19 @@ struct Species {
     // solve; one finalize kernel folds the partials in block order, so the
     // totals do not depend on scheduling.
     DevBuf<double> ledger;                // 3
-    DevBuf<double> ledger_part;           // 3 per push block, then 1 per work block
+    DevBuf<double> ledger_part;           // 4 per push block, then 1 per work block
     DevBuf<double> vold;                  // synchronised v_x at the start of the step
     int ledger_push_blocks = 0;           // grid of the last push
     bool ledger_pending = false;          // push partials not yet folded
+    // 1D: the survivors' work of the last push (none, to be summed, or summed
+    // in the work partials), that push's grid, and the slots it had (two words
+    // in turn, on the device)
+    enum WorkState { kWorkNone, kWorkDue, kWorkSummed };
+    WorkState work = kWorkNone;
+    bool work_in_push = false;            // the push partials hold the step before's
+    int work_blocks = 0;
+    DevBuf<long long> pushed_slots;
+    int pushed_turn = 0;
     DevBuf<int32_t> tile_start;           // ntiles + 1 segment starts after a sort
     bool tiled = false;                   // storage is tile-sorted (tile_start valid)
     int64_t sorted_slots = -1;            // slots right after the last sort
@@ -448,9 +457,13 @@ void deposit_all(Context& ctx);
 void convert_rho(Context& ctx);
 // defer_ledger: 1D push partials stay pending for ledger_work_1d
 void push_all(Context& ctx, double dt, bool fuse_deposit, bool defer_ledger = false);
-// 1D, after the field solve of a step: the survivors' electric work
-// (Simulation.cpp:1094-1131), then every pending ledger folded
+// 1D: the survivors' electric work of a step (Simulation.cpp:1094-1131) is
+// known after its field solve.  The next push adds it while it has the
+// particle and its field; a species whose velocities the collisions change
+// before that is summed here
 void ledger_work_1d(Context& ctx, double dt);
+// books what the steps so far have left pending (before a sort, at the end)
+void ledger_flush_1d(Context& ctx, double dt);
 // live particles of a species, counted on the device
 int64_t live_count(Context& ctx, Species& sp);
 void sort_species(Context& ctx, Species& sp);

@@ -218,6 +218,7 @@ void checkpoint_load(Context& c, const std::string& path) {
             AUR_HIP(hipMemset(sp.ledger.ptr, 0, 3 * sizeof(double)));
         }
         sp.ledger_pending = false;
+        sp.work = Species::kWorkNone;
         sp.slots = slots;
         sp.next_uid = next_uid;
         sp.tiled = false;           // the next sort rebuilds the tile index

@@ -222,8 +222,8 @@ __global__ void __launch_bounds__(kEnsThreads) k_ens_field(EnsArgs a, int solve_
         spectral_solve_1d(a.rho + o, a.phi + o, a.E64 + o, a.E32 + o, a.cs, a.sn, a.nx, a.L, a.eps,
                           sh, &mean_s);
     else
-        dirichlet_solve_1d(a.rho + o, a.phi + o, a.E64 + o, a.E32 + o, a.dp + o, a.nx, a.dx,
-                           a.eps, pv[0], pv[1]);
+        dirichlet_solve_1d(a.rho + o, [&](int i) { return a.rho[o + i]; }, a.phi + o, a.E64 + o,
+                           a.E32 + o, a.dp + o, a.nx, a.dx, a.eps, pv[0], pv[1]);
 }
 
 // MCC on the target species (collide_run): mgroups workgroups per instance,

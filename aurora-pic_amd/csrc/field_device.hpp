@@ -6,6 +6,7 @@
 #pragma once
 
 #include "aurora_internal.hpp"
+#include "push_device.hpp"
 
 namespace aurora {
 
@@ -19,6 +20,14 @@ struct RhoArgs {
     double vol;                // periodic node volume
     int dim;
 };
+
+// Threads of a periodic 1D solve: the direct sums use all there may be; the
+// FFTs of a power of two need a quarter of the mesh, loads and conversions
+// rather a thread per node.
+inline int spectral_1d_threads(int n) {
+    const bool pow2 = n >= 4 && (n & (n - 1)) == 0;
+    return !pow2 ? 1024 : n > 1024 ? n / 4 : 256;
+}
 
 // The context's species accumulators and weights (particles.hip).
 RhoArgs rho_args(const Context& c);
@@ -172,25 +181,48 @@ __device__ __forceinline__ void spectral_sums_1d(double* x, double* pr, double* 
     }
 }
 
-// Radix-2 complex FFT of n = 2^log2n points in LDS (z in bit-reversed
-// order on entry, natural order on exit): sign -1 sums z_j e^(-2 pi i jk/n),
-// sign +1 z_j e^(+2 pi i jk/n), with cos/sin(2 pi m / n) from cs, sn.
+// Complex FFT of n = 2^log2n points in LDS (z in bit-reversed order on entry,
+// natural order on exit): sign -1 sums z_j e^(-2 pi i jk/n), sign +1
+// z_j e^(+2 pi i jk/n), with cos/sin(2 pi m / n) from cs, sn.  Radix-2 stages,
+// two at a time in registers (the first alone when log2n is odd): half the
+// LDS round trips and barriers, which are its time on a small mesh, and the
+// same operations (k_spectral_1d_acc at n = 256: 10.1 -> 8.5 us).
 __device__ __forceinline__ void fft_radix2_1d(double2* z, int n, int log2n, const double* cs,
                                               const double* sn, double sign) {
 #pragma clang fp contract(off)
-    for (int lh = 0; lh < log2n; ++lh) {
-        const int half = 1 << lh;
-        const int tshift = log2n - lh - 1;   // twiddle index stride n / (2 half)
+    auto butterfly = [&](double2& a, double2& c, int m) {
+        const double wr = cs[m], wi = sign * sn[m];
+        const double tr = c.x * wr - c.y * wi;
+        const double ti = c.x * wi + c.y * wr;
+        c = make_double2(a.x - tr, a.y - ti);
+        a = make_double2(a.x + tr, a.y + ti);
+    };
+    int lh = 0;
+    if (log2n & 1) {
         for (int b = threadIdx.x; b < n / 2; b += blockDim.x) {
+            double2 a = z[2 * b], c = z[2 * b + 1];
+            butterfly(a, c, 0);
+            z[2 * b] = a;
+            z[2 * b + 1] = c;
+        }
+        __syncthreads();
+        lh = 1;
+    }
+    for (; lh < log2n; lh += 2) {
+        const int half = 1 << lh;
+        const int t1 = log2n - lh - 1;   // twiddle index stride n / (2 half), then half of it
+        for (int b = threadIdx.x; b < n / 4; b += blockDim.x) {
             const int k = b & (half - 1);
-            const int i0 = ((b >> lh) << (lh + 1)) + k, i1 = i0 + half;
-            const int m = k << tshift;
-            const double wr = cs[m], wi = sign * sn[m];
-            const double2 a = z[i0], c = z[i1];
-            const double tr = c.x * wr - c.y * wi;
-            const double ti = c.x * wi + c.y * wr;
-            z[i0] = make_double2(a.x + tr, a.y + ti);
-            z[i1] = make_double2(a.x - tr, a.y - ti);
+            const int i = ((b >> lh) << (lh + 2)) + k;
+            double2 z0 = z[i], z1 = z[i + half], z2 = z[i + 2 * half], z3 = z[i + 3 * half];
+            butterfly(z0, z1, k << t1);
+            butterfly(z2, z3, k << t1);
+            butterfly(z0, z2, k << (t1 - 1));
+            butterfly(z1, z3, (k + half) << (t1 - 1));
+            z[i] = z0;
+            z[i + half] = z1;
+            z[i + 2 * half] = z2;
+            z[i + 3 * half] = z3;
         }
         __syncthreads();
     }
@@ -261,10 +293,11 @@ __device__ inline void spectral_solve_1d(const double* rho, double* phi, double*
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {   // one wave: the order depends on n alone
         double m = 0.0;
-        for (int j = 0; j < n; ++j) m += x[j];
-        *mean_s = m / static_cast<double>(n);
+        for (int j = threadIdx.x; j < n; j += 64) m += x[j];
+        m = wave_sum(m);
+        if (threadIdx.x == 0) *mean_s = m / static_cast<double>(n);
     }
     __syncthreads();
     const double mean = *mean_s;
@@ -287,23 +320,72 @@ __device__ inline void spectral_solve_1d(const double* rho, double* phi, double*
 }
 
 
-// Exclusive prefix sum over the block of one double per thread (inclusive
-// Hillis-Steele in LDS, a fixed order of additions, then shifted by one);
-// total receives the block's sum.  Every thread of the block calls it.
-__device__ inline double block_exclusive_scan_f64(double x, double* sh, double& total) {
-    const int t = threadIdx.x, T = blockDim.x;
-    sh[t] = x;
-    __syncthreads();
-    for (int d = 1; d < T; d <<= 1) {
-        const double y = t >= d ? sh[t - d] : 0.0;
-        __syncthreads();
-        sh[t] = sh[t] + y;
-        __syncthreads();
+// A species' 1D ledger partials folded into its totals: per push block left
+// and right wall energy, electric work up to a crossing, and the survivors'
+// work of the step before; or that work in partials of its own.  Wave 0 of the
+// block folds them in a fixed order, the earlier step's work first, so the
+// totals do not depend on where a call's steps end.  Any block size.
+struct LedgerFold {
+    const double* push_part;   // null: no push to fold
+    int push_blocks;
+    int work_in_push;
+    const double* work_part;   // null: none
+    int work_blocks;
+    double* ledger;
+};
+struct LedgerFolds {
+    LedgerFold f[kMaxChannels];
+    int n;
+};
+
+// the pending ledger partials of every 1D species, for the step's field solve
+// to fold (particles.hip)
+LedgerFolds take_ledger_folds(Context& c);
+
+__device__ __forceinline__ void fold_ledger(const LedgerFold& f) {
+    if (threadIdx.x >= 64) return;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int b = threadIdx.x; b < f.push_blocks; b += 64) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] += f.push_part[4 * b + k];
     }
-    total = sh[T - 1];
-    const double ex = t > 0 ? sh[t - 1] : 0.0;
+    if (!f.work_in_push) v[3] = 0.0;
+    for (int b = threadIdx.x; b < f.work_blocks; b += 64) v[3] += f.work_part[b];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = wave_sum(v[k]);
+    if (threadIdx.x == 0) {
+        f.ledger[0] += v[0];
+        f.ledger[1] += v[1];
+        const double before = f.ledger[2] + v[3];
+        f.ledger[2] = before + v[2];
+    }
+}
+
+// Exclusive prefix sum over the block of one double per thread: the wave's
+// inclusive sums by shuffles, the wave totals through LDS (wsum: a double per
+// wave), a fixed order of additions; total receives the block's sum.  Every
+// thread of the block calls it.
+__device__ inline double block_exclusive_scan_f64(double x, double* wsum, double& total) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    double incl = x;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const double y = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += y;
+    }
+    double ex = __shfl_up(incl, 1, 64);
+    if (lane == 0) ex = 0.0;
+    if (lane == 63) wsum[wid] = incl;
     __syncthreads();
-    return ex;
+    double before = 0.0;
+    total = 0.0;
+    const int waves = static_cast<int>(blockDim.x) >> 6;
+    for (int w = 0; w < waves; ++w) {
+        if (w == wid) before = total;
+        total += wsum[w];
+    }
+    __syncthreads();
+    return before + ex;
 }
 
 // 1D Dirichlet solve of -phi'' = rho / eps with phi(0) = phi_left and
@@ -317,35 +399,43 @@ __device__ inline double block_exclusive_scan_f64(double x, double* sh, double& 
 // reference's difference of phi (central inside, one-sided at the
 // electrodes), formed from s: -(s_i + s_{i-1}) / 2dx inside.  Each thread
 // owns a contiguous run of k; the runs are combined by two block scans, so
-// the sums are formed in one fixed order.  s: n - 1 doubles of global
-// scratch.  Any block size up to 1024 threads.
-__device__ inline void dirichlet_solve_1d(const double* rho, double* phi, double* E, float* E32,
-                                          double* s, int n, double dx, double eps,
-                                          double phi_left, double phi_right) {
+// the sums are formed in one fixed order.  rho_of(i) gives (and may store)
+// the charge of node i, asked for once.  The b_i and s_k of meshes up to
+// kDirichletLds nodes stay in LDS; larger ones use rho and s (n - 1 doubles)
+// in global memory.  Latency bounds it: 513 nodes 9.6
+// us with rho, b and s in global memory and scans of 18 barriers, 7.7 so.
+// Whole waves, up to 1024 threads.
+constexpr int kDirichletLds = 2048;
+
+template <bool LDS>
+__device__ __forceinline__ void dirichlet_sums_1d(const double* b, double* s, double* phi,
+                                                  double* E, float* E32, int n, double dx,
+                                                  double eps, double phi_left, double phi_right) {
 #pragma clang fp contract(off)
-    __shared__ double scan_sh[1024];
-    __shared__ double s0_sh;
+    __shared__ double wsum[16];
     const int T = blockDim.x, t = threadIdx.x;
     const int N = n - 1;
     const int seg = (N + T - 1) / T;
     const int k0 = t * seg < N ? t * seg : N;
     const int k1 = k0 + seg < N ? k0 + seg : N;
     const double dx2 = dx * dx;
+    auto b_at = [&](int k) {
+        if (k >= n - 2) return 0.0;
+        return LDS ? b[k + 1] : b[k + 1] * dx2 / eps;
+    };
     double loc = 0.0;
-    for (int k = k0; k < k1; ++k) loc += k < n - 2 ? rho[k + 1] * dx2 / eps : 0.0;
+    for (int k = k0; k < k1; ++k) loc += b_at(k);
     double btot = 0.0;
-    double B = block_exclusive_scan_f64(loc, scan_sh, btot);
+    double B = block_exclusive_scan_f64(loc, wsum, btot);
     double locc = 0.0;
     for (int k = k0; k < k1; ++k) {
         s[k] = B;                          // B_k, replaced by s_k below
         locc += B;
-        B += k < n - 2 ? rho[k + 1] * dx2 / eps : 0.0;
+        B += b_at(k);
     }
     double ctot = 0.0;
-    double C = block_exclusive_scan_f64(locc, scan_sh, ctot);
-    if (t == 0) s0_sh = (phi_right - phi_left + ctot) / static_cast<double>(n - 1);
-    __syncthreads();
-    const double s0 = s0_sh;
+    double C = block_exclusive_scan_f64(locc, wsum, ctot);
+    const double s0 = (phi_right - phi_left + ctot) / static_cast<double>(n - 1);
     for (int k = k0; k < k1; ++k) {
         const double Bk = s[k];
         C += Bk;
@@ -364,6 +454,25 @@ __device__ inline void dirichlet_solve_1d(const double* rho, double* phi, double
         else e = -(s[i] + s[i - 1]) / (2.0 * dx);
         E[i] = e;
         E32[i] = static_cast<float>(e);
+    }
+}
+
+template <typename Rho>
+__device__ __forceinline__ void dirichlet_solve_1d(const double* rho, Rho rho_of, double* phi,
+                                                   double* E, float* E32, double* s, int n,
+                                                   double dx, double eps, double phi_left,
+                                                   double phi_right) {
+#pragma clang fp contract(off)
+    __shared__ double b_sh[kDirichletLds], s_sh[kDirichletLds];
+    const double dx2 = dx * dx;
+    if (n <= kDirichletLds) {
+        for (int i = threadIdx.x; i < n; i += blockDim.x) b_sh[i] = rho_of(i) * dx2 / eps;
+        __syncthreads();
+        dirichlet_sums_1d<true>(b_sh, s_sh, phi, E, E32, n, dx, eps, phi_left, phi_right);
+    } else {
+        for (int i = threadIdx.x; i < n; i += blockDim.x) (void)rho_of(i);
+        __syncthreads();
+        dirichlet_sums_1d<false>(rho, s, phi, E, E32, n, dx, eps, phi_left, phi_right);
     }
 }
 

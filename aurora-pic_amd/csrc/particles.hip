@@ -75,7 +75,10 @@ struct PushArgs {
     R dtd0, dtd1, dtd2;    // dt / d per axis
     long long* acc;        // deposit target (fused)
     unsigned long long* absorbed;  // 6 face counters, then pushes outside the tile box
-    double* ledger_part;   // 1D: per block [left energy, right energy, electric work]
+    double* ledger_part;   // 1D: per block [left energy, right energy, electric work of the
+                           // particles that end at a wall, survivors' work of the step before]
+    const long long* work_slots;   // 1D: slots of the push whose survivors' work is due, or null
+    long long* pushed_slots;       // 1D: where this push leaves its slots
     double* vold;          // 1D: synchronised v_x at the start of the step, per slot
     double half_qm, dt64;  // 0.5 * qm and dt in FP64: sync as (0.5 qm E) dt (Pusher.cpp:78-80)
     double half_mw;        // 0.5 * m * w (1D ledgers)
@@ -385,25 +388,39 @@ __global__ void __launch_bounds__(kBlock) k_deposit(SpeciesView<R> sp, MeshView 
 // (a 1D mesh has few nodes, so global atomics would all land on them)
 constexpr int kLds1dNodes = 4096;
 
+// Simulation.cpp:1094-1131: the work 0.5 m w (v^2 - v_old^2) on the particle in
+// slot p since the start of its last step, v_x synchronised with the field at
+// its end.
+template <typename R>
+__device__ __forceinline__ double survivor_work(const PushArgs<R>& a, double vsync, int64_t p) {
+    const double vo = a.vold[p];
+    return a.half_mw * (vsync * vsync - vo * vo);
+}
+
 // Block b of the nb pushing one species (lacc: the block's LDS charge sums
 // on small 1D meshes, else null).
-template <int DIM, typename R, int BMODE, bool DEPOSIT>
+template <int DIM, typename R, int BMODE, bool DEPOSIT, int T>
 __device__ __forceinline__ void push_blocks_of(const PushArgs<R>& a, int b, int nb,
                                                long long* lacc) {
     const SpeciesView<R>& sp = a.sp;
-    double led[3] = {0.0, 0.0, 0.0};   // 1D: left / right wall energy, electric work
+    double led[4] = {0.0, 0.0, 0.0, 0.0};   // 1D: as ledger_part
     constexpr bool kLds = DIM == 1 && DEPOSIT;
     long long* acc = a.acc;
     if constexpr (kLds) {
         if (a.m.nx <= kLds1dNodes) {
-            for (int i = threadIdx.x; i < a.m.nx; i += kBlock) lacc[i] = 0;
+            for (int i = threadIdx.x; i < a.m.nx; i += T) lacc[i] = 0;
             __syncthreads();
             acc = lacc;
         }
     }
     const int64_t nslot = slot_count(sp.slots, sp.nslots);
-    for (int64_t p = b * static_cast<int64_t>(kBlock) + threadIdx.x; p < nslot;
-         p += static_cast<int64_t>(nb) * kBlock) {
+    int64_t due = 0;
+    if constexpr (DIM == 1) {
+        if (a.work_slots) due = *a.work_slots;
+        if (a.pushed_slots && b == 0 && threadIdx.x == 0) *a.pushed_slots = nslot;
+    }
+    for (int64_t p = b * static_cast<int64_t>(T) + threadIdx.x; p < nslot;
+         p += static_cast<int64_t>(nb) * T) {
         const int c = sp.cell[p];
         if (c < 0) continue;
         int idx[3] = {0, 0, 0};
@@ -417,8 +434,10 @@ __device__ __forceinline__ void push_blocks_of(const PushArgs<R>& a, int b, int 
         // 1D: the time-centred v_x before the kick, the reference's stored
         // Particle::v (Pusher.cpp:78-80), for the electric-work ledger
         double vsync = 0.0;
-        if constexpr (DIM == 1)
+        if constexpr (DIM == 1) {
             vsync = static_cast<double>(v[0]) + a.half_qm * static_cast<double>(E[0]) * a.dt64;
+            if (p < due) led[3] += survivor_work(a, vsync, p);
+        }
         if constexpr (BMODE == 0) {
             // leapfrog kick on the mesh axes (Pusher.cpp:70-72, 126-129, 162-166)
 #pragma unroll
@@ -474,25 +493,39 @@ __device__ __forceinline__ void push_blocks_of(const PushArgs<R>& a, int b, int 
         if (acc != a.acc) {
             // the block's integer sums into the species accumulator
             __syncthreads();
-            for (int i = threadIdx.x; i < a.m.nx; i += kBlock)
+            for (int i = threadIdx.x; i < a.m.nx; i += T)
                 if (acc[i] != 0)
                     atomicAdd(reinterpret_cast<unsigned long long*>(a.acc + i),
                               static_cast<unsigned long long>(acc[i]));
         }
     }
     if constexpr (DIM == 1) {
-        const double s = block_sum<3, kBlock>(led);
-        if (threadIdx.x < 3) a.ledger_part[3 * b + threadIdx.x] = s;
+        const double s = block_sum<4, T>(led);
+        if (threadIdx.x < 4) a.ledger_part[4 * b + threadIdx.x] = s;
     }
 }
 
+// Threads of a push workgroup.  A 1D push with its deposit ends with every
+// workgroup's charge sums added to the same few nodes, so it has few
+// workgroups (push_blocks), of more waves each.  Pair push + k_work_1d of the
+// electrons, 513 nodes, 5e5 + 5e5 particles, by threads x workgroups per CU and
+// species: 512 x 1 19.6 + 5.5 us, 512 x 3/4 18.5 + 6.0, 512 x 1/2 19.2 + 7.5,
+// 1024 x 1 21.8 + 4.7, 1024 x 1/2 17.4 + 6.1, 1024 x 1/4 21.5 + 9.0 (256 x 1,
+// the work of both species by itself: 21.1 + 8.1); 16,000 FP64 particles on 256
+// nodes: 4.3 us with 512, 5.5 with 1024.
+template <int DIM, bool DEPOSIT>
+constexpr int push_threads() {
+    return DIM == 1 && DEPOSIT ? 512 : kBlock;
+}
+
 template <int DIM, typename R, int BMODE, bool DEPOSIT>
-__global__ void __launch_bounds__(kBlock) k_push(PushArgs<R> a) {
+__global__ void __launch_bounds__((push_threads<DIM, DEPOSIT>())) k_push(PushArgs<R> a) {
+    constexpr int T = push_threads<DIM, DEPOSIT>();
     if constexpr (DIM == 1 && DEPOSIT) {
         __shared__ long long lacc[kLds1dNodes];
-        push_blocks_of<DIM, R, BMODE, DEPOSIT>(a, blockIdx.x, gridDim.x, lacc);
+        push_blocks_of<DIM, R, BMODE, DEPOSIT, T>(a, blockIdx.x, gridDim.x, lacc);
     } else {
-        push_blocks_of<DIM, R, BMODE, DEPOSIT>(a, blockIdx.x, gridDim.x, nullptr);
+        push_blocks_of<DIM, R, BMODE, DEPOSIT, T>(a, blockIdx.x, gridDim.x, nullptr);
     }
 }
 
@@ -500,87 +533,51 @@ __global__ void __launch_bounds__(kBlock) k_push(PushArgs<R> a) {
 // launch: blocks [0, split) the first, the rest the second, each species'
 // blocks exactly those of its own k_push launch.
 template <typename R, int BMODE>
-__global__ void __launch_bounds__(kBlock) k_push_pair_1d(PushArgs<R> a0, PushArgs<R> a1,
-                                                         int split) {
+__global__ void __launch_bounds__((push_threads<1, true>()))
+    k_push_pair_1d(PushArgs<R> a0, PushArgs<R> a1, int split) {
+    constexpr int T = push_threads<1, true>();
     __shared__ long long lacc[kLds1dNodes];
     if (static_cast<int>(blockIdx.x) < split)
-        push_blocks_of<1, R, BMODE, true>(a0, blockIdx.x, split, lacc);
+        push_blocks_of<1, R, BMODE, true, T>(a0, blockIdx.x, split, lacc);
     else
-        push_blocks_of<1, R, BMODE, true>(a1, blockIdx.x - split, gridDim.x - split, lacc);
+        push_blocks_of<1, R, BMODE, true, T>(a1, blockIdx.x - split, gridDim.x - split, lacc);
 }
 
-
-// 1D survivors after the field solve at t+dt (Simulation.cpp:1094-1131):
-// v_x synchronised with E^{n+1}, and the work 0.5 m w (v^2 - v_old^2)
-// since the start of the step.  Block b of nb sums its particles into
-// part[b].
+// The survivors' work by itself: the sums the next push would leave in column
+// 3 of its partials (its blocks and threads), block b's at part[b].  Blocks
+// [0, split) one species, the rest another of the same precision.
 template <typename R>
-__device__ __forceinline__ void work_1d_blocks(const PushArgs<R>& a, double* part, int b,
-                                               int nb) {
+__device__ __forceinline__ void work_1d_blocks(const PushArgs<R>& a, double* part, int b, int nb) {
+    constexpr int T = push_threads<1, true>();
     const SpeciesView<R>& sp = a.sp;
     double w[1] = {0.0};
-    const int64_t nslot = slot_count(sp.slots, sp.nslots);
-    for (int64_t p = b * static_cast<int64_t>(kBlock) + threadIdx.x; p < nslot;
-         p += static_cast<int64_t>(nb) * kBlock) {
+    const int64_t due = *a.work_slots;
+    for (int64_t p = b * static_cast<int64_t>(T) + threadIdx.x; p < due;
+         p += static_cast<int64_t>(nb) * T) {
         const int c = sp.cell[p];
         if (c < 0) continue;
         int idx[3] = {c, 0, 0};
         R off[3] = {sp.off0[p], R(0), R(0)};
         R E[3] = {R(0), R(0), R(0)};
         gather<1, R>(a, idx, off, E);
-        const double vn =
+        const double vsync =
             static_cast<double>(sp.v0[p]) + a.half_qm * static_cast<double>(E[0]) * a.dt64;
-        const double vo = a.vold[p];
-        w[0] += a.half_mw * (vn * vn - vo * vo);
+        w[0] += survivor_work(a, vsync, p);
     }
-    const double s = block_sum<1, kBlock>(w);
+    const double s = block_sum<1, T>(w);
     if (threadIdx.x == 0) part[b] = s;
 }
 
 template <typename R>
-__global__ void __launch_bounds__(kBlock) k_work_1d(PushArgs<R> a, double* part) {
-    work_1d_blocks(a, part, blockIdx.x, gridDim.x);
-}
-
-// Two species of one precision in one launch: blocks [0, split) the first,
-// the rest the second (each species' partials as in k_work_1d).
-template <typename R>
-__global__ void __launch_bounds__(kBlock) k_work_1d_pair(PushArgs<R> a0, double* part0,
-                                                         PushArgs<R> a1, double* part1,
-                                                         int split) {
+__global__ void __launch_bounds__((push_threads<1, true>()))
+    k_work_1d(PushArgs<R> a0, double* part0, PushArgs<R> a1, double* part1, int split) {
     if (static_cast<int>(blockIdx.x) < split)
         work_1d_blocks(a0, part0, blockIdx.x, split);
     else
         work_1d_blocks(a1, part1, blockIdx.x - split, gridDim.x - split);
 }
 
-// A species' ledger partials, folded in block order into its totals: push
-// partials (3 per block) and, when present, work partials (1 per block).
-struct LedgerFold {
-    const double* push_part;
-    int push_blocks;
-    const double* work_part;
-    int work_blocks;
-    double* ledger;
-};
-
-__device__ __forceinline__ void fold_ledger(const LedgerFold& f) {
-    double v[3] = {0.0, 0.0, 0.0};
-    for (int b = threadIdx.x; b < f.push_blocks; b += kBlock) {
-        v[0] += f.push_part[3 * b];
-        v[1] += f.push_part[3 * b + 1];
-        v[2] += f.push_part[3 * b + 2];
-    }
-    if (f.work_part)
-        for (int b = threadIdx.x; b < f.work_blocks; b += kBlock) v[2] += f.work_part[b];
-    const double s = block_sum<3, kBlock>(v);
-    if (threadIdx.x < 3) f.ledger[threadIdx.x] += s;
-}
-
-// one workgroup per species: block 0 folds f0, block 1 (when launched) f1
-__global__ void __launch_bounds__(kBlock) k_ledger_1d(LedgerFold f0, LedgerFold f1) {
-    fold_ledger(blockIdx.x == 0 ? f0 : f1);
-}
+__global__ void __launch_bounds__(64) k_ledger_1d(LedgerFold f) { fold_ledger(f); }
 
 // one atomic per workgroup (a few per CU): per-wave atomics on one address
 // serialise
@@ -778,6 +775,8 @@ PushArgs<R> push_args(Context& c, Species& sp, double dt) {
     a.acc = reinterpret_cast<long long*>(sp.acc.ptr);
     a.absorbed = sp.absorbed.ptr;
     a.ledger_part = sp.ledger_part.ptr;
+    a.work_slots = sp.work == Species::kWorkDue ? sp.pushed_slots.ptr + sp.pushed_turn : nullptr;
+    a.pushed_slots = sp.pushed_slots.ptr ? sp.pushed_slots.ptr + (sp.pushed_turn ^ 1) : nullptr;
     a.vold = sp.vold.ptr;
     a.half_qm = 0.5 * qm;
     a.dt64 = dt;
@@ -1318,12 +1317,14 @@ bool launch_tile(Context& c, Species& sp, double dt) {
 
 // Workgroups of a push launch: 1D deposits flush one LDS copy of the mesh
 // per workgroup with global atomics on the same few nodes, so their
-// launches are capped at one workgroup per CU (measured on 513 nodes and
-// 5e5 + 5e5 particles: 21.5 us per pair push against 25.7 with two per CU
-// and 24.2 with one per two CUs).
+// launches are capped at three workgroups per four CUs (push_threads has the
+// figures).
 int push_blocks(const Context& c, int64_t slots, bool deposit) {
     const int g = launch_blocks(c, slots);
-    if (c.dim == 1 && deposit && c.n[0] <= kLds1dNodes) return std::min(g, c.cu_count);
+    if (c.dim == 1 && deposit && c.n[0] <= kLds1dNodes) {
+        constexpr int T = push_threads<1, true>();
+        return static_cast<int>(std::clamp<int64_t>((slots + T - 1) / T, 1, c.cu_count * 3 / 4));
+    }
     return g;
 }
 
@@ -1333,7 +1334,7 @@ void launch_push_b(Context& c, Species& sp, double dt, bool deposit) {
     const int g = push_blocks(c, slot_bound(c, sp), deposit);
     if (deposit) {
         KernelScope ks(c, "push_deposit");
-        k_push<DIM, R, BMODE, true><<<g, kBlock, 0, c.stream>>>(a);
+        k_push<DIM, R, BMODE, true><<<g, push_threads<DIM, true>(), 0, c.stream>>>(a);
     } else {
         KernelScope ks(c, "push");
         k_push<DIM, R, BMODE, false><<<g, kBlock, 0, c.stream>>>(a);
@@ -1346,8 +1347,8 @@ void launch_push_pair_1d_b(Context& c, Species& s0, Species& s1, double dt) {
     const int g0 = push_blocks(c, slot_bound(c, s0), true);
     const int g1 = push_blocks(c, slot_bound(c, s1), true);
     KernelScope ks(c, "push_deposit");
-    k_push_pair_1d<R, BMODE><<<g0 + g1, kBlock, 0, c.stream>>>(push_args<R>(c, s0, dt),
-                                                               push_args<R>(c, s1, dt), g0);
+    k_push_pair_1d<R, BMODE><<<g0 + g1, push_threads<1, true>(), 0, c.stream>>>(
+        push_args<R>(c, s0, dt), push_args<R>(c, s1, dt), g0);
     AUR_HIP(hipGetLastError());
 }
 
@@ -1524,69 +1525,112 @@ void ensure_ledger_1d(Context& c, Species& sp) {
         AUR_HIP(hipMemset(sp.ledger.ptr, 0, 3 * sizeof(double)));
     }
     if (!sp.ledger_part.ptr)
-        sp.ledger_part.alloc(static_cast<size_t>(4 * static_cast<int64_t>(c.cu_count) * 32));
+        sp.ledger_part.alloc(static_cast<size_t>(5 * static_cast<int64_t>(c.cu_count) * 32));
     if (!sp.vold.ptr) sp.vold.alloc(static_cast<size_t>(sp.capacity > 0 ? sp.capacity : 1));
+    if (!sp.pushed_slots.ptr) sp.pushed_slots.alloc(2);
 }
 
-LedgerFold ledger_fold(Species& sp, const double* work_part, int work_blocks) {
-    return LedgerFold{sp.ledger_part.ptr, sp.ledger_push_blocks, work_part, work_blocks,
-                      sp.ledger.ptr};
+double* work_partials(const Context& c, Species& sp) {
+    return sp.ledger_part.ptr + 4 * static_cast<int64_t>(c.cu_count) * 32;
 }
 
-void fold_ledger_1d(Context& c, Species& sp, const double* work_part, int work_blocks) {
+// what of the species' ledger is pending: the last push's partials, and the
+// survivors' work of the step before that (or of the last, once summed)
+LedgerFold take_ledger(Context& c, Species& sp) {
+    LedgerFold f{};
+    f.ledger = sp.ledger.ptr;
+    if (sp.ledger_pending) {
+        f.push_part = sp.ledger_part.ptr;
+        f.push_blocks = sp.ledger_push_blocks;
+        f.work_in_push = sp.work_in_push ? 1 : 0;
+        sp.ledger_pending = false;
+        sp.work_in_push = false;
+    }
+    if (sp.work == Species::kWorkSummed) {
+        f.work_part = work_partials(c, sp);
+        f.work_blocks = sp.work_blocks;
+        sp.work = Species::kWorkNone;
+    }
+    return f;
+}
+
+void fold_ledger_1d(Context& c, Species& sp) {
     KernelScope ks(c, "ledger");
-    const LedgerFold f = ledger_fold(sp, work_part, work_blocks);
-    k_ledger_1d<<<1, kBlock, 0, c.stream>>>(f, f);
+    k_ledger_1d<<<1, 64, 0, c.stream>>>(take_ledger(c, sp));
     AUR_HIP(hipGetLastError());
-    sp.ledger_pending = false;
+}
+
+// the survivors' work of one species, or of two of one precision
+void sum_work_1d(Context& c, Species& s0, Species* s1, double dt) {
+    KernelScope ks(c, "work");
+    const int g0 = s0.work_blocks, g = g0 + (s1 ? s1->work_blocks : 0);
+    auto launch = [&]<typename R>() {
+        const auto a0 = push_args<R>(c, s0, dt);
+        k_work_1d<R><<<g, push_threads<1, true>(), 0, c.stream>>>(
+            a0, work_partials(c, s0), s1 ? push_args<R>(c, *s1, dt) : a0,
+            s1 ? work_partials(c, *s1) : nullptr, g0);
+    };
+    if (s0.precision == 64) launch.template operator()<double>();
+    else launch.template operator()<float>();
+    AUR_HIP(hipGetLastError());
+    s0.work = Species::kWorkSummed;
+    if (s1) s1->work = Species::kWorkSummed;
+}
+
+// that of the species chosen, two to a launch where they agree
+template <typename F>
+void sum_due_work_1d(Context& c, double dt, F chosen) {
+    Species* first = nullptr;
+    for (auto& sp : c.species) {
+        if (sp.work != Species::kWorkDue || !chosen(sp)) continue;
+        if (!first) {
+            first = &sp;
+        } else if (first->precision == sp.precision) {
+            sum_work_1d(c, *first, &sp, dt);
+            first = nullptr;
+        } else {
+            sum_work_1d(c, sp, nullptr, dt);
+        }
+    }
+    if (first) sum_work_1d(c, *first, nullptr, dt);
+}
+
+// a species' 1D push has been queued with its deposit, or alone
+void pushed_1d(Context& c, Species& sp, bool deposit) {
+    sp.ledger_push_blocks = push_blocks(c, slot_bound(c, sp), deposit);
+    sp.ledger_pending = true;
+    sp.work_in_push = sp.work == Species::kWorkDue;
+    if (sp.work == Species::kWorkDue) sp.work = Species::kWorkNone;
+    sp.pushed_turn ^= 1;
 }
 
 }  // namespace
 
-void ledger_work_1d(Context& c, double dt) {
-    if (c.dim != 1) return;
-    // the usual pair (electrons and ions of one precision): both species'
-    // work in one launch, both folds in another
-    std::vector<Species*> pending;
-    for (auto& sp : c.species)
-        if (sp.ledger_pending) pending.push_back(&sp);
-    if (pending.size() == 2 && pending[0]->precision == pending[1]->precision) {
-        Species& s0 = *pending[0];
-        Species& s1 = *pending[1];
-        const int g0 = launch_blocks(c, slot_bound(c, s0));
-        const int g1 = launch_blocks(c, slot_bound(c, s1));
-        double* part0 = s0.ledger_part.ptr + 3 * static_cast<int64_t>(c.cu_count) * 32;
-        double* part1 = s1.ledger_part.ptr + 3 * static_cast<int64_t>(c.cu_count) * 32;
-        auto launch = [&]<typename R>() {
-            KernelScope ks(c, "work");
-            k_work_1d_pair<R><<<g0 + g1, kBlock, 0, c.stream>>>(
-                push_args<R>(c, s0, dt), part0, push_args<R>(c, s1, dt), part1, g0);
-            AUR_HIP(hipGetLastError());
-        };
-        if (s0.precision == 64) launch.template operator()<double>();
-        else launch.template operator()<float>();
-        KernelScope ks(c, "ledger");
-        k_ledger_1d<<<2, kBlock, 0, c.stream>>>(ledger_fold(s0, part0, g0),
-                                                ledger_fold(s1, part1, g1));
-        AUR_HIP(hipGetLastError());
-        s0.ledger_pending = false;
-        s1.ledger_pending = false;
-        return;
-    }
+LedgerFolds take_ledger_folds(Context& c) {
+    LedgerFolds f{};
     for (auto& sp : c.species) {
-        if (!sp.ledger_pending) continue;
-        const int g = launch_blocks(c, slot_bound(c, sp));
-        double* part = sp.ledger_part.ptr + 3 * static_cast<int64_t>(c.cu_count) * 32;
-        dispatch_dim_prec(c, sp, [&]<int DIM, typename R>() {
-            if constexpr (DIM == 1) {
-                auto a = push_args<R>(c, sp, dt);
-                KernelScope ks(c, "work");
-                k_work_1d<R><<<g, kBlock, 0, c.stream>>>(a, part);
-                AUR_HIP(hipGetLastError());
-            }
-        });
-        fold_ledger_1d(c, sp, part, g);
+        if (!sp.ledger_pending || f.n == kMaxChannels) continue;
+        f.f[f.n++] = take_ledger(c, sp);
+        // the survivors' work of this step, from the solve's field on
+        sp.work = Species::kWorkDue;
+        sp.work_blocks = sp.ledger_push_blocks;
     }
+    return f;
+}
+
+void ledger_work_1d(Context& c, double dt) {
+    if (!c.mcc.loaded) return;
+    sum_due_work_1d(c, dt, [&](const Species& sp) {
+        for (int k = 0; k < c.mcc_models(); ++k)
+            if (&c.species[c.mcc_model(k).target] == &sp) return true;
+        return false;
+    });
+}
+
+void ledger_flush_1d(Context& c, double dt) {
+    sum_due_work_1d(c, dt, [](const Species&) { return true; });
+    for (auto& sp : c.species)
+        if (sp.work == Species::kWorkSummed) fold_ledger_1d(c, sp);
 }
 
 int64_t live_count(Context& c, Species& sp) {
@@ -1624,14 +1668,13 @@ void push_all(Context& c, double dt, bool fuse_deposit, bool defer_ledger) {
         Species& s1 = c.species[1];
         for (Species* sp : {&s0, &s1}) {
             ensure_ledger_1d(c, *sp);
-            if (sp->ledger_pending) fold_ledger_1d(c, *sp, nullptr, 0);
+            if (sp->ledger_pending) fold_ledger_1d(c, *sp);
         }
         if (s0.precision == 64) launch_push_pair_1d<double>(c, s0, s1, dt);
         else launch_push_pair_1d<float>(c, s0, s1, dt);
         for (Species* sp : {&s0, &s1}) {
-            sp->ledger_push_blocks = push_blocks(c, slot_bound(c, *sp), true);
-            sp->ledger_pending = true;
-            if (!defer_ledger) fold_ledger_1d(c, *sp, nullptr, 0);
+            pushed_1d(c, *sp, true);
+            if (!defer_ledger) fold_ledger_1d(c, *sp);
         }
         return;
     }
@@ -1640,7 +1683,7 @@ void push_all(Context& c, double dt, bool fuse_deposit, bool defer_ledger) {
         if (c.dim == 1) {
             ensure_ledger_1d(c, sp);
             // a push whose partials were never folded (push without a step)
-            if (sp.ledger_pending) fold_ledger_1d(c, sp, nullptr, 0);
+            if (sp.ledger_pending) fold_ledger_1d(c, sp);
         }
         if (fuse_deposit && sp.tiled && c.tiled_push_ok() &&
             sp.slots < (int64_t{1} << 32) / static_cast<int64_t>(sp.elem())) {
@@ -1660,9 +1703,8 @@ void push_all(Context& c, double dt, bool fuse_deposit, bool defer_ledger) {
             launch_push<DIM, R>(c, sp, dt, fuse_deposit);
         });
         if (c.dim == 1) {
-            sp.ledger_push_blocks = push_blocks(c, slot_bound(c, sp), fuse_deposit);
-            sp.ledger_pending = true;
-            if (!defer_ledger) fold_ledger_1d(c, sp, nullptr, 0);
+            pushed_1d(c, sp, fuse_deposit);
+            if (!defer_ledger) fold_ledger_1d(c, sp);
         }
     }
 }

@@ -875,3 +875,38 @@ def test_tiled_push_undivided_mesh_and_precisions(n, shape, precision, bfield):
             out.append((c.charge_fixed(sid), p_[o], v_[o]))
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+# Runs of one node and less per thread, one and several waves, the last mesh
+# kept in LDS and the first that is not.
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [3, 64, 65, 256, 257, 258, 2048, 2049])
+def test_dirichlet_solve_at_the_edges_of_its_paths(hip_ctx, n):
+    print(f"n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    L, eps = 0.067, 8.8541878128e-12
+    rho = rng.normal(0.0, 1e-6, n)
+    hip_ctx.mesh([n], [L], 1, eps)
+    hip_ctx.set_rho(rho)
+    hip_ctx.solve(-20.0, 173.0, True)
+    _, phi, E = hip_ctx.fields()
+    ref_phi, ref_E = _dirichlet_long_double(rho, L / (n - 1), eps, -20.0, 173.0)
+    assert np.max(np.abs(phi - ref_phi)) <= 1e-12 * float(np.max(np.abs(ref_phi)))
+    assert np.max(np.abs(E[0] - ref_E)) <= 1e-12 * float(np.max(np.abs(ref_E)))
+
+
+# FFTs of an odd and an even number of radix-2 stages, fewer butterflies than
+# a wave and more than four waves have threads.
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [8, 16, 32, 128, 512, 2048])
+def test_spectral_1d_solve_stage_counts(hip_ctx, n):
+    print(f"n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    rho = rng.normal(size=n)
+    hip_ctx.mesh([n], [2.7], 0, 1.3)
+    hip_ctx.set_rho(rho)
+    hip_ctx.solve(0.0, 0.0, True)
+    _, phi, E = hip_ctx.fields()
+    phi_ref, E_ref = _spectral_reference(rho, [n], [2.7], 1.3)
+    assert np.max(np.abs(phi - phi_ref)) <= 1e-11 * np.max(np.abs(phi_ref))
+    assert np.max(np.abs(E[0] - E_ref[0])) <= 1e-11 * np.max(np.abs(E_ref))

@@ -145,3 +145,45 @@ def test_ledgers_are_run_to_run_identical_and_restart_exact(tmp_path):
     d.step(dt, 150)
     _same(runs[0], _tallies(d, dsids))
     d.close()
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+@pytest.mark.parametrize("walls", [False, True])
+@pytest.mark.parametrize("count", [1, 700, 120000])
+def test_ledgers_do_not_depend_on_where_a_call_ends(precision, walls, count):
+    # a step's survivors' work is summed by the next push, or by the end of the
+    # call: the same numbers, in calls of one step, of several and of all, with
+    # one species and with a pair, with fewer particles than threads and with more
+    from aurora_pic import hip
+    rng = np.random.default_rng(count)
+    L, eps = 0.03, 8.8541878128e-12
+    n = 65 if walls else 64
+    pos = rng.uniform(0.0, L, size=count)
+    vel = rng.normal(0.0, 6e5, size=(count, 3))
+    runs = []
+    for calls in ([12], [1] * 12, [5, 7]):
+        out = []
+        for species in (1, 2):
+            c = hip.Context(0)
+            c.mesh([n], [L], 1 if walls else 0, eps)
+            if walls:
+                c.electrodes((0.0, 250.0, 13.56e6, 0.0), (0.0, 0.0, 0.0, 0.0))
+            sids = [c.add_species(-workloads.EV, workloads.ME, 1e9 / count, count,
+                                  precision=precision)]
+            c.upload(sids[0], pos, vel)
+            if species == 2:
+                sids.append(c.add_species(workloads.EV, 6.67e-27, 1e9 / count, count,
+                                          precision=precision))
+                c.upload(sids[1], pos[::-1].copy(), 1e-3 * vel)
+            c.initialize(2e-10)
+            for k in calls:
+                c.step(2e-10, k)
+            for s in sids:
+                out.append(c.power_transfer(s))
+                if walls:
+                    out.append(tuple(np.asarray(x) for x in c.losses(s)))
+            c.close()
+        runs.append(out)
+    assert runs[0][0] != 0.0 or count == 1
+    _same(runs[0], runs[1])
+    _same(runs[0], runs[2])
