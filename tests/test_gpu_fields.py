@@ -910,3 +910,47 @@ def test_spectral_1d_solve_stage_counts(hip_ctx, n):
     phi_ref, E_ref = _spectral_reference(rho, [n], [2.7], 1.3)
     assert np.max(np.abs(phi - phi_ref)) <= 1e-11 * np.max(np.abs(phi_ref))
     assert np.max(np.abs(E[0] - E_ref[0])) <= 1e-11 * np.max(np.abs(E_ref))
+
+
+# Fewer nodes and particles than a workgroup's threads, one more than it, and
+# enough for every workgroup of the sums; half volumes at electrodes.
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [32, 64])
+@pytest.mark.parametrize("n,bc", [([3], 1), ([257], 1), ([64], 0), ([5, 7], 0), ([300, 257], 0),
+                                  ([3, 4, 5], 0), ([70, 65, 130], 0)])
+def test_energy_sums(hip_ctx, n, bc, precision):
+    # FP64 sums of positive terms in any order: within terms x 2^-53 relative of
+    # the exact sum, 1e-12 for the 6e5 nodes and fewer here
+    print(f"n={n}", flush=True)
+    rng = np.random.default_rng(sum(n))
+    L = [0.01 * (k + 1) for k in range(len(n))]
+    eps, m, w, dt = 1.3, 2.5, 3.0, 1e-9
+    hip_ctx.mesh(n, L, bc, eps)
+    counts = (1, 40000)
+    vel = []
+    for count in counts:
+        s = hip_ctx.add_species(0.0, m, w, count, precision=precision)   # no field acts on them
+        pos = rng.uniform(0.05, 0.95, size=(count, len(n))) * np.array(L)
+        v = rng.normal(0.0, 10.0, size=(count, 3)).astype(np.float32).astype(np.float64)
+        hip_ctx.upload(s, pos[:, 0] if len(n) == 1 else pos, v)
+        vel.append(v)
+    hip_ctx.set_rho(rng.normal(size=int(np.prod(n))))
+    hip_ctx.solve(-1.0, 2.0, True)
+    ke, fe, l1, live = hip_ctx.energy(dt)
+    rho, phi, E = hip_ctx.fields()
+    vol = np.ones(n[::-1])
+    for a, k in enumerate(n):
+        d = L[a] / (k if bc == 0 else k - 1)
+        wa = np.full(k, d)
+        if bc == 1:
+            wa[[0, -1]] *= 0.5
+        vol = vol * wa.reshape([-1 if b == a else 1 for b in range(len(n))][::-1])
+    vol = vol.ravel()
+    want_fe = math.fsum(0.5 * eps * np.sum(E ** 2, axis=0) * vol)
+    want_l1 = math.fsum(np.abs(rho) * vol)
+    assert abs(fe - want_fe) <= 1e-12 * want_fe
+    assert abs(l1 - want_l1) <= 1e-12 * want_l1
+    for k, v in zip(ke, vel):
+        want = math.fsum(0.5 * m * w * np.sum(v ** 2, axis=1))
+        assert abs(k - want) <= 1e-12 * want
+    assert live == sum(counts)
