@@ -398,13 +398,36 @@ struct RequestState {
     int64_t chunks = 0;
     int64_t steps_done = 0;
     uint64_t footprint = 0;
-    DevBuf<float> v;                       // 3 x particles (SoA)
-    DevBuf<float> dx;                      // 3 x particles displacement (SoA)
-    DevBuf<double> moments;                // chunks x 5
-    DevBuf<long long> part;
-    DevBuf<unsigned long long> counts;
-    DevBuf<unsigned> maxe;
-    DevBuf<uint32_t> status;
+    // One allocation, laid out by RequestLayout: the sums that start at zero,
+    // then the moments (together the request's result, read back in one copy),
+    // then the electrons.
+    DevBuf<uint8_t> slab;
+    long long* part = nullptr;             // chunks x blocks x 2
+    unsigned long long* counts = nullptr;  // kMaxChannels + 3
+    unsigned* maxe = nullptr;
+    uint32_t* status = nullptr;
+    double* moments = nullptr;             // chunks x 5
+    float* v = nullptr;                    // 3 x particles (SoA)
+    float* dx = nullptr;                   // 3 x particles displacement (SoA)
+};
+
+// byte offsets of a request's arrays in its slab; zeroed: the bytes that start
+// at zero, result: those read back at its end
+struct RequestLayout {
+    size_t counts, maxe, status, zeroed, moments, result, v, dx, bytes;
+    RequestLayout(const aurora_hip_swarm_request& q, int64_t chunks) {
+        const size_t lanes = static_cast<size_t>(3 * q.particles) * sizeof(float);
+        auto aligned = [](size_t b) { return (b + 255) / 256 * 256; };
+        counts = static_cast<size_t>(chunks * q.blocks * 2) * sizeof(long long);   // part at 0
+        maxe = counts + (kMaxChannels + 3) * sizeof(unsigned long long);
+        status = maxe + sizeof(unsigned);
+        zeroed = status + sizeof(uint32_t);
+        moments = (zeroed + 7) / 8 * 8;
+        result = moments + static_cast<size_t>(chunks * 5) * sizeof(double);
+        v = aligned(result);
+        dx = aligned(v + lanes);
+        bytes = dx + lanes;
+    }
 };
 
 // Descriptor and work-item arrays of one launch: pinned host staging and
@@ -437,7 +460,49 @@ struct SwarmState {
     bool in_flight = false;         // a launch has been queued and not collected
     std::vector<int64_t> finishing; // requests whose last steps the launch in flight runs
     int blocks_per_cu = 0;          // resident k_swarm workgroups per CU (occupancy)
+    // Slabs of requests that are done, for the next ones: 64 served requests
+    // spent 5 of 40 ms in allocating and freeing them (and 5 to 10 more while
+    // each request had seven allocations).  Used on the context's stream alone,
+    // after it has drained past the request; at most kSpareBytes, which no
+    // request's budget counts, freed with the context or when an allocation
+    // needs the memory.
+    std::vector<DevBuf<uint8_t>> spare;
+    size_t spare_bytes = 0;
 };
+constexpr size_t kSpareBytes = size_t{256} << 20;
+
+// a slab of at least the bytes: the smallest spare one that has them and not
+// four times them, else a new one
+DevBuf<uint8_t> take_slab(SwarmState& s, size_t bytes) {
+    size_t best = s.spare.size();
+    for (size_t k = 0; k < s.spare.size(); ++k)
+        if (s.spare[k].count >= bytes && s.spare[k].count / 4 <= bytes &&
+            (best == s.spare.size() || s.spare[k].count < s.spare[best].count))
+            best = k;
+    DevBuf<uint8_t> slab;
+    if (best < s.spare.size()) {
+        slab = std::move(s.spare[best]);
+        s.spare.erase(s.spare.begin() + static_cast<std::ptrdiff_t>(best));
+        s.spare_bytes -= slab.count;
+        return slab;
+    }
+    try {
+        slab.alloc(bytes);
+    } catch (const Failure&) {
+        if (s.spare.empty()) throw;
+        (void)hipGetLastError();
+        s.spare.clear();
+        s.spare_bytes = 0;
+        slab.alloc(bytes);
+    }
+    return slab;
+}
+
+void keep_slab(SwarmState& s, DevBuf<uint8_t>&& slab) {
+    if (slab.count > kSpareBytes - s.spare_bytes) return;   // freed by its owner
+    s.spare_bytes += slab.count;
+    s.spare.push_back(std::move(slab));
+}
 
 SwarmState& state(Context& c) {
     if (!c.swarm) c.swarm = new SwarmState();
@@ -485,19 +550,20 @@ void finalize(Context& c, SwarmState& s, int64_t handle, RequestState& r) {
     aurora_hip_swarm_result out{};
     const auto& q = r.req;
     const int64_t B = q.blocks, S = q.steps - q.burn_in, N = q.particles;
-    std::vector<long long> part(static_cast<size_t>(r.chunks * B * 2));
+    const RequestLayout lay(q, r.chunks);
+    std::vector<long long> part(lay.result / sizeof(long long));   // the whole result, part first
+    AUR_HIP(hipMemcpyAsync(part.data(), r.slab.ptr, lay.result, hipMemcpyDeviceToHost,
+                           c.stream));
+    AUR_HIP(hipStreamSynchronize(c.stream));
+    const uint8_t* bytes = reinterpret_cast<const uint8_t*>(part.data());
     unsigned long long counts[kMaxChannels + 3];
     unsigned maxe = 0;
     uint32_t status = 0;
-    AUR_HIP(hipStreamSynchronize(c.stream));
-    AUR_HIP(hipMemcpy(part.data(), r.part.ptr, part.size() * sizeof(long long),
-                      hipMemcpyDeviceToHost));
-    AUR_HIP(hipMemcpy(counts, r.counts.ptr, sizeof counts, hipMemcpyDeviceToHost));
-    AUR_HIP(hipMemcpy(&maxe, r.maxe.ptr, sizeof maxe, hipMemcpyDeviceToHost));
-    AUR_HIP(hipMemcpy(&status, r.status.ptr, sizeof status, hipMemcpyDeviceToHost));
+    std::memcpy(counts, bytes + lay.counts, sizeof counts);
+    std::memcpy(&maxe, bytes + lay.maxe, sizeof maxe);
+    std::memcpy(&status, bytes + lay.status, sizeof status);
     std::vector<double> mom(static_cast<size_t>(r.chunks * 5));
-    AUR_HIP(hipMemcpy(mom.data(), r.moments.ptr, mom.size() * sizeof(double),
-                      hipMemcpyDeviceToHost));
+    std::memcpy(mom.data(), bytes + lay.moments, mom.size() * sizeof(double));
     {
         // Swarm.cpp:1139-1176: variance of the displacement over the
         // sampling window; D_L = var_x / 2T, D_T = var_yz / 4T
@@ -1074,15 +1140,15 @@ void queue_launch(Context& c, SwarmState& s, int64_t max_steps) {
         const int64_t ns = std::min(max_steps, remaining);
         RequestDesc d{};
         const int64_t n = q.particles;
-        d.vx = r.v.ptr;
-        d.vy = r.v.ptr + n;
-        d.vz = r.v.ptr + 2 * n;
-        d.dx = r.dx.ptr;
-        d.moments = r.moments.ptr;
-        d.part = r.part.ptr;
-        d.counts = r.counts.ptr;
-        d.max_energy_bits = r.maxe.ptr;
-        d.status = r.status.ptr;
+        d.vx = r.v;
+        d.vy = r.v + n;
+        d.vz = r.v + 2 * n;
+        d.dx = r.dx;
+        d.moments = r.moments;
+        d.part = r.part;
+        d.counts = r.counts;
+        d.max_energy_bits = r.maxe;
+        d.status = r.status;
         d.particles = n;
         const double efield = q.reduced_field_td * kTownsend * s.gas.neutral_density;
         const double accel = -kElementaryCharge * efield / kElectronMass;
@@ -1171,6 +1237,7 @@ void collect_launch(Context& c, SwarmState& s, bool wait) {
         auto it = s.active.find(handle);
         if (it == s.active.end()) continue;
         finalize(c, s, handle, *it->second);
+        keep_slab(s, std::move(it->second->slab));
         s.active.erase(it);
     }
     s.finishing.clear();
@@ -1254,24 +1321,24 @@ int aurora_hip_swarm_submit(aurora_hip_ctx* h, const aurora_hip_swarm_request* r
         st->req = *r;
         st->chunks = (r->particles + kChunk - 1) / kChunk;
         st->footprint = fp;
-        st->v.alloc(static_cast<size_t>(3 * r->particles));
-        st->dx.alloc(static_cast<size_t>(3 * r->particles));
-        st->moments.alloc(static_cast<size_t>(st->chunks * 5));
-        st->part.alloc(static_cast<size_t>(st->chunks * r->blocks * 2));
-        st->counts.alloc(kMaxChannels + 3);
-        st->maxe.alloc(1);
-        st->status.alloc(1);
-        AUR_HIP(hipMemsetAsync(st->part.ptr, 0, st->part.count * sizeof(long long), c.stream));
-        AUR_HIP(hipMemsetAsync(st->counts.ptr, 0, (kMaxChannels + 3) * 8, c.stream));
-        AUR_HIP(hipMemsetAsync(st->maxe.ptr, 0, 4, c.stream));
-        AUR_HIP(hipMemsetAsync(st->status.ptr, 0, 4, c.stream));
+        const RequestLayout lay(*r, st->chunks);
+        st->slab = take_slab(s, lay.bytes);
+        uint8_t* base = st->slab.ptr;
+        st->part = reinterpret_cast<long long*>(base);
+        st->counts = reinterpret_cast<unsigned long long*>(base + lay.counts);
+        st->maxe = reinterpret_cast<unsigned*>(base + lay.maxe);
+        st->status = reinterpret_cast<uint32_t*>(base + lay.status);
+        st->moments = reinterpret_cast<double*>(base + lay.moments);
+        st->v = reinterpret_cast<float*>(base + lay.v);
+        st->dx = reinterpret_cast<float*>(base + lay.dx);
+        AUR_HIP(hipMemsetAsync(base, 0, lay.zeroed, c.stream));
         const double sigma =
             std::sqrt(2.0 * r->initial_mean_energy_ev * kElementaryCharge / (3.0 * kElectronMass));
         const int64_t n = r->particles;
         int64_t g = (n + 255) / 256;
         if (g > 4096) g = 4096;
         k_swarm_init<<<static_cast<unsigned>(g), 256, 0, c.stream>>>(
-            st->v.ptr, st->v.ptr + n, st->v.ptr + 2 * n, n, static_cast<float>(sigma), r->seed);
+            st->v, st->v + n, st->v + 2 * n, n, static_cast<float>(sigma), r->seed);
         AUR_HIP(hipGetLastError());
         s.bytes_in_use += fp;
         const int64_t id = s.next_handle++;

@@ -211,3 +211,20 @@ def test_reference_swarm_example_csv(ctx, tmp_path):
     check_against_reference([(r.drift, r.mean_energy_ev, r.collisions[0], r.candidates,
                               r.longitudinal_diffusion, r.transverse_diffusion)
                              for r in results])
+
+
+def test_requests_in_used_memory_give_the_same_results(ctx):
+    # requests of rising and falling sizes, one after the other in the memory of
+    # those before them, against a new context for each: the same bytes
+    from aurora_pic import hip
+    gas = workloads.synthetic_gas(rows=64)
+    ctx.swarm_gas(gas)
+    dt = 0.05 / gas["max_frequency"]
+    for particles, blocks in [(1, 2), (5000, 5), (300, 40), (5000, 3), (257, 4), (1, 2)]:
+        req = _request(120.0, particles, 60, 20, blocks, dt, particles)
+        used = _run_all(ctx, [req], 37)[0]
+        fresh = hip.Context(0)
+        fresh.swarm_gas(gas)
+        alone = _run_all(fresh, [req], 37)[0]
+        fresh.close()
+        assert bytes(used) == bytes(alone)
