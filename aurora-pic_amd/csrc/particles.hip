@@ -511,7 +511,7 @@ __device__ __forceinline__ void push_blocks_of(const PushArgs<R>& a, int b, int 
 // electrons, 513 nodes, 5e5 + 5e5 particles, by threads x workgroups per CU and
 // species: 512 x 1 19.6 + 5.5 us, 512 x 3/4 18.5 + 6.0, 512 x 1/2 19.2 + 7.5,
 // 1024 x 1 21.8 + 4.7, 1024 x 1/2 17.4 + 6.1, 1024 x 1/4 21.5 + 9.0 (256 x 1,
-// the work of both species by itself: 21.1 + 8.1); 16,000 FP64 particles on 256
+// the work of both species by itself: 21.1 + 8.1); 25,600 FP64 particles on 256
 // nodes: 4.3 us with 512, 5.5 with 1024.
 template <int DIM, bool DEPOSIT>
 constexpr int push_threads() {

@@ -333,7 +333,7 @@ struct Species3DConfig {          // Species3D.hpp:9-26 (uniform Maxwellian load
     Vec3 drift_velocity{};
     double thermal_velocity{0.1};
     std::size_t capacity{0};      // slots (0 = particles)
-    int precision{32};            // 64 keeps FP64 offsets and velocities (untiled push)
+    int precision{32};            // 64 keeps FP64 offsets and velocities
     double init_x_min{0.0}, init_x_max{-1.0};   // negative maxima mean the full axis
     double init_y_min{0.0}, init_y_max{-1.0};
     double init_z_min{0.0}, init_z_max{-1.0};

@@ -544,7 +544,7 @@ def main():
     ctx.sync()
     kernels = {}
     for name in ["push_deposit", "rho", "fft_fwd_x", "fft_axis", "fft_last", "fft_inv_x",
-                 "green", "fft_load", "fft_unpack", "clear_charge", "sort"]:
+                 "clear_charge", "sort"]:
         ms, n = ctx.kernel_time(name)
         if n:
             kernels[name] = {"avg_ms": ms / n, "launches": n}
