@@ -417,16 +417,15 @@ struct RequestLayout {
     size_t counts, maxe, status, zeroed, moments, result, v, dx, bytes;
     RequestLayout(const aurora_hip_swarm_request& q, int64_t chunks) {
         const size_t lanes = static_cast<size_t>(3 * q.particles) * sizeof(float);
-        auto aligned = [](size_t b) { return (b + 255) / 256 * 256; };
         counts = static_cast<size_t>(chunks * q.blocks * 2) * sizeof(long long);   // part at 0
         maxe = counts + (kMaxChannels + 3) * sizeof(unsigned long long);
         status = maxe + sizeof(unsigned);
         zeroed = status + sizeof(uint32_t);
         moments = (zeroed + 7) / 8 * 8;
         result = moments + static_cast<size_t>(chunks * 5) * sizeof(double);
-        v = aligned(result);
-        dx = aligned(v + lanes);
-        bytes = dx + lanes;
+        v = (result + 63) / 64 * 64;
+        dx = v + lanes;
+        bytes = dx + lanes;   // at most footprint_of(q), which leaves 64 bytes for the alignment
     }
 };
 
@@ -463,20 +462,20 @@ struct SwarmState {
     // Slabs of requests that are done, for the next ones: 64 served requests
     // spent 5 of 40 ms in allocating and freeing them (and 5 to 10 more while
     // each request had seven allocations).  Used on the context's stream alone,
-    // after it has drained past the request; at most kSpareBytes, which no
-    // request's budget counts, freed with the context or when an allocation
-    // needs the memory.
+    // after it has drained past the request; at most kSpareBytes, which a
+    // request's budget covers with the slabs in use (fit_budget), freed with
+    // the context or when a further slab needs the memory.
     std::vector<DevBuf<uint8_t>> spare;
     size_t spare_bytes = 0;
+    bool budgeted = false;          // a request came with an HBM budget
 };
 constexpr size_t kSpareBytes = size_t{256} << 20;
 
-// a slab of at least the bytes: the smallest spare one that has them and not
-// four times them, else a new one
-DevBuf<uint8_t> take_slab(SwarmState& s, size_t bytes) {
+// the smallest spare slab of bytes to most, or none
+DevBuf<uint8_t> take_spare(SwarmState& s, size_t bytes, size_t most) {
     size_t best = s.spare.size();
     for (size_t k = 0; k < s.spare.size(); ++k)
-        if (s.spare[k].count >= bytes && s.spare[k].count / 4 <= bytes &&
+        if (s.spare[k].count >= bytes && s.spare[k].count <= most &&
             (best == s.spare.size() || s.spare[k].count < s.spare[best].count))
             best = k;
     DevBuf<uint8_t> slab;
@@ -484,8 +483,20 @@ DevBuf<uint8_t> take_slab(SwarmState& s, size_t bytes) {
         slab = std::move(s.spare[best]);
         s.spare.erase(s.spare.begin() + static_cast<std::ptrdiff_t>(best));
         s.spare_bytes -= slab.count;
-        return slab;
     }
+    return slab;
+}
+
+// Spare slabs freed, the last kept first, until the budget holds them, the
+// slabs in use and the bytes of one more.
+void fit_budget(SwarmState& s, uint64_t bytes, uint64_t budget) {
+    while (!s.spare.empty() && s.bytes_in_use + bytes + s.spare_bytes > budget) {
+        s.spare_bytes -= s.spare.back().count;
+        s.spare.pop_back();
+    }
+}
+
+void alloc_slab(SwarmState& s, DevBuf<uint8_t>& slab, size_t bytes) {
     try {
         slab.alloc(bytes);
     } catch (const Failure&) {
@@ -495,7 +506,6 @@ DevBuf<uint8_t> take_slab(SwarmState& s, size_t bytes) {
         s.spare_bytes = 0;
         slab.alloc(bytes);
     }
-    return slab;
 }
 
 void keep_slab(SwarmState& s, DevBuf<uint8_t>&& slab) {
@@ -1320,9 +1330,16 @@ int aurora_hip_swarm_submit(aurora_hip_ctx* h, const aurora_hip_swarm_request* r
         auto st = std::make_unique<RequestState>();
         st->req = *r;
         st->chunks = (r->particles + kChunk - 1) / kChunk;
-        st->footprint = fp;
         const RequestLayout lay(*r, st->chunks);
-        st->slab = take_slab(s, lay.bytes);
+        // A request holds its footprint, as its admission counts, so that a
+        // budget has room for every request whose footprint it has room for.
+        // On a context that was never given a budget it may hold up to four
+        // times that in a spare slab, and is booked with what it holds.
+        s.budgeted = s.budgeted || hbm_budget != 0;
+        st->slab = take_spare(s, lay.bytes, s.budgeted ? fp : 4 * fp);
+        st->footprint = std::max<uint64_t>(fp, st->slab.count);
+        if (hbm_budget) fit_budget(s, st->footprint, hbm_budget);
+        if (!st->slab.ptr) alloc_slab(s, st->slab, lay.bytes);
         uint8_t* base = st->slab.ptr;
         st->part = reinterpret_cast<long long*>(base);
         st->counts = reinterpret_cast<unsigned long long*>(base + lay.counts);
@@ -1340,7 +1357,7 @@ int aurora_hip_swarm_submit(aurora_hip_ctx* h, const aurora_hip_swarm_request* r
         k_swarm_init<<<static_cast<unsigned>(g), 256, 0, c.stream>>>(
             st->v, st->v + n, st->v + 2 * n, n, static_cast<float>(sigma), r->seed);
         AUR_HIP(hipGetLastError());
-        s.bytes_in_use += fp;
+        s.bytes_in_use += st->footprint;
         const int64_t id = s.next_handle++;
         s.active[id] = std::move(st);
         if (handle) *handle = id;

@@ -413,7 +413,12 @@ int aurora_hip_swarm_gas(aurora_hip_ctx* ctx, int nchan, const int* kind,
                          double max_frequency, int64_t max_candidates,
                          double neutral_mass, double neutral_temperature);
 /* Admits a request when its device footprint fits the HBM budget
- * (bytes; 0 = no limit); returns AURORA_ERR_CAPACITY otherwise. */
+ * (bytes; 0 = no limit) beside those of the requests that run; returns
+ * AURORA_ERR_CAPACITY otherwise.  Memory of finished requests is kept for
+ * the next ones (at most 256 MiB) and given back where the budget would not
+ * hold it too.  A request submitted before the context's first budget may
+ * run in more memory than its footprint (at most four times), and counts
+ * with that. */
 int aurora_hip_swarm_submit(aurora_hip_ctx* ctx,
                             const aurora_hip_swarm_request* request,
                             uint64_t hbm_budget, int64_t* handle);

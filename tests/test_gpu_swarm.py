@@ -228,3 +228,44 @@ def test_requests_in_used_memory_give_the_same_results(ctx):
         alone = _run_all(fresh, [req], 37)[0]
         fresh.close()
         assert bytes(used) == bytes(alone)
+
+
+def _free_bytes():
+    """Device memory free to this process, from the HIP runtime."""
+    import ctypes as C
+    import os
+    lib = C.CDLL(os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "lib", "libamdhip64.so"))
+    free, total = C.c_size_t(), C.c_size_t()
+    assert lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+# two large requests, then as many small ones as the budget has room for
+@pytest.mark.parametrize("large,small", [(2_600_000, 700_000), (1_300_000, 1_250_000)])
+def test_requests_hold_no_more_than_the_budget(ctx, large, small):
+    # what finished requests leave behind neither refuses a request whose
+    # footprint fits nor lets those that run hold more than the budget: device
+    # memory in use grows by the budget at most (allocations are rounded up to
+    # 2 MiB here: 2 MiB for each request besides)
+    from aurora_pic import hip
+    gas = workloads.synthetic_gas(rows=64)
+    ctx.swarm_gas(gas)
+    dt = 0.05 / gas["max_frequency"]
+    warm = ctx.swarm_submit(_request(100.0, 1000, 4, 2, 2, dt, 1), hbm_budget=1 << 30)
+    ctx.swarm_advance(4)      # launch buffers, code
+    assert ctx.swarm_poll(warm)[0]
+    before = _free_bytes()
+    big, little = (_request(100.0, n, 4, 2, 2, dt, 1) for n in (large, small))
+    fp, fs = ctx.swarm_footprint(big), ctx.swarm_footprint(little)
+    budget = 2 * fp + fs // 2
+    fit = budget // fs
+    for sizes in ([big, big], [little] * fit, [little] * fit, [big, big]):
+        handles = [ctx.swarm_submit(r, hbm_budget=budget) for r in sizes]
+        with pytest.raises(hip.HipError, match="HBM budget"):
+            ctx.swarm_submit(little if sizes[0] is little else big, hbm_budget=budget)
+        used = before - _free_bytes()
+        assert used <= budget + (len(sizes) + 1) * (2 << 20), (used, budget)
+        ctx.swarm_advance(4)
+        assert all(ctx.swarm_poll(h)[0] for h in handles)
+        used = before - _free_bytes()
+        assert used <= budget + (len(sizes) + 1) * (2 << 20), (used, budget)
