@@ -64,6 +64,13 @@ struct CellPack {
 inline int pack_shift(int dim) { return dim == 3 ? 10 : (dim == 2 ? 15 : 31); }
 
 // --------------------------------------------------------- device memory
+struct Context;
+// The context whose call the thread runs (guarded), whose spare memory an
+// allocation that fails may use: release_spares frees it and says whether
+// there was any (swarm.hip).
+inline thread_local Context* calling_context = nullptr;
+bool release_spares(Context& ctx);
+
 template <typename T>
 struct DevBuf {
     T* ptr = nullptr;
@@ -71,7 +78,16 @@ struct DevBuf {
     void alloc(size_t n) {
         release();
         if (n == 0) return;
-        AUR_HIP(hipMalloc(reinterpret_cast<void**>(&ptr), n * sizeof(T)));
+        void* p = nullptr;
+        hipError_t e = hipMalloc(&p, n * sizeof(T));
+        if (e == hipErrorOutOfMemory && calling_context && release_spares(*calling_context))
+            e = hipMalloc(&p, n * sizeof(T));
+        if (e != hipSuccess) {
+            (void)hipGetLastError();   // reported here, not by the next launch
+            throw Failure{AURORA_ERR_HIP, "device allocation of " + std::to_string(n * sizeof(T)) +
+                                              " bytes: " + hipGetErrorString(e)};
+        }
+        ptr = static_cast<T*>(p);
         count = n;
     }
     void release() {
@@ -573,6 +589,11 @@ namespace aurora {
 template <typename F>
 int guarded(aurora_hip_ctx* h, F&& f) {
     if (!h) return AURORA_ERR_INVALID_ARGUMENT;
+    struct Calling {
+        Context* before = calling_context;
+        ~Calling() { calling_context = before; }
+    } calling;
+    calling_context = &h->c;
     try {
         h->c.last_error.clear();
         f(h->c);

@@ -464,7 +464,7 @@ struct SwarmState {
     // each request had seven allocations).  Used on the context's stream alone,
     // after it has drained past the request; at most kSpareBytes, which a
     // request's budget covers with the slabs in use (fit_budget), freed with
-    // the context or when a further slab needs the memory.
+    // the context or when an allocation of the context needs the memory.
     std::vector<DevBuf<uint8_t>> spare;
     size_t spare_bytes = 0;
     bool budgeted = false;          // a request came with an HBM budget
@@ -493,18 +493,6 @@ void fit_budget(SwarmState& s, uint64_t bytes, uint64_t budget) {
     while (!s.spare.empty() && s.bytes_in_use + bytes + s.spare_bytes > budget) {
         s.spare_bytes -= s.spare.back().count;
         s.spare.pop_back();
-    }
-}
-
-void alloc_slab(SwarmState& s, DevBuf<uint8_t>& slab, size_t bytes) {
-    try {
-        slab.alloc(bytes);
-    } catch (const Failure&) {
-        if (s.spare.empty()) throw;
-        (void)hipGetLastError();
-        s.spare.clear();
-        s.spare_bytes = 0;
-        slab.alloc(bytes);
     }
 }
 
@@ -1271,6 +1259,15 @@ void swarm_destroy(Context& c) {
     }
 }
 
+bool release_spares(Context& c) {
+    if (!c.swarm) return false;
+    SwarmState& s = *static_cast<SwarmState*>(c.swarm);
+    const bool any = !s.spare.empty();
+    s.spare.clear();
+    s.spare_bytes = 0;
+    return any;
+}
+
 }  // namespace aurora
 
 using namespace aurora;
@@ -1339,7 +1336,7 @@ int aurora_hip_swarm_submit(aurora_hip_ctx* h, const aurora_hip_swarm_request* r
         st->slab = take_spare(s, lay.bytes, s.budgeted ? fp : 4 * fp);
         st->footprint = std::max<uint64_t>(fp, st->slab.count);
         if (hbm_budget) fit_budget(s, st->footprint, hbm_budget);
-        if (!st->slab.ptr) alloc_slab(s, st->slab, lay.bytes);
+        if (!st->slab.ptr) st->slab.alloc(lay.bytes);
         uint8_t* base = st->slab.ptr;
         st->part = reinterpret_cast<long long*>(base);
         st->counts = reinterpret_cast<unsigned long long*>(base + lay.counts);

@@ -269,3 +269,23 @@ def test_requests_hold_no_more_than_the_budget(ctx, large, small):
         assert all(ctx.swarm_poll(h)[0] for h in handles)
         used = before - _free_bytes()
         assert used <= budget + (len(sizes) + 1) * (2 << 20), (used, budget)
+
+
+def test_kept_memory_is_given_back_to_an_allocation_that_fails(ctx):
+    # the memory that finished requests leave goes before any allocation of the
+    # context fails, not only another request's: one larger than the device
+    # still fails, as an error, with that memory free again
+    from aurora_pic import hip
+    gas = workloads.synthetic_gas(rows=64)
+    ctx.swarm_gas(gas)
+    dt = 0.05 / gas["max_frequency"]
+    handle = ctx.swarm_submit(_request(100.0, 5_000_000, 4, 2, 2, dt, 1))
+    ctx.swarm_advance(4)
+    assert ctx.swarm_poll(handle)[0]
+    kept = _free_bytes()
+    with pytest.raises(hip.HipError, match="out of memory"):
+        ctx.stream_bandwidth(0, nbytes=1 << 45)
+    assert _free_bytes() - kept >= 5_000_000 * 24
+    # nothing of the failure is left for the next call
+    req = _request(100.0, 1000, 4, 2, 2, dt, 1)
+    assert _run_all(ctx, [req], 4)[0].status == 0
