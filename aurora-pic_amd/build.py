@@ -62,7 +62,7 @@ def build_host() -> str:
     if r.returncode != 0:
         raise RuntimeError(f"host library build failed:\n{r.stderr[-6000:]}")
     os.replace(HOST_SO + ".tmp", HOST_SO)
-    cmd = [CXX, "-std=c++20", "-O2", "-Wall", "-Wextra", *inc,
+    cmd = [CXX, "-std=c++20", "-O2", "-Wall", "-Wextra", *inc, f"-I{CSRC}",
            os.path.join(HOST, "tests", "host_tests.cpp"), "-o", HOST_TESTS + ".tmp", f"-L{LIB}",
            "-laurora_gpu", "-laurora_hip", rpath]
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -72,42 +72,18 @@ bool sort_needed(Context& c, Species& sp) {
     return false;
 }
 
-// The renewal rule: with a cycle cost C(n) = sort + pushes 1..n and pushes
-// that slow down as the cycle ages, the long-run cost per step C(n)/n is
-// least at the first n whose push exceeds C(n)/n.  The push compared is the
-// mean of the last three timed pushes (timing noise).  Timings are read one
-// step late (the previous step's push has completed by then), so the
-// decision lags by one step and the host never stalls the queue.  The sort in
-// C(n) stands for the one that ends the cycle, a local sort: the general sort
-// that began the first cycle (a radix sort, a permutation of every array and
-// their allocations) counts for at most kLocalSortPushes of its pushes, the
-// local sort's order of cost (2 pushes of 128^3 x 16, 5 of 256^2 x 32).
-// Taken at its own cost it kept a new state unsorted until its pushes took
-// 1,640 us (430 freshly sorted) and 338 us (33).
-constexpr double kLocalSortPushes = 4.0;
-
+// The adaptive policy (sort_cycle.hpp).  Timings are read one step late (the
+// previous step's push has completed by then), so the decision lags by one
+// step and the host never stalls the queue.
 bool adaptive_sort_due(Context& c, Species& sp) {
     if (!c.tiled_push_ok()) return false;  // no tiled push to speed up
     if (!sp.tiled) return sp.slots > 0;
     if (sp.sort_ev.recorded && hipEventQuery(sp.sort_ev.b) == hipSuccess)
-        sp.sort_ms = sp.sort_ev.take_ms();
+        sp.cycle.sort_ms = sp.sort_ev.take_ms();
     EventPair& ev = sp.push_ev[sp.push_ev_cur];   // recorded by the previous step
-    if (ev.recorded) {
-        const double p = ev.take_ms();
-        if (sp.timed_pushes == 0) sp.first_push_ms = p;
-        sp.cycle_ms += p;
-        sp.recent_ms[2] = sp.recent_ms[1];
-        sp.recent_ms[1] = sp.recent_ms[0];
-        sp.recent_ms[0] = p;
-        ++sp.timed_pushes;
-    }
+    if (ev.recorded) sp.cycle.pushed(ev.take_ms());
     if (c.sort_max_interval > 0 && sp.pushes_since_sort >= c.sort_max_interval) return true;
-    if (sp.sort_ev.recorded || sp.timed_pushes < 3) return false;
-    const double recent = (sp.recent_ms[0] + sp.recent_ms[1] + sp.recent_ms[2]) / 3.0;
-    const double sort = sp.general_sort
-                            ? std::min(sp.sort_ms, kLocalSortPushes * sp.first_push_ms)
-                            : sp.sort_ms;
-    return recent * static_cast<double>(sp.timed_pushes) > sort + sp.cycle_ms;
+    return !sp.sort_ev.recorded && sp.cycle.due(c.sort_method == 0);
 }
 
 double electrode(const double* p, double t) {

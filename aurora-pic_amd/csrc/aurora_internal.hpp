@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "aurora_hip.h"
+#include "sort_cycle.hpp"
 
 namespace aurora {
 
@@ -225,12 +226,7 @@ struct Species {
     // they have completed, so the host does not wait on the device.
     EventPair push_ev[2], sort_ev;
     int push_ev_cur = 0;                  // pair the next push records into
-    double sort_ms = 0.0;                 // the last sort
-    bool general_sort = false;            // it was the general one, not a local sort
-    double first_push_ms = 0.0;           // the cycle's first timed push
-    double cycle_ms = 0.0;                // the timed pushes since the sort, ms
-    int64_t timed_pushes = 0;             // pushes of the cycle in cycle_ms
-    double recent_ms[3] = {0, 0, 0};      // the last three timed pushes
+    SortCycle cycle;
     size_t elem() const { return precision == 64 ? 8 : 4; }
 };
 

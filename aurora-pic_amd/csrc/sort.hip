@@ -654,7 +654,6 @@ void sort_species(Context& c, Species& sp) {
                           sp.tile_keyspace == static_cast<int64_t>(keyspace);
     if (local_ok && (sp.precision == 64 ? local_sort<double>(c, sp, k, ntz, bits)
                                         : local_sort<float>(c, sp, k, ntz, bits))) {
-        sp.general_sort = false;
         finish_sort(c, sp, timed);
         return;
     }
@@ -695,16 +694,14 @@ void sort_species(Context& c, Species& sp) {
     AUR_HIP(hipStreamSynchronize(c.stream));
     sp.slots = live;
     sp.tile_keyspace = static_cast<int64_t>(keyspace);
-    sp.general_sort = true;
     finish_sort(c, sp, timed);
 }
 
 void finish_sort(Context& c, Species& sp, bool timed) {
+    sp.cycle.begin(!sp.tiled);
     sp.tiled = true;
     sp.sorted_slots = sp.slots;
     sp.pushes_since_sort = 0;
-    sp.cycle_ms = 0.0;
-    sp.timed_pushes = 0;
     sp.push_ev[0].recorded = false;   // pushes of the previous cycle
     sp.push_ev[1].recorded = false;
     if (timed) sp.sort_ev.record_end(c.stream);

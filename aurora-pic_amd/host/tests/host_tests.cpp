@@ -31,6 +31,7 @@
 #include "aurora_gpu.hpp"
 #include "diagnostics.hpp"
 #include "particle_state.hpp"
+#include "sort_cycle.hpp"
 
 using namespace pic::gpu;
 
@@ -551,7 +552,29 @@ struct CpuCase {
     void (*body)(const std::filesystem::path&);
 };
 
+// The adaptive sort's rule on pushes of 1, 1.1, 1.2, ... ms: n pushes exceed
+// the average of a cycle of sort S when 0.05 n^2 - 0.15 n > S.  A new state's
+// first sort counts for four of its first push when a local sort ends the
+// cycle; any other, general or not, for what it took.
+int pushes_until_due(bool first, bool local, double sort_ms) {
+    aurora::SortCycle c;
+    c.begin(first);
+    c.sort_ms = sort_ms;
+    int n = 0;
+    while (!c.due(local) && n < 1000) c.pushed(1.0 + 0.1 * n++);
+    return n;
+}
+
+void adaptive_sort_cycles(const std::filesystem::path&) {
+    require(pushes_until_due(true, true, 100.0) == 11, "first cycle, capped sort");
+    require(pushes_until_due(true, true, 2.3) == 9, "first cycle, sort below the cap");
+    require(pushes_until_due(true, false, 100.0) == 47, "first cycle under radix sorts");
+    require(pushes_until_due(false, true, 100.0) == 47, "later cycle begun by a general sort");
+    require(pushes_until_due(false, false, 100.0) == 47, "later cycle under radix sorts");
+}
+
 const CpuCase kCpuCases[] = {
+    {"adaptive_sort_cycles", adaptive_sort_cycles},
     {"aps_reference_example_signature", aps_reference_example_signature},
     {"aps_round_trip", aps_round_trip},
     {"aps_errors", aps_errors},

@@ -954,3 +954,45 @@ def test_energy_sums(hip_ctx, n, bc, precision):
         want = math.fsum(0.5 * m * w * np.sum(v ** 2, axis=1))
         assert abs(k - want) <= 1e-12 * want
     assert live == sum(counts)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("method", ["SORT_LOCAL", "SORT_RADIX"])
+@pytest.mark.parametrize("n,precision", [([24, 16, 16], 32), ([21, 13, 30], 32), ([21, 13, 30], 64),
+                                         ([37, 45], 32), ([37, 45], 64)])
+def test_adaptive_sort_methods_precisions_and_meshes(n, precision, method):
+    """The adaptive policy by either sort method, for both precisions and on
+    meshes that the tiles divide and do not: it sorts within its longest
+    interval, and particles and charge equal the untiled, unsorted run's bit
+    for bit."""
+    from aurora_pic import hip
+    print(f"case={n} {precision} {method}", flush=True)
+    rng = np.random.default_rng(37)
+    dim = len(n)
+    L = [1.0, 0.75, 1.25][:dim]
+    N = 20000
+    pos = rng.uniform(0, 1, (N, dim)) * np.asarray(L)
+    vel = rng.normal(0, 0.5, (N, 3))
+    out = []
+    for policy in (None, 0, 4):
+        with hip.Context(0) as c:
+            c.mesh(n, L, 0, 1.0)
+            if policy is None:
+                c.tiling(0)
+            else:
+                c.sort_policy(hip.SORT_ADAPTIVE, policy)
+                c.sort_method(getattr(hip, method))
+            sid = c.add_species(-1.0, 1.0, 1.0 / N, N, precision)
+            c.upload(sid, pos, vel, kind=1)
+            c.initialize(0.01)
+            c.timing()
+            c.sort_interval(0)
+            c.step(0.01, 21)
+            if policy is not None:
+                assert c.kernel_time("sort")[1] >= (5 if policy else 1)
+            p_, v_, _, u_ = c.download(sid)
+            o = np.argsort(u_)
+            out.append((c.charge_fixed(sid), p_[o], v_[o]))
+    for other in out[1:]:
+        for a, b in zip(out[0], other):
+            assert np.array_equal(a, b)
