@@ -704,6 +704,7 @@ void finish_sort(Context& c, Species& sp, bool timed) {
     sp.pushes_since_sort = 0;
     sp.push_ev[0].recorded = false;   // pushes of the previous cycle
     sp.push_ev[1].recorded = false;
+    sp.sort_ev.recorded = false;      // an earlier sort's, never read
     if (timed) sp.sort_ev.record_end(c.stream);
     AUR_HIP(hipMemsetAsync(sp.absorbed.ptr + 6, 0, sizeof(unsigned long long), c.stream));
 }

@@ -24,14 +24,16 @@ namespace aurora {
 constexpr double kLocalSortPushes = 4.0;
 
 struct SortCycle {
-    double sort_ms = 0.0;         // the sort that began the cycle
+    double sort_ms = 0.0;         // the sort that began the cycle; 0: not timed
     bool first = false;           // a new state's
     double first_push_ms = 0.0;   // the cycle's first timed push
     double push_ms = 0.0;         // its timed pushes
     int64_t pushes = 0;
     double recent_ms[3] = {0.0, 0.0, 0.0};   // the last three
 
+    // a sort has been queued; its time, if it is timed, comes later (sort_ms)
     void begin(bool first_cycle) {
+        sort_ms = 0.0;
         first = first_cycle;
         push_ms = 0.0;
         pushes = 0;

@@ -571,6 +571,21 @@ void adaptive_sort_cycles(const std::filesystem::path&) {
     require(pushes_until_due(true, false, 100.0) == 47, "first cycle under radix sorts");
     require(pushes_until_due(false, true, 100.0) == 47, "later cycle begun by a general sort");
     require(pushes_until_due(false, false, 100.0) == 47, "later cycle under radix sorts");
+    // a sort that is not timed (another policy's) does not inherit the time
+    // of an earlier one: pushes that do not slow down are never due, those
+    // that do at once
+    aurora::SortCycle c;
+    c.begin(false);
+    c.sort_ms = 100.0;
+    for (int n = 0; n < 10; ++n) c.pushed(1.0);
+    c.begin(false);
+    require(c.sort_ms == 0.0, "an earlier sort's time");
+    for (int n = 0; n < 10; ++n) {
+        c.pushed(1.0);
+        require(!c.due(true), "pushes that do not slow down");
+    }
+    c.pushed(1.2);
+    require(c.due(true), "pushes that slow down after an untimed sort");
 }
 
 const CpuCase kCpuCases[] = {
