@@ -349,10 +349,7 @@ struct Context {
     DevBuf<int32_t> ls_new_start;
     DevBuf<unsigned> ls_far_key, ls_far_key2, ls_far_val, ls_far_val2;
     DevBuf<uint8_t> ls_stage;
-    // the product count of each model's MCC pass, read back through pinned memory
-    DevBuf<long long> product_total;
-    PinnedHost<long long> product_total_host;
-    int64_t product_total_models = 0;
+    DevBuf<long long> product_total;   // the product count of each model's MCC pass
     // 1D MCC steps inside one aurora_hip_step call keep the slot counts and
     // next uids on the device (products are reserved and placed without a
     // host wait; kernels read the counts, launches are sized for the

@@ -138,7 +138,7 @@ __global__ void __launch_bounds__(kMccBlock, kMccWaves)
 // All models' products reserved together on the device (the counts kept
 // there during aurora_hip_step): the all-or-nothing capacity check over
 // every model (Simulation.cpp:929-964), then slots and uids per model in
-// model order, as mcc_append reserves them on the host.  Run by one thread
+// model order (Simulation.cpp:965-1005).  Run by one thread
 // (the last model's k_mcc_finish, after every model's total is known).
 struct CommitArgs {
     int models, nspecies;
@@ -236,30 +236,19 @@ __global__ void __launch_bounds__(kFold) k_collide_finish(const double* rows, in
                                       : AURORA_ERR_INVALID_ARGUMENT;
 }
 
-__global__ void k_zero_total(long long* total) { *total = 0; }
-
-// the reservation alone (a last model whose target holds no slots)
-__global__ void k_mcc_commit(CommitArgs a) {
-    __shared__ long long need[kMaxChannels];
-    if (blockIdx.x == 0 && threadIdx.x == 0) commit_products(a, need);
-}
-
 // the products of every listed parent, a wave per run (the runs of the
-// collide: groups workgroups of it); with place (device counts), the parents
-// and the bases come from commit_products' placement
+// collide: groups workgroups of it); the parents and the bases come from
+// commit_products' placement
 __global__ void __launch_bounds__(kBlk) k_append_products(
     const int32_t* pcell, const float* poff, const int32_t* list, const int32_t* run_parents,
-    const int32_t* run_off, const float* prod, int64_t slots, int groups, const float* E32, int nx,
+    const int32_t* run_off, const float* prod, int groups, const float* E32, int nx,
     AppendSide sec, AppendSide ion, const long long* place) {
-    if (place) {
-        if (place[5] == 0) return;
-        sec.base_slot = place[0];
-        ion.base_slot = place[1];
-        sec.base_uid = static_cast<uint32_t>(place[2]);
-        ion.base_uid = static_cast<uint32_t>(place[3]);
-        slots = place[4];
-    }
-    const RunPlan plan(slots, groups * (kMccBlock / 64));
+    if (place[5] == 0) return;
+    sec.base_slot = place[0];
+    ion.base_slot = place[1];
+    sec.base_uid = static_cast<uint32_t>(place[2]);
+    ion.base_uid = static_cast<uint32_t>(place[3]);
+    const RunPlan plan(place[4], groups * (kMccBlock / 64));
     const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (uint32_t r = blockIdx.x * (kBlk / 64) + wid; r < plan.runs;
          r += gridDim.x * (kBlk / 64)) {
@@ -504,12 +493,7 @@ void mcc_collide_pass(Context& c, int model, double dt, const CommitArgs& commit
     const int64_t n = slot_bound(c, sp);
     const long long* nslots = c.counts_on_device ? c.dev_counts.ptr + h.target : nullptr;
     long long* total = c.product_total.ptr + model;
-    if (n == 0) {
-        k_zero_total<<<1, 1, 0, c.stream>>>(total);
-        if (commit.models > 0) k_mcc_commit<<<1, 64, 0, c.stream>>>(commit);
-        AUR_HIP(hipGetLastError());
-        return;
-    }
+    if (n == 0) return;   // (a capacity is not 0: nothing has products)
     const bool products = h.secondary_species >= 0;
     const int g = mcc_groups(c.cu_count, n);
     const int64_t runs = max_runs(n, static_cast<int64_t>(g) * (kMccBlock / 64));
@@ -560,17 +544,16 @@ void mcc_collide_pass(Context& c, int model, double dt, const CommitArgs& commit
     AUR_HIP(hipGetLastError());
 }
 
-// Places the `total` product pairs staged by one model's pass after the
-// live particles of the secondary and ion species (Simulation.cpp:965-1005).
-// place: the model's placement reserved on the device by commit_products (the
-// counts on the device; total and the host's counts are then unused).
-void mcc_append(Context& c, int model, int64_t total, double dt, const long long* place) {
+// Places the product pairs staged by one model's pass after the live particles
+// of the secondary and ion species (Simulation.cpp:965-1005); place: its slots
+// and uids, reserved on the device by commit_products.
+void mcc_append(Context& c, int model, double dt, const long long* place) {
     MccModelHost& h = c.mcc_model(model);
     Species& sp = c.species[h.target];
-    const int64_t n = slot_bound(c, sp);
+    const int64_t n = slot_bound(c, sp);   // the collide pass's
     Species& se = c.species[h.secondary_species];
     Species& si = c.species[h.ion_species];
-    auto side = [&](Species& s, int64_t base_slot) {
+    auto side = [&](Species& s) {
         AppendSide d{};
         d.cell = s.cell.ptr;
         d.off = reinterpret_cast<float*>(s.off[0].ptr);
@@ -578,40 +561,20 @@ void mcc_append(Context& c, int model, int64_t total, double dt, const long long
         d.v1 = reinterpret_cast<float*>(s.vel[1].ptr);
         d.v2 = reinterpret_cast<float*>(s.vel[2].ptr);
         d.uid = s.uid.ptr;
-        d.base_slot = base_slot;
         d.half_qm_dt = static_cast<float>(0.5 * s.charge / s.mass * dt);
         return d;
     };
-    AppendSide sec = side(se, se.slots), ion{};
-    sec.base_uid = se.next_uid;
-    if (h.secondary_species == h.ion_species) {
-        ion = side(si, si.slots + total);
-        ion.base_uid = se.next_uid + static_cast<uint32_t>(total);
-    } else {
-        ion = side(si, si.slots);
-        ion.base_uid = si.next_uid;
-    }
     {
         KernelScope ks(c, "append_products");
         const int g = mcc_groups(c.cu_count, n);
         k_append_products<<<g, kBlk, 0, c.stream>>>(
             sp.cell.ptr, reinterpret_cast<const float*>(sp.off[0].ptr), h.product_list.ptr,
-            h.run_parents.ptr, h.run_off.ptr, h.product_vel.ptr, n, g, c.E32.ptr,
-            static_cast<int>(c.n[0]), sec, ion, place);
+            h.run_parents.ptr, h.run_off.ptr, h.product_vel.ptr, g, c.E32.ptr,
+            static_cast<int>(c.n[0]), side(se), side(si), place);
         AUR_HIP(hipGetLastError());
     }
     se.tiled = false;
     si.tiled = false;
-    if (place) return;
-    if (h.secondary_species == h.ion_species) {
-        se.slots += 2 * total;
-        se.next_uid += static_cast<uint32_t>(2 * total);
-    } else {
-        se.slots += total;
-        se.next_uid += static_cast<uint32_t>(total);
-        si.slots += total;
-        si.next_uid += static_cast<uint32_t>(total);
-    }
 }
 
 }  // namespace
@@ -640,17 +603,16 @@ void mcc_step(Context& c, double dt) {
                             AURORA_ERR_INVALID_ARGUMENT,
                             "ionization and anisotropic MCC require the 3V collision interface");
         }
-    if (c.product_total_models < models) {
+    if (c.product_total.count < static_cast<size_t>(models))
         c.product_total.alloc(static_cast<size_t>(models));
-        c.product_total_host.alloc(static_cast<size_t>(models));
-        c.product_total_models = models;
-    }
     bool products = false;
     for (int k = 0; k < models; ++k) products = products || c.mcc_model(k).secondary_species >= 0;
-    // with the counts on the device: the last model's finishing kernel
-    // reserves every model's products (no host wait)
+    // the last model's finishing kernel reserves every model's products from
+    // the counts on the device (device_counts_apply: no host wait)
+    AUR_REQUIRE(!products || c.counts_on_device, AURORA_ERR_UNSUPPORTED,
+                "MCC products need the slot counts on the device");
     CommitArgs ca{};
-    if (products && c.counts_on_device) {
+    if (products) {
         ca.models = models;
         ca.nspecies = static_cast<int>(c.species.size());
         for (int k = 0; k < models; ++k) {
@@ -669,35 +631,9 @@ void mcc_step(Context& c, double dt) {
     }
     const CommitArgs none{};
     for (int k = 0; k < models; ++k) mcc_collide_pass(c, k, dt, k == models - 1 ? ca : none);
-    if (!products) return;
-    if (c.counts_on_device) {
-        for (int k = 0; k < models; ++k)
-            if (c.mcc_model(k).secondary_species >= 0)
-                mcc_append(c, k, 0, dt, c.mcc_place.ptr + static_cast<int64_t>(k) * kPlaceFields);
-        return;
-    }
-    // every model's product count in one copy into pinned memory, one wait
-    AUR_HIP(hipMemcpyAsync(c.product_total_host.ptr, c.product_total.ptr,
-                           static_cast<size_t>(models) * sizeof(long long), hipMemcpyDeviceToHost,
-                           c.stream));
-    AUR_HIP(hipStreamSynchronize(c.stream));
-    std::vector<int64_t> total(static_cast<size_t>(models), 0);
     for (int k = 0; k < models; ++k)
-        total[static_cast<size_t>(k)] = static_cast<int64_t>(c.product_total_host.ptr[k]);
-    std::vector<int64_t> need(c.species.size(), 0);
-    for (int k = 0; k < models; ++k) {
-        const MccModelHost& h = c.mcc_model(k);
-        if (total[static_cast<size_t>(k)] == 0) continue;
-        need[static_cast<size_t>(h.secondary_species)] += total[static_cast<size_t>(k)];
-        need[static_cast<size_t>(h.ion_species)] += total[static_cast<size_t>(k)];
-    }
-    for (size_t s = 0; s < c.species.size(); ++s)
-        if (need[s] && c.species[s].slots + need[s] > c.species[s].capacity)
-            throw Failure{AURORA_ERR_CAPACITY,
-                          "reactive collisions exceeded max_particles_per_species for species"};
-    for (int k = 0; k < models; ++k)
-        if (total[static_cast<size_t>(k)] > 0)
-            mcc_append(c, k, total[static_cast<size_t>(k)], dt, nullptr);
+        if (c.mcc_model(k).secondary_species >= 0)
+            mcc_append(c, k, dt, c.mcc_place.ptr + static_cast<int64_t>(k) * kPlaceFields);
 }
 
 namespace {
