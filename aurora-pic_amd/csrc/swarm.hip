@@ -1039,6 +1039,7 @@ __global__ void __launch_bounds__(T) k_br_small(MccParams m, BranchArgs a, int n
                 if (lane == 0) log_samples[step - a.burn_in] = n * w_new;
             }
             w = w_new;
+            wave_lds_fence();   // lane c + 2 clears the counter that lane c has read
             if (lane < 2 + NCH) cnt[lane] = 0u;
         }
         __syncthreads();
