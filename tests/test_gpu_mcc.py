@@ -605,3 +605,80 @@ def test_collide_at_the_edges_of_a_waves_run(ctx, oracle, n, part):
             far.append(st.margin)
     assert max(far, default=0.0) <= MARGIN
     assert len(far) <= 0.02 * at.size + 1
+
+
+def past_lds(gas, shared):
+    """The gas with 2,000 rows more past the end of every table, at its last
+    cross section, which is also what stands for energies past the end: the
+    same rates to the bit, from tables that no longer fit a workgroup's LDS
+    (4,096 words).  Not shared: the channels' further energies differ."""
+    out = dict(gas)
+    out["channels"] = []
+    for k, (kind, threshold, e, s) in enumerate(gas["channels"]):
+        further = np.geomspace(1.01, 10.0 + (0 if shared else k), 2000) * e[-1]
+        out["channels"].append((kind, threshold, np.concatenate([e, further]),
+                                np.concatenate([s, np.full(2000, s[-1])])))
+    return out
+
+
+@pytest.mark.parametrize("shared", [True, False])
+@pytest.mark.parametrize("temperature", [0.0, 300.0])
+def test_tables_past_lds_give_the_same_bits(shared, temperature):
+    # the builds that read the tables from global memory against those that
+    # keep them in LDS: bare collide (3V, 1V), the 1D step with its products,
+    # and an ensemble
+    from aurora_pic import hip
+    small = workloads.synthetic_gas(rows=200, neutral_density=1.0e22)
+    small["neutral_temperature"] = temperature
+    if temperature:      # the thermal bound takes speeds 8 sigma above a particle's
+        small["max_frequency"] *= 1.2
+    n = 3000
+    dt = min(1.0 / (400 * 13.56e6), 0.09 / small["max_frequency"])
+    hot = math.sqrt(30.0 * workloads.EV / workloads.ME)
+    rng = np.random.default_rng(5)
+    vin = rng.normal(0.0, hot, (5000, 3)).astype(np.float32).astype(np.float64)
+
+    def run(gas):
+        out = []
+        with hip.Context(0) as c:
+            c.mesh([65], [0.067], hip.DIRICHLET, workloads.EPS0)
+            se = c.add_species(-workloads.EV, workloads.ME, 1e6, 6 * n)
+            si = c.add_species(workloads.EV, 6.67e-27, 1e6, 6 * n)
+            c.mcc_load(se, gas, product_species=(se, si), seed=23,
+                       neutral_temperature=temperature)
+            v, counts, ech = c.mcc_collide(vin, 40 * dt, step=1)
+            out += [v, np.asarray(counts), np.asarray(ech)]
+            assert counts[2 + 2] > 0
+            ens = c.ensemble_create(3, [6 * n, 6 * n])
+            for k in range(3):
+                c.init_maxwellian(se, n - 100 * k, hot, seed=21 + k)
+                c.init_maxwellian(si, n, 500.0, seed=41 + k)
+                c.initialize(dt)
+                ens.load(k, 60 + k)
+            ens.step(dt, 20)
+            for k in range(3):
+                for s in (se, si):
+                    p, v, a, u = ens.download(k, s)
+                    o = np.argsort(u)
+                    out += [p[o], v[o], u[o]]
+            c.step(dt, 20)
+            for s in (se, si):
+                p, v, a, u = c.download(s)
+                o = np.argsort(u)
+                out += [p[o], v[o], u[o]]
+            counts, ech = c.mcc_stats()
+            assert counts[2 + 2] > 0
+            out += [np.asarray(counts), np.asarray(ech)]
+        with hip.Context(0) as c:
+            c.mesh([65], [0.067], hip.DIRICHLET, workloads.EPS0)
+            se = c.add_species(-workloads.EV, workloads.ME, 1e6, n)
+            one = dict(gas)
+            one["channels"] = gas["channels"][:2]
+            c.mcc_load(se, one, seed=23, neutral_temperature=temperature)
+            c.velocity_dimensions(1)
+            v, counts, ech = c.mcc_collide(vin, 40 * dt, step=1)
+            out += [v, np.asarray(counts), np.asarray(ech)]
+        return out
+
+    for a, b in zip(run(small), run(past_lds(small, shared))):
+        assert np.array_equal(a, b)

@@ -289,3 +289,33 @@ def test_kept_memory_is_given_back_to_an_allocation_that_fails(ctx):
     # nothing of the failure is left for the next call
     req = _request(100.0, 1000, 4, 2, 2, dt, 1)
     assert _run_all(ctx, [req], 4)[0].status == 0
+
+
+@pytest.mark.parametrize("shared", [True, False])
+def test_swarm_tables_past_lds_give_the_same_bits(shared):
+    # the build that reads the tables from global memory
+    from aurora_pic import hip
+    from test_gpu_mcc import past_lds
+    gas = workloads.synthetic_gas(rows=200)
+    dt = 0.09 / gas["max_frequency"]
+    reqs = [_request(300.0, 700, 200, 50, 5, dt, 3, e0=20.0),
+            _request(30.0, 2000, 120, 20, 4, dt, 4)]
+    out = []
+    for g in (gas, past_lds(gas, shared)):
+        with hip.Context(0) as c:
+            c.swarm_gas(g)
+            out.append([bytes(r) for r in _run_all(c, reqs, 64)])
+    assert out[0] == out[1]
+
+
+@pytest.mark.parametrize("launch", [1000, 130, 98])
+def test_swarm_blocks_of_one_launch(ctx, launch):
+    # a launch over more uncertainty blocks (80, 37, 26) than a workgroup sums
+    # in LDS (32) against launches of 13 and fewer: the same bytes
+    gas = workloads.synthetic_gas(rows=64)
+    ctx.swarm_gas(gas)
+    dt = 0.09 / gas["max_frequency"]
+    reqs = [_request(200.0, n, 260, 20, 80, dt, n) for n in (1, 300, 700)]
+    few = [bytes(r) for r in _run_all(ctx, reqs, 37)]
+    many = [bytes(r) for r in _run_all(ctx, reqs, launch)]
+    assert few == many
