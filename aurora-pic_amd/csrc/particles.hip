@@ -1115,7 +1115,7 @@ bool launch_tile3d_t(Context& c, Species& sp, const PushArgs<R>& a, int mode) {
     if (c.tile[0] != TX || c.tile[1] != TY || c.tile[2] != TZ || c.halo != H) return false;
     const int ntx = c.tiles_axis(0), nty = c.tiles_axis(1);
     const unsigned grid = static_cast<unsigned>(c.ntiles());
-    KernelScope ks(c, "push_deposit");
+    KernelScope tiled(c, "push_tiled"), ks(c, "push_deposit");
     const int32_t* ts = sp.tile_start.ptr;
     if (mode == 0)
         k_push_tile3d<R, TX, TY, TZ, H, 0, BLOCK, PF><<<grid, BLOCK, 0, c.stream>>>(a, ts, ntx, nty);
@@ -1318,7 +1318,7 @@ bool launch_tile2d_t(Context& c, Species& sp, const PushArgs<R>& a, int mode) {
     if (c.tile[0] != TX || c.tile[1] != TY || c.halo != H) return false;
     const int ntx = c.tiles_axis(0);
     const unsigned grid = static_cast<unsigned>(c.ntiles());
-    KernelScope ks(c, "push_deposit");
+    KernelScope tiled(c, "push_tiled"), ks(c, "push_deposit");
     const int32_t* ts = sp.tile_start.ptr;
     if (mode == 0)
         k_push_tile2d<R, TX, TY, H, 0, BLOCK, PF><<<grid, BLOCK, 0, c.stream>>>(a, ts, ntx);

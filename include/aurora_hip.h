@@ -535,7 +535,8 @@ int aurora_hip_stream_bandwidth(aurora_hip_ctx* ctx, int pattern, int64_t bytes,
                                 int repeats, double* gbs);
 /* Per-kernel HIP-event timing on the context stream (off by default). */
 int aurora_hip_kernel_timing(aurora_hip_ctx* ctx, int enable);
-/* Total milliseconds and launch count of kernel `name` since enabled. */
+/* Total milliseconds and launch count of kernel `name` since enabled
+ * (push_tiled: the launches of push_deposit that were LDS-tiled). */
 int aurora_hip_kernel_time(aurora_hip_ctx* ctx, const char* name,
                            double* total_ms, int64_t* launches);
 
