@@ -338,7 +338,6 @@ struct Context {
     int push_block = 512;        // tiled push workgroup size
     int push_prefetch = -1;      // tiled push variant; -1: the library's choice for the tile shape
     bool tiled_enabled = true;
-    DevBuf<int32_t> tile_count, tile_offset;
     DevBuf<double> energy_sums;           // partials and results of aurora_hip_energy
     DevBuf<unsigned> sort_keys, sort_keys2, sort_vals, sort_vals2;
     DevBuf<uint8_t> sort_temp;
@@ -448,8 +447,8 @@ inline dim3 grid_for(int64_t n, int block) {
 // host-side API pieces implemented in separate translation units
 void solve_fields(Context& ctx, double phi_left, double phi_right, bool want_phi,
                   bool want_e64 = true);
-// the step's field solve: rho from the accumulators and the Poisson solve,
-// fused on the power-of-two FFT path (rho itself is then written on demand)
+// the step's field solve: rho from the accumulators and the Poisson solve in
+// one (in 2D and 3D rho itself is then written on demand)
 void solve_step_fields(Context& ctx, double phi_left, double phi_right);
 // converts the accumulators when the last step did not write rho
 void ensure_rho(Context& ctx);

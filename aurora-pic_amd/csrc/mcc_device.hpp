@@ -604,7 +604,9 @@ constexpr int kTallyErr = 2 * kMaxChannels + 3;
 // A lane's tally: the counters of mcc_candidate, of which candidates, nsec
 // and err are the current particle's (begin, finish) and the others sums.
 // Products go to memory when they are made (prod: 2 x (secondary, ion), or
-// null).  A lane has at most 2^32 / (64 waves) particles, so 32 bits do.
+// null).  32 bits hold a lane's sums: its particles (2^32 / (64 waves) at
+// most) times their candidates of the launch, each a chain of some hundred
+// cycles, stay below 2^32 in any launch that ends within hours.
 template <int NCH>
 struct LaneTally {
     uint32_t candidates, nsec, err;

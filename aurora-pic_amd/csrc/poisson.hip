@@ -1,6 +1,7 @@
 // poisson.hip - FP64 field solves (FieldSolver.cpp:384-759):
-//   1D periodic   direct spectral sum with continuous k (407-440)
-//   1D Dirichlet  Thomas algorithm, same recurrence (733-759)
+//   1D periodic   spectral solve with continuous k (407-440): FFTs on a power
+//                 of two, direct sums on other meshes
+//   1D Dirichlet  the tridiagonal solve (733-759) as two prefix sums
 //   2D/3D periodic FFT Poisson with spectral E (442-499, 659-731)
 // The 2D/3D solve transforms rho forward and the spectral fields back.
 // Each spectral field is first projected onto its Hermitian part (zeroing

@@ -16,7 +16,7 @@ __device__ __forceinline__ int wrap_index(int i, int n) {
 // Sums over the wave's 64 lanes (all of them active), in a fixed order: four
 // rotations within each row of 16 lanes (DPP, plain VALU operations), then the
 // four rows.  Through ds_bpermute a sum is twelve LDS round trips, one after
-// the other: k_work_1d_pair at 1e6 particles 10.8 -> 8.1 us, k_mcc_1d 26.1 ->
+// the other: the work of 1e6 1D particles (k_work_1d) 10.8 -> 8.1 us, k_mcc_1d 26.1 ->
 // 25.1 us.
 template <int ROTATE>
 __device__ __forceinline__ uint64_t row_rotate(uint64_t v) {

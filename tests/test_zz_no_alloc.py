@@ -1,5 +1,5 @@
 """aurora_hip_mcc_collide_device, the collide that allocates nothing (its
-per-wave energy rows live in a fixed device array), against
+per-workgroup tally rows live in a fixed device array), against
 aurora_hip_mcc_collide on the same velocities: velocities, counts and energy
 change identical, on two calls in a row (the second smaller), so nothing the
 first call left in the shared scratch leaks into the second.  Device buffers
