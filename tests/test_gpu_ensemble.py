@@ -175,3 +175,22 @@ def test_capacity_error_names_instance():
     with pytest.raises(hip.HipError, match="max_particles_per_species \\(ensemble instance"):
         ens.step(DT, 50)
     c.close()
+
+
+# MCC workgroups: several for each instance, one where two would not all run
+# at once, and more instances than run at once
+@pytest.mark.parametrize("instances", [200, 520, 769])
+def test_many_instances_equal_single_context_runs(instances):
+    from aurora_pic import hip
+    gas = workloads.synthetic_gas(rows=200, neutral_density=1.0e22)
+    c, sids, ens = _build_ensemble(hip, gas, instances, 10, capacity=2 * N)
+    ens.step(DT, 30)
+    for k in (0, instances - 1):
+        ref, _, ref_counts, _, _ = _alone(hip, gas, k, 500 + k, 30)
+        for sid in sids:
+            a = _by_uid(*ens.download(k, sid))
+            b = _by_uid(*ref[sid])
+            for x, y in zip(a, b):
+                assert np.array_equal(x, y), (k, sid)
+        assert np.array_equal(ens.stats(k, 3)[0], ref_counts)
+    c.close()
