@@ -76,7 +76,7 @@ bool sort_needed(Context& c, Species& sp) {
 // previous step's push has completed by then), so the decision lags by one
 // step and the host never stalls the queue.
 bool adaptive_sort_due(Context& c, Species& sp) {
-    if (!c.tiled_push_ok()) return false;  // no tiled push to speed up
+    if (!c.tiled_push_pays(sp)) return false;  // no tiled push to speed up
     if (!sp.tiled) return sp.slots > 0;
     if (sp.sort_ev.recorded && hipEventQuery(sp.sort_ev.b) == hipSuccess)
         sp.cycle.sort_ms = sp.sort_ev.take_ms();

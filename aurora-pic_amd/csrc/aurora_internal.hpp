@@ -407,6 +407,26 @@ struct Context {
             if (n[a] < tile[a] + 1 + 2 * halo) return false;
         return true;
     }
+    // and are used for a species, once it is tile-sorted: always for FP32 on
+    // tiles that divide the mesh.  For FP64, or where a last tile is partial,
+    // unless its tiles hold too few particles: a workgroup stages and writes
+    // back a box for each, which shows from two tiles per CU on and is paid
+    // back by about kTileSlots of them (us per step at 0.2, 0.6 and 2 particles
+    // per cell, 13, 38 and 128 a tile: FP64 on 512^2 51.6, 51.0 and 55.3
+    // tiled, 43.1, 51.3 and 81.1 untiled; FP32 on 1000 x 700 101, 103 and 110
+    // against 88, 111 and 193; on 100^3 with 36 a tile 138 and 138).  The
+    // adaptive policy's timing and re-sorts, 5 to 10 us per step, want
+    // kAdaptiveSlots (FP64 on 300^2: 9e4 particles 50.2 against 46.9 us left
+    // alone, 1.8e5 51.8 against 60.5; on 64^3 5e4 58.2 against 66.2).
+    static constexpr int64_t kTileSlots = 40, kAdaptiveSlots = 100000;
+    bool tiled_push_pays(const Species& sp) const {
+        if (!tiled_push_ok()) return false;
+        bool divides = true;
+        for (int a = 0; a < dim; ++a) divides = divides && n[a] % tile[a] == 0;
+        if (sp.precision == 32 && divides) return true;
+        if (ntiles() > 2 * cu_count && sp.slots < kTileSlots * ntiles()) return false;
+        return sort_policy != AURORA_SORT_ADAPTIVE || sp.slots >= kAdaptiveSlots;
+    }
 };
 
 // Scoped kernel timer: records HIP events around a launch when enabled.

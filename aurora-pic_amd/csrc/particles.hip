@@ -1735,7 +1735,7 @@ void push_all(Context& c, double dt, bool fuse_deposit, bool defer_ledger) {
             // a push whose partials were never folded (push without a step)
             if (sp.ledger_pending) fold_ledger_1d(c, sp);
         }
-        if (fuse_deposit && sp.tiled && c.tiled_push_ok() &&
+        if (fuse_deposit && sp.tiled && c.tiled_push_pays(sp) &&
             sp.slots < (int64_t{1} << 32) / static_cast<int64_t>(sp.elem())) {
             const bool timed = c.sort_policy == AURORA_SORT_ADAPTIVE;
             EventPair& ev = sp.push_ev[sp.push_ev_cur];

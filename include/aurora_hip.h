@@ -214,7 +214,9 @@ int aurora_hip_time(aurora_hip_ctx* ctx, double* time, int64_t* step);
 /* Tile shape (cells per axis) of the cell sort and of the LDS-tiled 2D and
  * 3D pushes, and its halo in cells; tx = 0 keeps the sort but disables the
  * tiled push.  The tiles need not divide the mesh, which holds at least a
- * tile with its halo per axis (else the untiled push runs).  Built 3D
+ * tile with its halo per axis (else the untiled push runs; it also runs for
+ * FP64 species, and on meshes that the tiles do not divide, where there are
+ * many tiles of few particles).  Built 3D
  * shapes: 8x8x8 (halo 1, 2), 8x8x4 (halo 1, 2), 4x4x4, 16x8x4 (halo 2); 2D (tz ignored; 1 names them): 8x8 (halo 1, 2;
  * 512 threads, or 256 with prefetch), 16x16 and 16x8 (halo 2).
  * No reference counterpart (the reference keeps particles unsorted). */

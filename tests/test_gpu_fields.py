@@ -986,7 +986,7 @@ def test_adaptive_sort_methods_precisions_and_meshes(n, precision, method):
     rng = np.random.default_rng(37)
     dim = len(n)
     L = [1.0, 0.75, 1.25][:dim]
-    N = 20000
+    N = 100000       # the fewest that the policy sorts on undivided meshes and for FP64
     pos = rng.uniform(0, 1, (N, dim)) * np.asarray(L)
     vel = rng.normal(0, 0.5, (N, 3))
     out = []
@@ -1006,6 +1006,54 @@ def test_adaptive_sort_methods_precisions_and_meshes(n, precision, method):
             c.step(0.01, 21)
             if policy is not None:
                 assert c.kernel_time("sort")[1] >= (5 if policy else 1)
+            p_, v_, _, u_ = c.download(sid)
+            o = np.argsort(u_)
+            out.append((c.charge_fixed(sid), p_[o], v_[o]))
+    for other in out[1:]:
+        for a, b in zip(out[0], other):
+            assert np.array_equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,shape,precision,per_tile", [
+    ([192, 176], (8, 8, 1, 2), 64, 1), ([192, 176], (8, 8, 1, 2), 64, 40),      # 528 tiles
+    ([192, 168], (8, 8, 1, 2), 64, 1),                                          # 504: two per CU
+    ([188, 173], (8, 8, 1, 2), 32, 39), ([188, 173], (8, 8, 1, 2), 32, 40),     # 528, partial
+    ([192, 176], (8, 8, 1, 2), 32, 1),                                          # FP32, divided
+    ([70, 70, 70], (8, 8, 8, 2), 32, 39), ([70, 70, 70], (8, 8, 8, 2), 32, 40), # 729
+    ([72, 72, 72], (8, 8, 8, 2), 64, 39), ([72, 72, 72], (8, 8, 8, 2), 64, 40)])
+def test_tiled_push_where_it_pays(n, shape, precision, per_tile):
+    """Sparse tiles of FP64 species and of undivided meshes are pushed untiled,
+    from 40 slots a tile on (and up to two tiles a CU always) tiled, under
+    interval sorts and, from 1e5 slots on, under the adaptive policy, which
+    sorts none of the others; results equal the untiled run's."""
+    from aurora_pic import hip
+    print(f"case={n} {shape} {precision} {per_tile}", flush=True)
+    tiles = int(np.prod([-(-m // t) for m, t in zip(n, shape)]))
+    divided = all(m % t == 0 for m, t in zip(n, shape))
+    N = per_tile * tiles
+    dense = (precision == 32 and divided) or tiles <= 512 or per_tile >= 40
+    out = []
+    for mode in ("untiled", "interval", "adaptive"):
+        with hip.Context(0) as c:
+            c.mesh(n, [1.0] * len(n), 0, 1.0)
+            c.tiling(*shape if mode != "untiled" else (0,))
+            sid = c.add_species(-1.0, 1.0, 1.0 / N, N, precision)
+            c.init_maxwellian(sid, N, 0.3, seed=5)
+            if mode == "adaptive":
+                c.sort_policy(hip.SORT_ADAPTIVE, 2)
+            else:
+                c.sort_interval(3)
+            c.initialize(0.005)
+            c.timing()
+            c.sort()
+            c.step(0.005, 7)
+            tiled, sorts = c.kernel_time("push_tiled")[1], c.kernel_time("sort")[1]
+            if mode == "interval":
+                assert (tiled, sorts) == (7 if dense else 0, 3)
+            if mode == "adaptive":
+                used = dense and ((precision == 32 and divided) or N >= 100000)
+                assert tiled == (7 if used else 0) and (sorts > 1) == used
             p_, v_, _, u_ = c.download(sid)
             o = np.argsort(u_)
             out.append((c.charge_fixed(sid), p_[o], v_[o]))
