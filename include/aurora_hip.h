@@ -418,7 +418,7 @@ int aurora_hip_swarm_gas(aurora_hip_ctx* ctx, int nchan, const int* kind,
  * (bytes; 0 = no limit) beside those of the requests that run; returns
  * AURORA_ERR_CAPACITY otherwise.  Memory of finished requests is kept for
  * the next ones (at most 256 MiB) and given back where the budget would not
- * hold it too.  A request submitted before the context's first budget may
+ * hold it too and before an allocation of the context fails.  A request submitted before the context's first budget may
  * run in more memory than its footprint (at most four times), and counts
  * with that. */
 int aurora_hip_swarm_submit(aurora_hip_ctx* ctx,
